@@ -248,6 +248,36 @@ int luna_uvw_bwd(const LunaUvwPlan* plan, const void* x, const void* y, const vo
                  size_t workspace_bytes, int64_t rows, LunaStream stream);
 
 /* ------------------------------------------------------------------------ */
+/* Shared-weight contraction of the UVW convolution (fp32, fp64 matrix cores). */
+
+typedef struct LunaConPlan LunaConPlan;
+
+/*
+ * Per output block o (d3 components, mul3 copies) over the channels c of its
+ * paths, c = (path, v, u) and row(c) = w_off + (u * mul2 + v) * mul3:
+ *   out[n, out_off + m*d3 + k] = sum_c a[n, a_off + c*d3 + k] weight[row(c) + m]
+ * Specification (degrees up to 5):
+ *   "LUNACON1 <dtype_bits> <aggregate_dim> <out_dim> <weight_numel> <nblocks>"
+ *   then per block "<out_off> <a_off> <d3> <mul3> <npaths> (<w_off> <mul1> <mul2>)*npaths"
+ * Columns of out (or a, for the gradient) outside every block are not written.
+ * replaces: the per-edge weight contraction of the UVW convolution
+ * (src/lunatp/uvw_conv/interface.py:190-245)
+ */
+int luna_con_plan_create(const char* spec, const char* cache_dir, LunaConPlan** plan);
+int luna_con_plan_destroy(LunaConPlan* plan);
+int luna_con_plan_precompile(LunaConPlan* plan);
+int luna_con_fwd(const LunaConPlan* plan, const void* a, const void* weight, void* out, int64_t rows,
+                 LunaStream stream);
+/* ga[n, a_off + c*d3 + k] = sum_m g[n, out_off + m*d3 + k] weight[row(c) + m]. */
+int luna_con_grad_a(const LunaConPlan* plan, const void* g, const void* weight, void* ga, int64_t rows,
+                    LunaStream stream);
+/* gw[row(c) + m] = sum_{n,k} a[n, a_off + c*d3 + k] g[n, out_off + m*d3 + k] through
+ * partial tiles in `workspace` (luna_con_grad_w_workspace bytes). */
+int luna_con_grad_w_workspace(const LunaConPlan* plan, int64_t rows, size_t* bytes);
+int luna_con_grad_w(const LunaConPlan* plan, const void* a, const void* g, void* gw, void* workspace,
+                    size_t workspace_bytes, int64_t rows, LunaStream stream);
+
+/* ------------------------------------------------------------------------ */
 /* UUU (channel-wise) tensor-product convolution.                            */
 
 typedef struct LunaUuuPlan LunaUuuPlan;

@@ -47,6 +47,13 @@ PROTOTYPES = {
     "luna_uvw_fwd": (ctypes.c_int, [_VP] * 5 + [_I64, _VP]),
     "luna_uvw_bwd_workspace": (ctypes.c_int, [_VP, _I64, ctypes.POINTER(ctypes.c_size_t)]),
     "luna_uvw_bwd": (ctypes.c_int, [_VP] * 9 + [ctypes.c_size_t, _I64, _VP]),
+    "luna_con_plan_create": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(_VP)]),
+    "luna_con_plan_destroy": (ctypes.c_int, [_VP]),
+    "luna_con_plan_precompile": (ctypes.c_int, [_VP]),
+    "luna_con_fwd": (ctypes.c_int, [_VP] * 4 + [_I64, _VP]),
+    "luna_con_grad_a": (ctypes.c_int, [_VP] * 4 + [_I64, _VP]),
+    "luna_con_grad_w_workspace": (ctypes.c_int, [_VP, _I64, ctypes.POINTER(ctypes.c_size_t)]),
+    "luna_con_grad_w": (ctypes.c_int, [_VP] * 5 + [ctypes.c_size_t, _I64, _VP]),
     "luna_uuu_plan_create": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(_VP)]),
     "luna_uuu_plan_create_ex": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_char_p, ctypes.c_int, ctypes.POINTER(_VP)]),
     "luna_uuu_plan_destroy": (ctypes.c_int, [_VP]),

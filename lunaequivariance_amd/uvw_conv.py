@@ -16,23 +16,26 @@ convolution whose weights are all one (a single broadcast weight row, never
 read per edge) and whose output keeps every edge channel v in its own block;
 it runs on the HIP UVU kernels.  The contraction with ``W_p`` then happens
 once per node instead of once per edge: the paths into one output block are
-contiguous columns of A, so each output block is one batched library GEMM
-(``W_o^T [mul3, C] @ A_o [N, C, d3]``, C = the sum of mul1 * mul2 over its
-paths), which lands directly in the output layout.  Per-edge weights cannot be
+contiguous columns of A, and the contraction kernels (``csrc/contract.cpp``, fp32
+and fp64 matrix cores) take every block ``W_o^T [mul3, C] @ A_o [N, C, d3]``
+(C = the sum of mul1 * mul2 over its paths) in one launch, reading A and
+writing the output in their own layouts.  Per-edge weights cannot be
 moved out of the edge sum: the same kernels aggregate over a graph whose
 destinations are the edges themselves (``Z`` per edge), the per-edge
 contraction is a batched GEMM, and the messages are summed at destinations.
 
 Every piece is differentiable (the UVU autograd classes for the aggregation,
-torch for the GEMMs and the sum), so derivatives of every order follow.
+the contraction's three bilinear maps, torch for the batched GEMM and the sum), so derivatives of every order follow.
 """
 
 from __future__ import annotations
 
+import ctypes
 from math import prod
 
 import torch
 
+from . import _native
 from .tracing import recording
 from .cg import sparse_terms
 from .graph import LunaTPGraph, make_graph
@@ -80,6 +83,95 @@ def _rows_times_weight(rows, weight):
     if recording():
         return rows @ weight
     return _RowsTimesWeight.apply(rows, weight)
+
+
+class NativeContraction:
+    """Owner of one C-ABI contraction plan (``luna_con_*``): every output block of an
+    operator in one launch, on the layouts of the aggregate and of the output."""
+
+    MAX_COMPONENTS = 11  # output blocks of degree 5; wider ones take the library products
+
+    def __init__(self, op):
+        self.adim, self.out_dim, self.weight_numel = op.aggregate_dim, op.out_dim, op.weight_numel
+        self.dtype = op.compute_dtype
+        bits = 64 if op.compute_dtype == torch.float64 else 32
+        lines = [f"LUNACON1 {bits} {self.adim} {self.out_dim} {self.weight_numel} {len(op.blocks)}"]
+        for blk in op.blocks:
+            paths = [p for p in op.paths if p["out_off"] == blk["out_off"]]
+            lines.append(f"{blk['out_off']} {blk['a_lo']} {blk['d3']} {blk['mul3']} {len(paths)} "
+                         + " ".join(f"{p['w_off']} {p['mul1']} {p['mul2']}" for p in paths))
+        covered = sum(blk["mul3"] * blk["d3"] for blk in op.blocks)
+        self.out_factory = torch.empty if covered == self.out_dim else torch.zeros
+        handle = ctypes.c_void_p()
+        lib = _native.lib()
+        _native.check(lib.luna_con_plan_create("\n".join(lines).encode(), _native.cache_dir().encode(),
+                                               ctypes.byref(handle)), "luna_con_plan_create")
+        self.handle = handle
+
+    def precompile(self):
+        _native.check(_native.lib().luna_con_plan_precompile(self.handle), "luna_con_plan_precompile")
+
+    def _check(self, *tensors):
+        for t in tensors:
+            if not t.is_cuda or t.device != tensors[0].device:
+                raise RuntimeError("UVW convolution operands must be on one GPU")
+            if t.dtype != self.dtype:
+                raise TypeError(f"expected {self.dtype}, got {t.dtype}")
+
+    def run(self, kind, a, b):
+        """"out": (A, W) -> out; "a": (g, W) -> gA; "w": (A, g) -> gW."""
+        self._check(a, b)
+        a, b = a.contiguous(), b.contiguous()
+        lib, rows, stream = _native.lib(), a.shape[0], torch.cuda.current_stream(a.device).cuda_stream
+        like = dict(device=a.device, dtype=a.dtype)
+        if kind == "w":
+            out = torch.empty((self.weight_numel,), **like)
+            size = ctypes.c_size_t()
+            _native.check(lib.luna_con_grad_w_workspace(self.handle, rows, ctypes.byref(size)),
+                          "luna_con_grad_w_workspace")
+            workspace = torch.empty((size.value,), device=a.device, dtype=torch.uint8)
+            _native.check(lib.luna_con_grad_w(self.handle, a.data_ptr(), b.data_ptr(), out.data_ptr(),
+                                              workspace.data_ptr(), size.value, rows, stream), "luna_con_grad_w")
+            return out
+        if kind == "out":
+            out, call = self.out_factory((rows, self.out_dim), **like), lib.luna_con_fwd
+        else:  # A's columns are covered by the blocks by construction
+            out, call = torch.empty((rows, self.adim), **like), lib.luna_con_grad_a
+        _native.check(call(self.handle, a.data_ptr(), b.data_ptr(), out.data_ptr(), rows, stream), "luna_con")
+        return out
+
+    def __del__(self):
+        handle = getattr(self, "handle", None)
+        try:
+            if handle is not None and _native._lib is not None:
+                _native._lib.luna_con_plan_destroy(handle)
+        except Exception:  # interpreter shutdown
+            pass
+        self.handle = None
+
+
+class _Contract(torch.autograd.Function):
+    """One of the three bilinear maps of the contraction.  out, gA and gW are each linear in
+    both operands, and each map's derivatives are the other two, so every order follows."""
+
+    @staticmethod
+    def forward(ctx, plan, kind, a, b):
+        ctx.plan, ctx.kind = plan, kind
+        ctx.save_for_backward(a, b)
+        return plan.run(kind, a, b)
+
+    @staticmethod
+    def backward(ctx, r):
+        a, b = ctx.saved_tensors
+        plan, kind = ctx.plan, ctx.kind
+        need_a, need_b = ctx.needs_input_grad[2:]
+        apply = lambda *args: _Contract.apply(plan, *args)  # noqa: E731
+        if kind == "out":    # (A, W), r along out
+            return None, None, apply("a", r, b) if need_a else None, apply("w", a, r) if need_b else None
+        if kind == "a":      # (g, W), r along A
+            return None, None, apply("out", r, b) if need_a else None, apply("w", r, a) if need_b else None
+        # (A, g), r along W
+        return None, None, apply("a", b, r) if need_a else None, apply("out", a, r) if need_b else None
 
 
 class LunaTPUVWConv:
@@ -172,6 +264,10 @@ class LunaTPUVWConv:
                     "broadcast_weights": True}
             self.agg = LunaTPUVUConv(meta, dtype=dtype)
         self._ones = {}
+        self._contraction = None
+        # Every output block whose degree the contraction kernels stage.
+        self.native_contraction = bool(self.blocks) and all(
+            blk["d3"] <= NativeContraction.MAX_COMPONENTS for blk in self.blocks)
         # The reference's "paths" configuration string, the constant a compiled
         # graph passes to lunatp::uvw_conv_* (built here, outside tracing).
         from .ops import paths_config
@@ -182,7 +278,14 @@ class LunaTPUVWConv:
         state = dict(self.__dict__)
         state["_ones"] = {}
         state["_perm_cache"] = {}
+        state["_contraction"] = None
         return state
+
+    @property
+    def contraction(self) -> NativeContraction:
+        if self._contraction is None:
+            self._contraction = NativeContraction(self)
+        return self._contraction
 
     def _unit_weights(self, like):
         key = (like.device, like.dtype)
@@ -205,10 +308,13 @@ class LunaTPUVWConv:
         """out[n, o + w*d3 + k] = sum_c W[c, w] A[n, c, k] per output block; weight is the
         shared row [weight_numel] or per-row [rows, weight_numel].
 
-        Shared weights: one 2-D GEMM per block over rows (n, k), [rows * d3, C] x [C, mul3],
-        so the weight gradient is also one GEMM.  Per-row weights: a batched GEMM.  The
-        blocks are taken with one split (its backward is one concatenation).
+        Shared weights: the contraction kernels (csrc/contract.cpp), every block in one
+        launch.  Output degrees above 5: one library 2-D GEMM per block over rows (n, k),
+        [rows * d3, C] x [C, mul3].  Per-row weights: a batched GEMM.  The blocks are taken
+        with one split (its backward is one concatenation).
         """
+        if weight.dim() == 1 and self.native_contraction:
+            return _Contract.apply(self.contraction, "out", values, weight)
         key = weight.device
         if key not in self._perm_cache:
             self._perm_cache[key] = self._perm.to(weight.device)
