@@ -53,6 +53,7 @@ struct Options {
   int fwd_prefetch = 1;  // edge-loop software pipelining depth (0 none, 1 x/w, 2 all operands)
   int bwd_prefetch = 2;
   int prefetch = 0;      // the level of the kernel being emitted
+  int packed_prefetch = 2;  // the level of packed and split forward groups
   int fwd_depth = 1;     // edges in flight with prefetch level 2 (1 or 2)
   int bwd_depth = 1;
   int depth = 1;
@@ -98,6 +99,7 @@ Options options() {
     return at == std::string::npos ? fallback : std::atoi(s.c_str() + at + k.size());
   };
   o.fwd_prefetch = value("fpre", o.fwd_prefetch);
+  o.packed_prefetch = value("ppre", o.packed_prefetch);
   o.fwd_depth = value("fdepth", o.fwd_depth);
   o.bwd_depth = value("bdepth", o.bwd_depth);
   o.fwd_nt_w = value("fntw", o.fwd_nt_w) != 0;
@@ -255,6 +257,36 @@ std::string emit_lds_reduce(Code& c, const std::vector<std::string>& names, cons
   return std::string(prefix) + "s";
 }
 
+// The reduction for a wave that holds several edges (lane = edge * cw +
+// channel): the sums of every edge and column, 64 / (edges * columns) lanes per
+// sum, or several rounds where there are more than 64 sums.  Calls
+// store(edge-of-wave, column rank, total, condition) per round.
+void emit_packed_reduce(Code& c, const std::vector<std::string>& names, const char* prefix, int cw,
+                        const std::function<void(const char*, const char*, const char*, const char*)>& store) {
+  const int n = (int)names.size(), pitch = reduce_pitch(n), edges = 64 / cw;
+  int cols = 1;
+  while (cols < n) cols *= 2;
+  const int sums = edges * cols, lanes = std::max(1, 64 / sums), rounds = std::max(1, sums / 64);
+  const int rows = cw / lanes;
+  for (int v = 0; v < n; ++v) c.line("        red[lane * %d + %d] = %s;", pitch, v, names[v].c_str());
+  c.line("        asm volatile(\"\" ::: \"memory\");");
+  for (int r = 0; r < rounds; ++r) {
+    c.line("        {");
+    c.line("          const int %so = %d + lane / %d, %se = %so / %d, %sr = %so %% %d, %sp = lane %% %d;", prefix, r * 64,
+           lanes, prefix, prefix, cols, prefix, prefix, cols, prefix, lanes);
+    c.line("          const int %sb = (%se * %d + %sp) * %d + min(%sr, %d);", prefix, prefix, cw, prefix, pitch, prefix,
+           n - 1);
+    c.line("          real %ss = red[%sb];", prefix, prefix);
+    for (int q = 1; q < rows; ++q) c.line("          %ss += red[%sb + %d];", prefix, prefix, q * lanes * pitch);
+    for (int m = lanes / 2; m >= 1; m /= 2) c.line("          %ss += xchg<%d>(%ss);", prefix, m, prefix);
+    const std::string e = std::string(prefix) + "e", rank = std::string(prefix) + "r", sum = std::string(prefix) + "s";
+    const std::string own = std::string(prefix) + "p == 0 && " + rank + " < " + std::to_string(n);
+    store(e.c_str(), rank.c_str(), sum.c_str(), own.c_str());
+    c.line("        }");
+  }
+  c.line("        asm volatile(\"\" ::: \"memory\");");
+}
+
 // (i, j) pairs of one path grouped by their coefficient vector over k, equal
 // up to a global sign (relative tolerance 1e-12 absorbs last-bit differences
 // between equal Clebsch-Gordan values).
@@ -322,11 +354,22 @@ struct YCopies {
 //   just issued (vmcnt counts loads and stores in issue order).
 // depth 2 (with prefetch 2): two edges in flight, from two register buffers
 //   used alternately by a loop unrolled twice.
+//
+// Packed groups (cw < 64) take 64 / cw edges per iteration, so the edge, its
+// source and its y row differ between the lanes (vector loads); lanes past the
+// last edge repeat it with ok == false.  One edge at a time, a block of 32
+// channels ran half of its lanes idle and its weight rows as 128-byte requests:
+// 1,000 nodes, 52,000 edges, lmax 2, 32 channels, forward 76 -> 31 us (100 MB of
+// weights, 3.4 TB/s), backward 81 -> 64 us (4.2 TB/s).  `split`: the workgroup's
+// waves take the iterations in turn.
 void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& use, bool env,
                     const Options& opt, const std::vector<std::string>& resident,
-                    const std::function<void()>& body) {
+                    const std::function<void()>& body, bool split = false) {
   const int np = (int)g.paths.size();
+  const int nsub = 64 / g.cw;
+  const bool packed = nsub > 1;
   const bool full = opt.prefetch >= 2;
+  const char cls = packed ? 'v' : 's';
   auto load_edge = [&](const char* edge, const char* srcv, char b) {
     c.line("      {");
     c.line("        const real* xq = x + (i64)%s * IN1 + (%d + uc * %d);", srcv, g.x_off, g.d1);
@@ -365,9 +408,11 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
   auto waits = [&](char b) {
     for (int i = 0; i < g.d1; ++i) c.line("      asm volatile(\"\" :: \"v\"(%cx%d));", b, i);
     for (int n = 0; n < np; ++n) c.line("      asm volatile(\"\" :: \"v\"(%cw%d));", b, n);
-    for (int yi : use.ys) c.line("      asm volatile(\"\" :: \"s\"(%cy%d));", b, yi);
-    if (env) c.line("      asm volatile(\"\" :: \"s\"(%cev));", b);
-    c.line("      asm volatile(\"\" :: \"s\"(sn));");
+    if (full) {
+      for (int yi : use.ys) c.line("      asm volatile(\"\" :: \"%c\"(%cy%d));", cls, b, yi);
+      if (env) c.line("      asm volatile(\"\" :: \"%c\"(%cev));", cls, b);
+    }
+    c.line("      asm volatile(\"\" :: \"%c\"(sn));", cls);
   };
   auto inline_y = [&]() {
     c.line("      const real* yr = y + (i64)e * IN2;");
@@ -378,6 +423,35 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
     for (const auto& name : resident) c.line("      asm volatile(\"\" :: \"v\"(%s));", name.c_str());
   };
 
+  if (packed || split) {
+    const std::string step = split ? std::to_string(nsub) + " * split" : std::to_string(nsub);
+    const std::string lane_edge = packed ? " + sub" : "";
+    auto clamped = [&](const std::string& edge) {
+      return "(" + edge + lane_edge + " < end ? " + edge + lane_edge + " : end - 1)";
+    };
+    c.line("    const eix first = %s;", split ? ("beg + part * " + std::to_string(nsub)).c_str() : "beg");
+    c.line("    if (first < end) {");
+    declare('n');
+    c.line("      int sn = src[%s];", clamped("first").c_str());
+    load_edge(clamped("first").c_str(), "sn", 'n');
+    c.line("      sn = src[%s];", clamped("first + " + step).c_str());
+    waits('n');
+    resident_waits();
+    if (packed) c.line("      int it = 0;");
+    c.line("      for (eix e0 = first; e0 < end; e0 += %s%s) {", step.c_str(), packed ? ", ++it" : "");
+    c.line("      const eix e = %s;", clamped("e0").c_str());
+    if (packed) c.line("      const bool ok = e0 + sub < end;");
+    bind('n');
+    c.line("      const eix en = %s;", clamped("e0 + " + step).c_str());
+    load_edge("en", "sn", 'n');
+    c.line("      sn = src[%s];", clamped("e0 + 2 * " + step).c_str());
+    if (!full) inline_y();
+    body();
+    waits('n');
+    c.line("      }");
+    c.line("    }");
+    return;
+  }
   if (opt.prefetch == 0) {
     c.line("    {");
     c.line("      for (eix e = beg; e < end; ++e) {");
@@ -461,16 +535,32 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
   c.line("    }");
 }
 
-void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt) {
+// Channel u (uc: clamped to the last) of this lane, and the edge of the wave it
+// works on (`sub`) in a packed group.
+void emit_lanes(Code& c, const Group& g, int slot_base, int subsets) {
+  const std::string chunk = subsets > 1 ? "((slot - " + std::to_string(slot_base) + ") / " + std::to_string(subsets) + ")"
+                                        : "(slot - " + std::to_string(slot_base) + ")";
+  if (g.cw < 64) {
+    c.line("    const int u = %s * %d + lane %% %d;", chunk.c_str(), g.cw, g.cw);
+    c.line("    const int sub = lane / %d;", g.cw);
+  } else {
+    c.line("    const int u = %s * 64 + lane;", chunk.c_str());
+  }
+  c.line("    const bool active = u < %d;", g.channels);
+  c.line("    const int uc = active ? u : %d;", g.channels - 1);
+}
+
+void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt,
+                        bool split) {
   const int bits = spec.dtype_bits;
   GroupUse use = group_use(spec, g);
   const int np = (int)g.paths.size();
-  c.line("    const int u = (slot - %d) * 64 + lane;", g.slot_base);
-  c.line("    const bool active = u < %d;", g.channels);
-  c.line("    const int uc = active ? u : %d;", g.channels - 1);
+  const bool packed = g.cw < 64;
+  emit_lanes(c, g, g.slot_base, 1);
   for (size_t b = 0; b < g.blocks.size(); ++b)
     for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
   auto body = [&]() {
+  if (packed) c.line("      if (ok) {");
   // l0 columns are summed over the paths (edge copies) sharing them.
   std::map<int, std::vector<int>> l0_cols;
   for (int n = 0; n < np; ++n) {
@@ -544,8 +634,37 @@ void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, boo
   }
   for (const auto& col : l0_cols)
     c.line("      l0[(i64)e * L0DIM + %d + uc] = L%d;", col.first, col.first);
+  if (packed) c.line("      }");
   };
-  emit_edge_loop(c, spec, g, use, env, opt, {}, body);
+  emit_edge_loop(c, spec, g, use, env, opt, {}, body, split);
+  if (packed || split) {
+    // The sums of a wave's edges, and of the waves sharing the node, meet in
+    // LDS: piece q (wave and edge of the wave) holds its cw * d3 values in the
+    // order they are stored.
+    const char* pieces = split ? "split" : "1";
+    c.line("    {");
+    c.line("      const int c0 = (slot - %d) * %d;", g.slot_base, g.cw);
+    c.line("      const int nch = %d - c0 < %d ? %d - c0 : %d;", g.channels, g.cw, g.channels, g.cw);
+    for (size_t b = 0; b < g.blocks.size(); ++b) {
+      const AccBlock& blk = g.blocks[b];
+      for (int k = 0; k < blk.d3; ++k)
+        c.line("      obuf[(%slane) * %d + %d] = A%zu_%d;", split ? "part * 64 + " : "", blk.d3, k, b, k);
+      c.line(split ? "      __syncthreads();" : "      __builtin_amdgcn_wave_barrier();");
+      c.line("      {");
+      c.line("        real* ob = out + (i64)t * OUTD + (%d + c0 * %d);", blk.out_off, blk.d3);
+      c.line("        for (int i = %s; i < nch * %d; i += 64%s) {", split ? "(int)threadIdx.x" : "lane", blk.d3,
+             split ? " * split" : "");
+      c.line("          real v = obuf[i];");
+      c.line("          #pragma unroll %d", split ? 2 : 64 / g.cw);
+      c.line("          for (int q = 1; q < %s * %d; ++q) v += obuf[q * %d + i];", pieces, 64 / g.cw, g.cw * blk.d3);
+      c.line(blk.accumulate ? "          ob[i] += v;" : "          __builtin_nontemporal_store(v, ob + i);");
+      c.line("        }");
+      c.line("      }");
+      c.line(split ? "      __syncthreads();" : "      __builtin_amdgcn_wave_barrier();");
+    }
+    c.line("    }");
+    return;
+  }
   if (!opt.out_lds) {
     c.line("    if (active) {");
     for (size_t b = 0; b < g.blocks.size(); ++b) {
@@ -612,12 +731,9 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   GroupUse use = group_use(spec, g);
   const int np = (int)g.paths.size();
   const bool lds_reduce = opt.lds_reduce != 0;
-  if (g.subsets > 1)
-    c.line("    const int u = ((slot - %d) / %d) * 64 + lane;", g.slot_base, g.subsets);
-  else
-    c.line("    const int u = (slot - %d) * 64 + lane;", g.slot_base);
-  c.line("    const bool active = u < %d;", g.channels);
-  c.line("    const int uc = active ? u : %d;", g.channels - 1);
+  const bool packed = g.cw < 64;
+  const int nsub = 64 / g.cw;
+  emit_lanes(c, g, g.slot_base, g.subsets);
   std::vector<std::string> seeds;
   for (size_t b = 0; b < g.blocks.size(); ++b) {
     const AccBlock& blk = g.blocks[b];
@@ -708,7 +824,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   // index, env last) of both subsets' partials; r0 / r1 are that column's
   // positions in the two subsets' value lists (-1: not there).
   const bool combine = whole && whole->combine_subsets && want_part;
-  if (combine && sub == 0) {
+  if (combine && sub == 0 && !packed) {
     for (int s2 = 0; s2 < 2; ++s2) {
       const GroupUse other = group_use(spec, subset_view(*whole, s2));
       std::string chain = "-1";
@@ -744,6 +860,16 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     const std::string tag = "r" + std::to_string(flush_id++) + "_";
     c.line("      {");
     for (const auto& v : values) c.line("        %s = active ? %s : (real)0;", v.c_str(), v.c_str());
+    if (packed) {
+      emit_packed_reduce(c, values, tag.c_str(), g.cw,
+                         [&](const char* edge, const char* rank, const char* total, const char* own) {
+        c.line("          if (%s && e0 + %s < end)", own, edge);
+        c.line("            part[((i64)(%d + (slot - %d)) * E + (e0 + %s)) * PART_W + %d + %s] = %s;", g.gy_slot_base,
+               g.slot_base, edge, column[values[0]], rank, total);
+      });
+      c.line("      }");
+      return;
+    }
     int shift = 0, low = 0;
     std::string total = lds_reduce ? emit_lds_reduce(c, values, tag.c_str(), &shift, &low)
                                    : emit_butterfly(c, values, tag.c_str(), &shift, &low);
@@ -769,6 +895,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     }
     c.line("      }");
   };
+  if (packed) c.line("      if (ok) {");
   for (int n = 0; n < np; ++n) {
     const Path& q = spec.paths[g.paths[n]];
     const int b = g.path_block[n];
@@ -863,6 +990,8 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     for (int i : is) c.line("        M%d = FMA(ws, a%d, M%d);", i, i, i);
     c.line("      }");
   }
+  if (packed) c.line("      }");
+  const std::string parity = packed ? "it & 1" : "(e - beg) & 1";
   std::vector<std::string> values;
   for (int yi : use.ys) values.push_back("GY" + std::to_string(yi));
   if (env) values.push_back("GE");
@@ -872,8 +1001,22 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   auto reduce_to_lds = [&]() {
     c.line("      {");
     for (const auto& v : values) c.line("        %s = active ? %s : (real)0;", v.c_str(), v.c_str());
-    int shift = 0, low = 0;
     const std::string tag = "s" + std::to_string(sub) + "_";
+    if (packed) {
+      // Every column at its own place (the y index, env last) of its edge.
+      std::string place;
+      int rank = 0;
+      for (int yi : use.ys) place += "rank == " + std::to_string(rank++) + " ? " + std::to_string(yi) + " : ";
+      emit_packed_reduce(c, values, tag.c_str(), g.cw,
+                         [&](const char* edge, const char* r, const char* total, const char* own) {
+        c.line("          { const int rank = %s;", r);
+        c.line("          if (%s) gy_sub[%d][%s][%s * PART_W + (%s%d)] = %s; }", own, sub, parity.c_str(), edge,
+               place.c_str(), (int)spec.in2, total);
+      });
+      c.line("      }");
+      return;
+    }
+    int shift = 0, low = 0;
     std::string total = lds_reduce ? emit_lds_reduce(c, values, tag.c_str(), &shift, &low)
                                    : emit_butterfly(c, values, tag.c_str(), &shift, &low);
     c.line("        const int col = lane >> %d;", shift);
@@ -885,7 +1028,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     // The second subset hands its message share to the first through LDS
     // (two buffers by edge parity: one barrier per edge orders both uses).
     c.line("      {");
-    c.line("        const int par = (e - beg) & 1;");
+    c.line("        const int par = %s;", parity.c_str());
     if (sub == 1) {
       if (want_msg)
         for (int i = 0; i < g.d1; ++i) c.line("        msg_share[par][%d][lane] = M%d;", i, i);
@@ -905,7 +1048,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     // one contiguous 256-byte run (full-line stores; the x layout, d1 values
     // per lane, made every store a strided partial-line write).
     const int stride = cmajor ? g.channels : 1;
-    c.line("      {");
+    c.line(packed ? "      if (ok) {" : "      {");
     if (cmajor)
       c.line("        real* mr = msg + (i64)e * IN1 + (%d + uc);", g.x_off);
     else
@@ -920,7 +1063,23 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     }
     c.line("      }");
   }
-  if (combine && sub == 0) {
+  if (combine && sub == 0 && packed) {
+    reduce_to_lds();
+    auto present = [&](int s2) {
+      std::string mask;
+      for (int yi : group_use(spec, subset_view(*whole, s2)).ys) mask += "col == " + std::to_string(yi) + " || ";
+      return mask + (env ? "col == " + std::to_string((int)spec.in2) : std::string("false"));
+    };
+    c.line("      asm volatile(\"\" ::: \"memory\");");
+    c.line("      for (int o = lane; o < %d * (int)PART_W; o += 64) {", nsub);
+    c.line("        const int par = it & 1, edge = o / (int)PART_W, col = o %% (int)PART_W;");
+    c.line("        const bool a = %s, b = %s;", present(0).c_str(), present(1).c_str());
+    c.line("        if ((a || b) && e0 + edge < end)");
+    c.line("          part[((i64)(%d + (slot - %d) / 2) * E + (e0 + edge)) * PART_W + col] =", whole->gy_slot_base,
+           whole->slot_base);
+    c.line("              (a ? gy_sub[0][par][o] : (real)0) + (b ? gy_sub[1][par][o] : (real)0);");
+    c.line("      }");
+  } else if (combine && sub == 0) {
     reduce_to_lds();
     c.line("      {");
     c.line("        const int par = (e - beg) & 1;");
@@ -978,7 +1137,15 @@ std::string kernel_attributes(int wpe) {
 
 }  // namespace
 
-std::string emit_forward(const Plan& plan, bool env, bool l0) {
+int split_forward_lds(const Plan& plan, int phase) {
+  int max_d3 = 1;
+  for (const Group& g : plan.fwd_groups)
+    if (g.phase == phase)
+      for (const auto& b : g.blocks) max_d3 = std::max(max_d3, b.d3);
+  return 64 * max_d3;
+}
+
+std::string emit_forward(const Plan& plan, bool env, bool l0, bool split) {
   const Spec& spec = plan.spec;
   Options opt = options();
   opt.prefetch = opt.fwd_prefetch;
@@ -987,22 +1154,27 @@ std::string emit_forward(const Plan& plan, bool env, bool l0) {
   Code c;
   c.raw(prelude(spec, plan.edge_index_bits));
   for (int phase = 0; phase < plan.fwd_phases; ++phase) {
-    const int waves = plan.fwd_block_waves[phase], slots = plan.phase_slots[phase];
-    c.line("extern \"C\" __global__ void __launch_bounds__(%d) %sluna_uvu_fwd_p%d(", 64 * std::max(waves, 1),
-           kernel_attributes(opt.fwd_wpe).c_str(), phase);
+    const int waves = split ? 1 : plan.fwd_block_waves[phase], slots = plan.phase_slots[phase];
+    c.line("extern \"C\" __global__ void __launch_bounds__(%d) %sluna_uvu_fwd_p%d(",
+           split ? 512 : 64 * std::max(waves, 1), kernel_attributes(opt.fwd_wpe).c_str(), phase);
     c.line("    const real* __restrict__ x, const real* __restrict__ y, const real* __restrict__ w,");
     c.line("    const real* __restrict__ env, const int* __restrict__ src, const eix* __restrict__ rowptr,");
     c.line("    const int* __restrict__ order, real* __restrict__ out, real* __restrict__ l0) {");
-    if (opt.out_lds) {
-      int max_d3 = 1;
-      for (const Group& g : plan.fwd_groups)
-        if (g.phase == phase)
-          for (const auto& b : g.blocks) max_d3 = std::max(max_d3, b.d3);
-      c.line("  __shared__ __attribute__((aligned(16))) real obuf_lds[%d];", std::max(waves, 1) * 64 * max_d3);
+    if (split) {
+      c.line("  extern __shared__ __attribute__((aligned(16))) unsigned char obuf_lds[];");
+      c.line("  real* const obuf = (real*)obuf_lds;");
+    } else {
+      const int per = split_forward_lds(plan, phase);
+      c.line("  __shared__ __attribute__((aligned(16))) real obuf_lds[%d];", std::max(waves, 1) * per);
       c.line("  real* const obuf = obuf_lds + %s * %d;",
-             waves > 0 ? "__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)" : "0", 64 * max_d3);
+             waves > 0 ? "__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)" : "0", per);
     }
-    if (waves == 0) {
+    if (split) {
+      c.line("  const int lane = threadIdx.x & 63;");
+      c.line("  const int split = blockDim.x >> 6, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);");
+      c.line("  const int slot = blockIdx.y;");
+      c.line("  const int t = order[blockIdx.x];");
+    } else if (waves == 0) {
       // One wave per workgroup, the slots of a node on consecutive workgroups.
       c.line("  const int lane = threadIdx.x;");
       c.line("  const int t = order[blockIdx.x / %d];", slots);
@@ -1021,7 +1193,9 @@ std::string emit_forward(const Plan& plan, bool env, bool l0) {
       if (g.phase != phase) continue;
       c.line("  %sif (slot < %d) {", first ? "" : "else ", g.slot_base + g.chunks);
       first = false;
-      emit_forward_group(c, spec, g, env, l0, opt);
+      Options own = opt;
+      if (g.cw < 64 || split) own.prefetch = opt.packed_prefetch;
+      emit_forward_group(c, spec, g, env, l0, own, split);
       c.line("  }");
     }
     c.line("}");
@@ -1057,8 +1231,15 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
     if (pairs && want_part) c.line("  __shared__ real gy_share[2][PART_W];");
     bool combined = false;
     for (const Group& g : plan.bwd_groups) combined = combined || (g.phase == phase && g.combine_subsets);
-    if (combined && want_part) c.line("  __shared__ real gy_sub[2][2][PART_W];");
-    if (want_part && opt.lds_reduce != 0) {
+    if (combined && want_part) {
+      int nsub = 1;
+      for (const Group& g : plan.bwd_groups)
+        if (g.phase == phase && g.combine_subsets) nsub = std::max(nsub, 64 / g.cw);
+      c.line("  __shared__ real gy_sub[2][2][%d * PART_W];", nsub);
+    }
+    bool packed = false;
+    for (const Group& g : plan.bwd_groups) packed = packed || (g.phase == phase && g.cw < 64);
+    if (want_part && (packed || opt.lds_reduce != 0)) {
       // Per-wave table of the LDS reduction of the gy partials.
       int most = 1;
       for (const Group& g : plan.bwd_groups)
@@ -1080,8 +1261,14 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
       c.line("  const int t = order[blockIdx.x];");
       c.line("  const int slot = blockIdx.y * %d + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);", waves);
     }
-    c.line("  const eix beg = rowptr[t];");
-    c.line("  const eix end = rowptr[t + 1];");
+    // Few nodes: a grid of more than one layer cuts every node's edges into as
+    // many runs (nothing is summed over a node's edges here).
+    c.line("  eix beg = rowptr[t], end = rowptr[t + 1];");
+    c.line("  if (gridDim.z > 1) {");
+    c.line("    const eix run = (end - beg + (eix)gridDim.z - 1) / (eix)gridDim.z;");
+    c.line("    beg += run * (eix)blockIdx.z;");
+    c.line("    end = beg + run < end ? beg + run : end;");
+    c.line("  }");
     bool first = true;
     for (const Group& g : plan.bwd_groups) {
       if (g.phase != phase) continue;
@@ -1233,13 +1420,22 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
   const char* vtype = vec == 1 ? "real"
                                : (spec.dtype_bits == 64 ? "double __attribute__((ext_vector_type(2)))"
                                                         : "float __attribute__((ext_vector_type(4)))");
-  c.line("extern \"C\" __global__ void __launch_bounds__(256) luna_uvu_bwd_gather(");
+  // A workgroup takes gather_columns() vectors of one source row; narrow rows
+  // leave room for several teams of threads, which share the source's edges
+  // and add up through LDS.
+  const int cols = gather_columns(plan), teams = gather_teams(plan);
+  c.line("extern \"C\" __global__ void __launch_bounds__(%d) luna_uvu_bwd_gather(", cols * teams);
   c.line("    const real* __restrict__ msg, const eix* __restrict__ srow, const eix* __restrict__ ebs,");
   c.line("    real* __restrict__ gx) {");
   c.line("  typedef %s vec_t;", vtype);
   c.line("  const int s = blockIdx.x;");
-  c.line("  const int col = (blockIdx.y * 256 + threadIdx.x) * %d;", vec);
-  c.line("  if (col >= IN1) return;");
+  if (teams > 1) {
+    c.line("  __shared__ vec_t share[%d];", cols * (teams - 1));
+    c.line("  const int team = threadIdx.x / %d, col = (threadIdx.x - team * %d) * %d;", cols, cols, vec);
+  } else {
+    c.line("  const int col = (blockIdx.y * %d + threadIdx.x) * %d;", cols, vec);
+    c.line("  if (col >= IN1) return;");
+  }
   const Options gopt = options();
   const int un = gopt.gather_unroll;
   auto load = [&](const std::string& row) {
@@ -1248,17 +1444,23 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
   };
   for (int n = 0; n < un; ++n) c.line("  vec_t acc%d = {};", n);
   c.line("  if (covered(col)) {");
-  c.line("    const eix beg = srow[s], end = srow[s + 1];");
+  c.line("    const eix beg = srow[s]%s, end = srow[s + 1];", teams > 1 ? " + team" : "");
   c.line("    eix p = beg;");
-  c.line("    for (; p + %d <= end; p += %d) {", un, un);
+  c.line("    for (; p + %d < end; p += %d) {", (un - 1) * teams, un * teams);
   for (int n = 0; n < un; ++n)
-    c.line("      acc%d += %s;", n, load("ebs[p + " + std::to_string(n) + "]").c_str());
+    c.line("      acc%d += %s;", n, load("ebs[p + " + std::to_string(n * teams) + "]").c_str());
   c.line("    }");
-  c.line("    for (; p < end; ++p) acc0 += %s;", load("ebs[p]").c_str());
+  c.line("    for (; p < end; p += %d) acc0 += %s;", teams, load("ebs[p]").c_str());
   c.line("  }");
   // pairwise sum of the partial accumulators
   for (int width = 1; width < un; width *= 2)
     for (int n = 0; n + width < un; n += 2 * width) c.line("  acc%d += acc%d;", n, n + width);
+  if (teams > 1) {
+    c.line("  if (team) share[threadIdx.x - %d] = acc0;", cols);
+    c.line("  __syncthreads();");
+    c.line("  if (team) return;");
+    for (int n = 1; n < teams; ++n) c.line("  acc0 += share[threadIdx.x + %d];", (n - 1) * cols);
+  }
   if (cmajor && vec > 1) {
     // The values of one vector are consecutive channels of one component:
     // their gx positions are d1 apart.

@@ -42,9 +42,11 @@ struct AccBlock {
 };
 
 // Paths sharing one input block (x_off, d1, channels), run by one wave per
-// (node, 64-channel chunk).
+// (node, chunk of `cw` channels).  A chunk narrower than 64 channels lets a wave
+// take 64 / cw edges at once: lane = edge * cw + channel.
 struct Group {
   int x_off, d1, channels, chunks;
+  int cw = 64;
   std::vector<int> paths;            // indices into Spec::paths
   std::vector<AccBlock> blocks;      // forward output blocks
   std::vector<int> path_block;       // path -> index in blocks
@@ -94,6 +96,10 @@ Spec parse_spec(const std::string& text);
 // Elements per access of the gx gather: 16-byte vectors when every covered
 // input range and the row length are multiples of it, else 1 (Plan::gather_vec).
 int gather_vector_width(const Plan& plan);
+// The gather's workgroup: vectors of a source row it covers, and the teams of
+// threads that share the row's edges where the whole row is narrow (256 threads).
+int gather_columns(const Plan& plan);
+int gather_teams(const Plan& plan);
 // True when the gx messages are stored component-major per input block
 // (msg[e, x_off + i * C + u]: every store of a wave is 64 contiguous values)
 // instead of in the x layout (msg[e, x_off + u * d1 + i]); the gather kernel
@@ -103,8 +109,11 @@ int gather_vector_width(const Plan& plan);
 bool message_component_major(const Plan& plan);
 void build_schedule(Plan& plan);
 
-// Emitted HIP source of one kernel module variant.
-std::string emit_forward(const Plan& plan, bool env, bool l0);
+// Emitted HIP source of one kernel module variant.  `split`: a workgroup's waves
+// share the edges of one (node, slot) instead of taking a slot each.
+std::string emit_forward(const Plan& plan, bool env, bool l0, bool split);
+// LDS reals per wave of the split forward.
+int split_forward_lds(const Plan& plan, int phase);
 std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bool want_msg, bool want_part);
 
 // The first-order backward launches (luna_uvu_conv_bwd without the plan

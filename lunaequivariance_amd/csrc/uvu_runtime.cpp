@@ -11,9 +11,11 @@ using namespace luna;
 namespace {
 
 std::string source_for(const Plan& plan, const std::string& variant) {
-  // Variant names: fwd<env><l0> and bwd<env><gl0><gw><msg><part>, each flag '0' or '1'.
+  // Variant names: fwd<env><l0>, fws<env><l0> (split over waves) and
+  // bwd<env><gl0><gw><msg><part>, each flag '0' or '1'.
   auto flag = [&](size_t i) { return variant.size() > i && variant[i] == '1'; };
-  if (variant.compare(0, 3, "fwd") == 0) return emit_forward(plan, flag(3), flag(4));
+  if (variant.compare(0, 3, "fwd") == 0) return emit_forward(plan, flag(3), flag(4), false);
+  if (variant.compare(0, 3, "fws") == 0) return emit_forward(plan, flag(3), flag(4), true);
   return emit_backward(plan, flag(3), flag(4), flag(5), flag(6), flag(7));
 }
 
@@ -38,6 +40,24 @@ dim3 grid_for(int64_t nodes, int slots, int waves) {
   }
   return dim3((unsigned)nodes, (unsigned)((slots + waves - 1) / waves));
 }
+
+// Pieces a node's edges are cut into when the graph alone gives few waves:
+// doubled (up to 8) until the launch holds `target` waves, while each piece
+// keeps at least four iterations of the edge loop (a piece pays for the node's
+// seeds or output again).  Targets: 4,096 waves (four per SIMD) for the
+// forward, 8,192 for the backward.  150 nodes of 128 channels, lmax 3: forward
+// 83 us whole, 46 / 44 / 45 us for targets of 2,048 / 4,096 / 8,192, backward
+// 133 us, 107 / 90 / 86 us; 1,000 nodes of 32 channels, lmax 2: forward 31, 31
+// and (8,192) 34 us, backward 68, 66, 64 us.
+int edge_split(const std::vector<Group>& groups, int phase, int64_t waves, int64_t nodes, int64_t edges, int64_t target) {
+  int at_once = 1;
+  for (const Group& g : groups)
+    if (g.phase == phase) at_once = std::max(at_once, 64 / g.cw);
+  int split = 1;
+  while (split < 8 && waves * split < target && edges >= nodes * at_once * split * 8) split *= 2;
+  return split;
+}
+constexpr int64_t kForwardWaves = 4096, kBackwardWaves = 8192;
 
 void check_sizes(const Plan& plan, int64_t num_nodes, int64_t num_edges) {
   if (num_nodes < 0 || num_edges < 0) fail("negative problem size");
@@ -90,8 +110,10 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
       for (int phase = 0; phase < plan.bwd_phases; ++phase) {
         hipFunction_t f = function_for(module, "luna_uvu_bwd_p" + std::to_string(phase));
         void* args[] = {&x, &y, &w, &env, &g, &gl0, &src, &dst_rowptr, &node_order, &gw, &msg, &part, &E};
-        launch("uvu_bwd_p" + std::to_string(phase), f,
-               grid_for(num_nodes, plan.bwd_phase_slots[phase], plan.bwd_block_waves[phase]),
+        dim3 grid = grid_for(num_nodes, plan.bwd_phase_slots[phase], plan.bwd_block_waves[phase]);
+        grid.z = edge_split(plan.bwd_groups, phase, num_nodes * plan.bwd_phase_slots[phase], num_nodes, E,
+                            kBackwardWaves);
+        launch("uvu_bwd_p" + std::to_string(phase), f, grid,
                dim3(64 * std::max(plan.bwd_block_waves[phase], 1)), s, args);
       }
     }
@@ -104,10 +126,10 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
       // With no edges the gather still writes zeros (every source row is empty).
       void* args[] = {&msg, &src_rowptr, &edge_ids_by_src, &gx};
       const int vec = gather_vector_width(plan);
-      const int64_t per_block = 256LL * vec;
+      const int64_t per_block = (int64_t)gather_columns(plan) * vec;
       launch("uvu_bwd_gather", function_for(module, "luna_uvu_bwd_gather"),
-             dim3((unsigned)num_nodes, (unsigned)((plan.spec.in1 + per_block - 1) / per_block)), dim3(256), s,
-             args);
+             dim3((unsigned)num_nodes, (unsigned)((plan.spec.in1 + per_block - 1) / per_block)),
+             dim3(gather_columns(plan) * gather_teams(plan)), s, args);
     }
 }
 
@@ -158,7 +180,7 @@ int luna_uvu_plan_info(const LunaUvuPlan* plan, LunaUvuPlanInfo* info) {
 int luna_uvu_plan_precompile(LunaUvuPlan* plan) {
   return guard_call([&] {
     if (!plan) fail("luna_uvu_plan_precompile: null plan");
-    for (const char* v : {"fwd00", "bwd00111"})
+    for (const char* v : {"fwd00", "fws00", "bwd00111"})
       plan->plan.kernels.code_for(v, [&] { return source_for(plan->plan, v); });
   });
 }
@@ -175,11 +197,21 @@ int luna_uvu_conv_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
     if (!x || !out || !dst_rowptr || !node_order) fail("luna_uvu_conv_fwd: null tensor");
     if (num_edges > 0 && (!y || !w || !src)) fail("luna_uvu_conv_fwd: null edge tensor");
     if (l0 && plan.spec.l0_dim == 0) l0 = nullptr;
-    std::string variant = std::string("fwd") + (env ? '1' : '0') + (l0 ? '1' : '0');
-    hipModule_t module = module_for(plan, variant);
     for (int phase = 0; phase < plan.fwd_phases; ++phase) {
+      int split = edge_split(plan.fwd_groups, phase, num_nodes * plan.phase_slots[phase], num_nodes, num_edges,
+                             kForwardWaves);
+      const size_t wave_lds = split_forward_lds(plan, phase) * (plan.spec.dtype_bits / 8);
+      while (split > 1 && split * wave_lds > 65536) split /= 2;
+      const std::string variant = std::string(split > 1 ? "fws" : "fwd") + (env ? '1' : '0') + (l0 ? '1' : '0');
+      hipModule_t module = module_for(plan, variant);
       hipFunction_t f = function_for(module, "luna_uvu_fwd_p" + std::to_string(phase));
       void* args[] = {&x, &y, &w, &env, &src, &dst_rowptr, &node_order, &out, &l0};
+      if (split > 1) {
+        launch("uvu_fwd_p" + std::to_string(phase), f, dim3((unsigned)num_nodes, (unsigned)plan.phase_slots[phase]),
+               dim3(64 * split), (hipStream_t)stream, args,
+               (unsigned)(split * wave_lds));
+        continue;
+      }
       launch("uvu_fwd_p" + std::to_string(phase), f,
              grid_for(num_nodes, plan.phase_slots[phase], plan.fwd_block_waves[phase]),
              dim3(64 * std::max(plan.fwd_block_waves[phase], 1)), (hipStream_t)stream, args);

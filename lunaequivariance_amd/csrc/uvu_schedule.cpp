@@ -105,9 +105,23 @@ Spec parse_spec(const std::string& text) {
 
 namespace {
 
+// Channels per chunk.  Up to 32 channels would leave half of a wave's lanes
+// idle or more, so such chunks are a power of two wide and a wave takes several
+// edges at once (at most eight).  `halves`: also cut wider blocks by 32 where
+// that saves more than an eighth of the lanes (65-96 and 129-160 channels).
+int chunk_width(int channels, bool halves) {
+  if (channels <= 32) {
+    int w = 8;
+    while (w < channels) w *= 2;
+    return w;
+  }
+  const int whole = (channels + 63) / 64 * 64, half = (channels + 31) / 32 * 32;
+  return halves && 8 * (whole - half) > whole ? 32 : kWave;
+}
+
 // Split the paths sharing one input block into groups whose output blocks fit
 // the accumulator budget.  Paths writing the same output block stay together.
-std::vector<Group> make_groups(const Spec& spec, int budget) {
+std::vector<Group> make_groups(const Spec& spec, int budget, bool halves) {
   std::map<std::tuple<int, int, int>, std::vector<int>> by_input;
   std::vector<std::tuple<int, int, int>> key_order;
   for (int p = 0; p < (int)spec.paths.size(); ++p) {
@@ -149,7 +163,8 @@ std::vector<Group> make_groups(const Spec& spec, int budget) {
       g.x_off = std::get<0>(key);
       g.d1 = std::get<1>(key);
       g.channels = std::get<2>(key);
-      g.chunks = (g.channels + kWave - 1) / kWave;
+      g.cw = chunk_width(g.channels, halves);
+      g.chunks = (g.channels + g.cw - 1) / g.cw;
       // Keep the original block order inside the bin.
       for (const auto& b : blocks) {
         if (std::find(bin.second.begin(), bin.second.end(), b) == bin.second.end()) continue;
@@ -221,6 +236,13 @@ static int compute_gather_vector_width(const Plan& plan) {
 
 bool message_component_major(const Plan& plan) { return plan.msg_cmajor; }
 int gather_vector_width(const Plan& plan) { return plan.gather_vec; }
+int gather_columns(const Plan& plan) {
+  return std::max(1, std::min(256, (plan.spec.in1 + plan.gather_vec - 1) / plan.gather_vec));
+}
+int gather_teams(const Plan& plan) {
+  const int row = (plan.spec.in1 + plan.gather_vec - 1) / plan.gather_vec;
+  return row > 128 ? 1 : std::min(16, 256 / gather_columns(plan));
+}
 
 void build_schedule(Plan& plan) {
   const Spec& spec = plan.spec;
@@ -232,7 +254,7 @@ void build_schedule(Plan& plan) {
   // have to accumulate their gx messages.
   int acc_regs = kAccumulatorRegisters;
   if (const char* e = std::getenv("LUNAEQ_AMD_FACC")) acc_regs = std::max(8, std::atoi(e));
-  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32));
+  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32), true);
   auto out_ranges = [](const Group& g) {
     std::vector<std::pair<long, long>> r;
     for (const auto& b : g.blocks) r.push_back({b.out_off, b.out_off + (long)g.channels * b.d3});
@@ -325,7 +347,7 @@ void build_schedule(Plan& plan) {
     if (s > 65535) fail("too many channel chunks for one launch");
 
   // ---- backward ----
-  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters);
+  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters, false);
   auto in_ranges = [](const Group& g) {
     return std::vector<std::pair<long, long>>{{g.x_off, g.x_off + (long)g.channels * g.d1}};
   };
@@ -388,6 +410,8 @@ void build_schedule(Plan& plan) {
   int bwd_limit = limit;
   if (const char* e = std::getenv("LUNAEQ_AMD_BWG")) bwd_limit = std::max(0, std::min(16, std::atoi(e)));
   for (int s : plan.bwd_phase_slots) plan.bwd_block_waves.push_back(any_split ? 2 : std::min(s, bwd_limit));
+  // (Blocks of 65-96 channels keep two chunks here: three of 32 would need a
+  // partial slot each, a larger workspace.)
   // A group whose two chunks are the two waves of one workgroup adds their gy
   // partials through LDS and writes one slot (half the partial traffic).
   bool pair = true;
