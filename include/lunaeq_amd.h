@@ -368,6 +368,26 @@ int luna_graph_build(const void* src, const void* dst, int index_bits, int64_t n
                      int32_t* seg_begin, int32_t* seg_end, int32_t* seg_order, void* workspace,
                      size_t workspace_bytes, LunaStream stream);
 
+/*
+ * luna_graph_build in steps that let the caller size the second one, all on one
+ * workspace of luna_graph_workspace bytes and one stream.
+ * luna_graph_scan writes src32, dst32, both edge id lists, the row pointers, seg_rowptr
+ * and status[8] = smallest and largest index, dst not sorted, segments, largest in- and
+ * out-degree, 0, 0; indices outside [0, num_nodes) or out of order are reported, and the
+ * tables are valid only if there are none.
+ * luna_graph_finish, for validated indices, writes the node orders, tiers and the
+ * `segments` source segments; largest_degree bounds both degrees.
+ */
+int luna_graph_scan(const void* src, const void* dst, int index_bits, int64_t num_nodes, int64_t num_edges,
+                    int32_t* src32, int32_t* dst32, int32_t* dst_rowptr, int32_t* src_rowptr,
+                    int32_t* edge_ids_by_src, int32_t* edge_ids_by_dst, int32_t* seg_rowptr, int64_t* status,
+                    void* workspace, size_t workspace_bytes, LunaStream stream);
+int luna_graph_finish(const int32_t* dst_rowptr, const int32_t* src_rowptr, const int32_t* seg_rowptr,
+                      int64_t num_nodes, int64_t num_edges, int64_t largest_degree, int64_t segments,
+                      int32_t* node_order, int32_t* source_node_order, int32_t* node_tiers, int32_t* seg_nodes,
+                      int32_t* seg_begin, int32_t* seg_end, int32_t* seg_order, void* workspace,
+                      size_t workspace_bytes, LunaStream stream);
+
 /* Compile (or load from cache_dir) the graph kernels without touching a device;
  * also sets the cache directory the graph kernels use afterwards. */
 int luna_graph_precompile(const char* cache_dir);

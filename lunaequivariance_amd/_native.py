@@ -72,6 +72,8 @@ PROTOTYPES = {
     "luna_graph_workspace": (ctypes.c_int, [_I64, _I64, ctypes.POINTER(ctypes.c_size_t)]),
     "luna_graph_build": (ctypes.c_int, [_VP, _VP, ctypes.c_int, _I64, _I64] + [_VP] * 15
                          + [ctypes.c_size_t, _VP]),
+    "luna_graph_scan": (ctypes.c_int, [_VP, _VP, ctypes.c_int, _I64, _I64] + [_VP] * 9 + [ctypes.c_size_t, _VP]),
+    "luna_graph_finish": (ctypes.c_int, [_VP] * 3 + [_I64] * 4 + [_VP] * 8 + [ctypes.c_size_t, _VP]),
     "luna_graph_precompile": (ctypes.c_int, [ctypes.c_char_p]),
     "luna_profile_enable": (ctypes.c_int, [ctypes.c_int]),
     "luna_profile_collect": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_size_t,

@@ -3,22 +3,35 @@
 // make_graph / make_source_segments, src/lunatp/graph.py:49-141 and
 // src/lunatp/uvu_conv/graph.py:38-99), as a short pipeline of integer
 // kernels:
-//   * CSR row pointers by binary search: rowptr[n] = first edge with key >= n
-//     in a key-sorted edge list (dst as given; src after the sort below);
-//   * edge ids by source: stable LSD radix sort of (src, edge id), 4-bit
-//     digits, one upsweep (digit counts per 2048-edge tile), one scan and one
-//     stable scatter per digit;
-//   * node orders: the same sort on keys E - degree (descending degree,
-//     ties by node id, as a stable descending argsort);
+//   * one pass over the edges: validation (min, max, dst sorted), int32 copies,
+//     edge ids;
+//   * edge ids by source: stable LSD radix sort of (src, edge id), 8-bit digits
+//     (count per 2048-element tile, scan per digit, stable scatter);
+//   * CSR row pointers by binary search in dst and in the sorted src (counting
+//     the sources with atomics took 45 us more: 1M scattered 4-byte atomics);
+//   * segment counts and largest degrees;
+//   * node orders: the same sort on keys (largest degree - degree), ties by node
+//     id; both orders and the segments' first sort share their launches;
 //   * node tiers: scan of the ordered degrees and a search for E/4, 2E/4, 3E/4;
 //   * source segments: max(1, ceil(degree/32)) chunks per node, ordered by
 //     descending length, then descending node degree, then segment index.
+// The caller may read the validation, the segment count and the largest
+// degrees back after the first half (luna_graph_scan), which sizes the sorts of
+// the second (luna_graph_finish): degrees below 256 take one digit instead of
+// the three that E needs.
+//
+// Bound: launches, each a few microseconds of latency on tables of a few MB.
+// 20,000 nodes and 1.05M edges: 702 us with 4-bit digits (22 sort passes,
+// about 110 launches, 190 us of them 64-bit atomics of the validation pass on
+// three addresses), 178 us with 24 launches, none above 20 us.
 // Every buffer is the caller's; scratch comes from one caller-sized
 // workspace.  Kernels are compiled with hipRTC once (code-object cache).
 #include <algorithm>
 #include <cstdint>
+#include <initializer_list>
 #include <memory>
 #include <string>
+#include <vector>
 
 #include "../../include/lunaeq_amd.h"
 #include "common.h"
@@ -26,8 +39,10 @@
 namespace luna {
 namespace {
 
-constexpr int kTile = 2048;    // elements per workgroup (256 threads x 8)
-constexpr int kDigits = 16;    // radix 16 (4-bit digits)
+constexpr int kTile = 2048;    // scan: elements per workgroup (256 threads x 8)
+constexpr int kSortTile = 2048;  // sort: elements per workgroup (4 waves x 8 x 64)
+constexpr int kDigits = 256;   // 8-bit digits
+constexpr int kFewTiles = 64;   // scan: up to this many tile sums are added up by every workgroup itself
 constexpr int kSegment = 32;   // edges per source segment
 
 const char* kGraphSource = R"(
@@ -43,6 +58,34 @@ extern "C" __global__ void luna_graph_bounds_init(i64* status) {
   }
 }
 
+// min / max and the flag of a workgroup of 256, then one set of atomics each
+// (per wave they were 24,576 on three addresses for a million edges, 190 us).
+__device__ void publish(i64 lo, i64 hi, int unsorted, i64* status) {
+  __shared__ i64 los[4], his[4];
+  __shared__ int flags[4];
+  for (int m = 32; m >= 1; m >>= 1) {
+    lo = min(lo, (i64)__shfl_xor(lo, m, 64));
+    hi = max(hi, (i64)__shfl_xor(hi, m, 64));
+    unsorted |= __shfl_xor(unsorted, m, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    los[threadIdx.x >> 6] = lo;
+    his[threadIdx.x >> 6] = hi;
+    flags[threadIdx.x >> 6] = unsorted;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    // Most workgroups find the bounds already there.
+    lo = min(min(los[0], los[1]), min(los[2], los[3]));
+    hi = max(max(his[0], his[1]), max(his[2], his[3]));
+    if (lo < __hip_atomic_load(&status[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin((long long*)&status[0], (long long)lo);
+    if (hi > __hip_atomic_load(&status[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax((long long*)&status[1], (long long)hi);
+    if (flags[0] | flags[1] | flags[2] | flags[3]) atomicOr((unsigned long long*)&status[2], 1ULL);
+  }
+}
+
 // min / max over src and dst, and whether dst descends anywhere.
 template <typename T>
 __device__ void bounds(const T* src, const T* dst, i64 E, i64* status) {
@@ -54,16 +97,7 @@ __device__ void bounds(const T* src, const T* dst, i64 E, i64* status) {
     hi = max(hi, max(s, d));
     if (i + 1 < E && (i64)dst[i + 1] < d) unsorted = 1;
   }
-  for (int m = 32; m >= 1; m >>= 1) {
-    lo = min(lo, (i64)__shfl_xor(lo, m, 64));
-    hi = max(hi, (i64)__shfl_xor(hi, m, 64));
-    unsorted |= __shfl_xor(unsorted, m, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMin((long long*)&status[0], (long long)lo);
-    atomicMax((long long*)&status[1], (long long)hi);
-    if (unsorted) atomicOr((unsigned long long*)&status[2], 1ULL);
-  }
+  publish(lo, hi, unsorted, status);
 }
 extern "C" __global__ void __launch_bounds__(256) luna_graph_bounds32(const int* src, const int* dst, i64 E,
                                                                       i64* status) {
@@ -74,35 +108,51 @@ extern "C" __global__ void __launch_bounds__(256) luna_graph_bounds64(const i64*
   bounds(src, dst, E, status);
 }
 
-// int32 copies of the indices (values already checked to fit).
-extern "C" __global__ void __launch_bounds__(256) luna_graph_narrow(const void* in, int is64, int* out, i64 n) {
-  const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  out[i] = is64 ? (int)((const i64*)in)[i] : ((const int*)in)[i];
+// status: min, max, unsorted, segments, largest in- and out-degree, 0, 0.
+extern "C" __global__ void luna_graph_scan_init(i64* status) {
+  const int i = threadIdx.x;
+  if (i < 8) status[i] = i == 0 ? 0x7fffffffffffffffLL : i == 1 ? -0x7fffffffffffffffLL - 1 : 0;
 }
 
-extern "C" __global__ void __launch_bounds__(256) luna_graph_iota(int* out, i64 n) {
-  const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] = (int)i;
+// One pass over the edges: bounds, int32 copies, edge ids.
+template <typename T>
+__device__ void edges(const T* src, const T* dst, i64 E, int* src32, int* dst32, int* ids, i64* status) {
+  i64 lo = 0x7fffffffffffffffLL, hi = -0x7fffffffffffffffLL - 1;
+  int unsorted = 0;
+  #pragma unroll 4
+  for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < E; i += (i64)gridDim.x * 256) {
+    const i64 s = (i64)src[i], d = (i64)dst[i];
+    lo = min(lo, min(s, d));
+    hi = max(hi, max(s, d));
+    if (i + 1 < E && (i64)dst[i + 1] < d) unsorted = 1;
+    src32[i] = (int)s;
+    dst32[i] = (int)d;
+    ids[i] = (int)i;
+  }
+  publish(lo, hi, unsorted, status);
+}
+extern "C" __global__ void __launch_bounds__(256) luna_graph_edges(const void* src, const void* dst, int is64, i64 E,
+                                                                   int* src32, int* dst32, int* ids, i64* status) {
+  if (is64)
+    edges((const i64*)src, (const i64*)dst, E, src32, dst32, ids, status);
+  else
+    edges((const int*)src, (const int*)dst, E, src32, dst32, ids, status);
 }
 
-// rowptr[n] = first index i with keys[i] >= n, for n = 0..N (keys ascending).
-extern "C" __global__ void __launch_bounds__(256) luna_graph_rowptr(const int* keys, i64 E, int N, int* rowptr) {
+// rowptr[n] = first index i with keys[i] >= n, for n = 0..N (keys ascending), of
+// two lists at once.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_rowptr(const int* keys0, const int* keys1, i64 E, int N,
+                                                                    int* rowptr0, int* rowptr1) {
   const i64 n = (i64)blockIdx.x * 256 + threadIdx.x;
   if (n > N) return;
+  const int* const keys = blockIdx.y ? keys1 : keys0;
+  int* const rowptr = blockIdx.y ? rowptr1 : rowptr0;
   i64 lo = 0, hi = E;
   while (lo < hi) {
     const i64 mid = (lo + hi) >> 1;
     if (keys[mid] < n) lo = mid + 1; else hi = mid;
   }
   rowptr[n] = (int)lo;
-}
-
-// keys[n] = E - degree[n] with degree from a row-pointer array.
-extern "C" __global__ void __launch_bounds__(256) luna_graph_degree_keys(const int* rowptr, int N, int E,
-                                                                        u32* keys) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
-  if (n < N) keys[n] = (u32)(E - (rowptr[n + 1] - rowptr[n]));
 }
 
 // ---- exclusive scan of int32 (tiles of 2048, block sums scanned recursively)
@@ -145,74 +195,159 @@ extern "C" __global__ void __launch_bounds__(256) luna_graph_scan_tiles(const in
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-extern "C" __global__ void __launch_bounds__(256) luna_graph_scan_add(int* out, i64 n_out, const int* offsets) {
+// Adds each tile's offset, or the sum of the sums before it (at most 64 of
+// them); the last value also goes to *last, if given.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_scan_add(int* out, i64 n_out, const int* offsets,
+                                                                      const int* sums, i64* last) {
   const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (i < n_out) out[i] += offsets[i / 2048];
+  const i64 tile = (i64)blockIdx.x * 256 / 2048;
+  int before;
+  if (offsets) {
+    before = offsets[tile];
+  } else {
+    const int lane = threadIdx.x & 63;
+    before = lane < tile ? sums[lane] : 0;
+    for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
+  }
+  if (i >= n_out) return;
+  const int v = out[i] + before;
+  out[i] = v;
+  if (last && i == n_out - 1) *last = v;
 }
 
-// ---- stable LSD radix sort, 4-bit digits
-// hist[d * tiles + tile] = count of digit d in the tile.
-extern "C" __global__ void __launch_bounds__(256) luna_graph_radix_count(const u32* keys, i64 n, int shift,
-                                                                         int* hist, int tiles) {
-  __shared__ int table[16][256];
+// ---- stable LSD radix sort, 8-bit digits, up to three sorts per launch
+struct Job {
+  const u32* keys;
+  const int* vals;  // null: the element index
+  u32* keys_out;    // null: not wanted
+  int* vals_out;
+  int* hist;        // [tiles + 1][256]: counts, then offsets within a digit; last row: totals
+  i64 n;
+  int tiles;
+};
+struct Jobs {
+  Job job[3];
+};
+
+extern "C" __global__ void __launch_bounds__(256) luna_graph_radix_count(Jobs jobs, int shift) {
+  const Job& j = jobs.job[blockIdx.y];
+  __shared__ int count[256];
   const int t = threadIdx.x;
-  for (int d = 0; d < 16; ++d) table[d][t] = 0;
-  const i64 base = (i64)blockIdx.x * 2048 + t * 8;
-  for (int j = 0; j < 8; ++j)
-    if (base + j < n) ++table[(keys[base + j] >> shift) & 15][t];
+  if (blockIdx.x >= j.tiles) return;
+  count[t] = 0;
   __syncthreads();
-  if (t < 16) {
-    int s = 0;
-    for (int k = 0; k < 256; ++k) s += table[t][k];
-    hist[(i64)t * tiles + blockIdx.x] = s;
-  }
+  const i64 base = (i64)blockIdx.x * 2048 + t;
+  #pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (base + k * 256 < j.n) atomicAdd(&count[(j.keys[base + k * 256] >> shift) & 255], 1);
+  __syncthreads();
+  j.hist[(i64)blockIdx.x * 256 + t] = count[t];
 }
 
-// Scatter of one tile: position = offsets[d][tile] + count of digit d in the
-// earlier elements of the tile (threads own 8 consecutive elements, in order).
-extern "C" __global__ void __launch_bounds__(256) luna_graph_radix_scatter(
-    const u32* keys, const int* vals, u32* keys_out, int* vals_out, i64 n, int shift, const int* offsets,
-    int tiles) {
-  __shared__ int table[16][256];
-  __shared__ int wsum[16][4];
-  __shared__ int start[16];
+// Exclusive scan of one digit's counts over the tiles.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_radix_columns(Jobs jobs) {
+  const Job& j = jobs.job[blockIdx.y];
+  __shared__ int wsum[4];
+  int run = 0;
+  for (int base = 0; base < j.tiles; base += 256) {
+    const int tile = base + threadIdx.x;
+    int* const at = j.hist + (i64)tile * 256 + blockIdx.x;
+    const int v = tile < j.tiles ? *at : 0;
+    int total;
+    const int before = block_exclusive_scan(v, wsum, &total);
+    if (tile < j.tiles) *at = run + before;
+    run += total;
+  }
+  if (threadIdx.x == 0) j.hist[(i64)j.tiles * 256 + blockIdx.x] = run;
+}
+
+// Scatter of one tile, in order: a wave owns 512 consecutive elements, 64 at a
+// time; equal digits of the 64 find each other by eight ballots.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_radix_scatter(Jobs jobs, int shift) {
+  const Job& j = jobs.job[blockIdx.y];
+  __shared__ int at[4][256];
+  __shared__ int wsum[4];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int d = 0; d < 16; ++d) table[d][t] = 0;
-  const i64 base = (i64)blockIdx.x * 2048 + t * 8;
-  u32 k[8];
-  for (int j = 0; j < 8; ++j) {
-    k[j] = base + j < n ? keys[base + j] : 0u;
-    if (base + j < n) ++table[(k[j] >> shift) & 15][t];
+  if (blockIdx.x >= j.tiles) return;
+  for (int w = 0; w < 4; ++w) at[w][t] = 0;
+  __syncthreads();
+  const i64 base = (i64)blockIdx.x * 2048 + wave * 512 + lane;
+  u32 key[8];
+  #pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    key[k] = base + k * 64 < j.n ? j.keys[base + k * 64] : 0u;
+    if (base + k * 64 < j.n) atomicAdd(&at[wave][(key[k] >> shift) & 255], 1);
   }
-  if (t < 16) start[t] = offsets[(i64)t * tiles + blockIdx.x];
-  // Exclusive prefix over threads, for every digit.
-  int inc[16];
-  for (int d = 0; d < 16; ++d) {
-    inc[d] = table[d][t];
-    for (int m = 1; m < 64; m <<= 1) {
-      const int o = __shfl_up(inc[d], m, 64);
-      if (lane >= m) inc[d] += o;
-    }
-    if (lane == 63) wsum[d][wave] = inc[d];
+  int unused;
+  const int first = block_exclusive_scan(j.hist[(i64)j.tiles * 256 + t], wsum, &unused);
+  __syncthreads();
+  int run = first + j.hist[(i64)blockIdx.x * 256 + t];
+  for (int w = 0; w < 4; ++w) {
+    const int c = at[w][t];
+    at[w][t] = run;
+    run += c;
   }
   __syncthreads();
-  for (int d = 0; d < 16; ++d) {
-    int before = 0;
-    for (int w = 0; w < 4; ++w) before += w < wave ? wsum[d][w] : 0;
-    table[d][t] = start[d] + before + inc[d] - table[d][t];
-  }
-  for (int j = 0; j < 8; ++j) {
-    if (base + j >= n) break;
-    const int pos = table[(k[j] >> shift) & 15][t]++;
-    keys_out[pos] = k[j];
-    vals_out[pos] = vals ? vals[base + j] : (int)(base + j);
+  volatile int* const mine = at[wave];
+  #pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const i64 i = base + k * 64;
+    const bool real = i < j.n;
+    const int d = (key[k] >> shift) & 255;
+    unsigned long long same = __ballot(real);
+    #pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const unsigned long long set = __ballot((d >> b) & 1);
+      same &= (d >> b) & 1 ? set : ~set;
+    }
+    const int rank = __popcll(same & ((1ULL << lane) - 1));
+    const int pos = mine[d] + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (real && (same >> lane) == 1ULL) mine[d] = pos + 1;
+    __builtin_amdgcn_wave_barrier();
+    if (real) {
+      if (j.keys_out) j.keys_out[pos] = key[k];
+      j.vals_out[pos] = j.vals ? j.vals[i] : (int)i;
+    }
   }
 }
 
-// Keys of the first pass from int32 indices.
-extern "C" __global__ void __launch_bounds__(256) luna_graph_keys_from(const int* in, u32* keys, i64 n) {
+// Keys of the two node orders, and the nodes' segments with their degree keys.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_node_keys(const int* dst_rowptr, const int* src_rowptr,
+                                                                       const int* seg_rowptr, int N, int most,
+                                                                       u32* in_key, u32* out_key, int* nodes,
+                                                                       int* begin, int* end, u32* seg_key) {
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n >= N) return;
+  const int r0 = src_rowptr[n], r1 = src_rowptr[n + 1];
+  in_key[n] = (u32)(most - (dst_rowptr[n + 1] - dst_rowptr[n]));
+  out_key[n] = (u32)(most - (r1 - r0));
+  for (int s = seg_rowptr[n], k = 0; s < seg_rowptr[n + 1]; ++s, ++k) {
+    nodes[s] = n;
+    begin[s] = r0 + 32 * k;
+    end[s] = min(r0 + 32 * k + 32, r1);
+    seg_key[s] = (u32)(most - (r1 - r0));
+  }
+}
+
+// Past the real segments (seg_rowptr[N] of them): empty ranges whose keys sort
+// after all others.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_segment_padding(const int* seg_rowptr, int N, i64 S,
+                                                                            int most, int* begin, int* end,
+                                                                            u32* seg_key) {
+  const i64 s = (i64)blockIdx.x * 256 + threadIdx.x;
+  if (s < S && s >= seg_rowptr[N]) {
+    begin[s] = 1;
+    end[s] = 0;
+    seg_key[s] = (u32)most + 1u;
+  }
+}
+
+// Length keys in the order of the degree sort (padding: 33, after every real one).
+extern "C" __global__ void __launch_bounds__(256) luna_graph_length_keys(const int* order, const int* begin,
+                                                                         const int* end, i64 S, u32* keys) {
   const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) keys[i] = (u32)in[i];
+  if (i < S) keys[i] = (u32)(32 - (end[order[i]] - begin[order[i]]));
 }
 
 // node_tiers[t-1] = (first i with cum[i] >= t*E/4) + 1, cum = inclusive scan of
@@ -240,45 +375,26 @@ extern "C" __global__ void __launch_bounds__(256) luna_graph_gather_degree(const
   }
 }
 
-// Segments per node: max(1, ceil(degree / 32)).
-extern "C" __global__ void __launch_bounds__(256) luna_graph_segment_counts(const int* rowptr, int N, int* count) {
+// Segments per node, max(1, ceil(out-degree / 32)), and the largest degrees.
+extern "C" __global__ void __launch_bounds__(256) luna_graph_segment_counts(const int* dst_rowptr, const int* src_rowptr,
+                                                                            int N, int* count, i64* status) {
   const int n = blockIdx.x * 256 + threadIdx.x;
+  int in = 0, out = 0;
   if (n < N) {
-    const int d = rowptr[n + 1] - rowptr[n];
-    count[n] = d > 0 ? (d + 31) / 32 : 1;
+    in = dst_rowptr[n + 1] - dst_rowptr[n];
+    out = src_rowptr[n + 1] - src_rowptr[n];
+    count[n] = out > 0 ? (out + 31) / 32 : 1;
   }
-}
-
-extern "C" __global__ void __launch_bounds__(256) luna_graph_segments(const int* rowptr, const int* seg_rowptr,
-                                                                     int N, int E, int* nodes, int* begin, int* end,
-                                                                     u32* deg_key, u32* len_key) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
-  if (n >= N) return;
-  const int r0 = rowptr[n], r1 = rowptr[n + 1];
-  for (int s = seg_rowptr[n], k = 0; s < seg_rowptr[n + 1]; ++s, ++k) {
-    const int b = r0 + 32 * k, e = min(b + 32, r1);
-    nodes[s] = n;
-    begin[s] = b;
-    end[s] = e;
-    deg_key[s] = (u32)(E - (r1 - r0));
-    len_key[s] = (u32)(32 - (e - b));
+  for (int m = 32; m >= 1; m >>= 1) {
+    in = max(in, __shfl_xor(in, m, 64));
+    out = max(out, __shfl_xor(out, m, 64));
   }
-}
-
-// Past the real segments (seg_rowptr[N] of them): keys that sort after all.
-extern "C" __global__ void __launch_bounds__(256) luna_graph_segment_padding(const int* seg_rowptr, int N, i64 S,
-                                                                            int E, u32* deg_key, u32* len_key) {
-  const i64 s = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (s < S && s >= seg_rowptr[N]) {
-    deg_key[s] = (u32)E + 1u;
-    len_key[s] = 63u;
+  if ((threadIdx.x & 63) == 0) {
+    if (in > __hip_atomic_load(&status[4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax((long long*)&status[4], (long long)in);
+    if (out > __hip_atomic_load(&status[5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax((long long*)&status[5], (long long)out);
   }
-}
-
-extern "C" __global__ void __launch_bounds__(256) luna_graph_gather_keys(const int* order, const u32* keys, i64 n,
-                                                                        u32* out) {
-  const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] = keys[order[i]];
 }
 )";
 
@@ -299,6 +415,7 @@ hipModule_t graph_module(const char* cache_dir) {
 }
 
 unsigned blocks_of(int64_t n, int64_t per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
+int64_t sort_tiles(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
 int64_t tiles_of(int64_t n) { return (n + kTile - 1) / kTile; }
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -318,6 +435,20 @@ struct Arena {
   }
 };
 
+// The kernels' Job and Jobs.
+struct GraphJob {
+  const uint32_t* keys;
+  const int* vals;
+  uint32_t* keys_out;
+  int* vals_out;
+  int* hist;
+  int64_t n;
+  int tiles;
+};
+struct GraphJobs {
+  GraphJob job[3];
+};
+
 struct Builder {
   hipModule_t module;
   hipStream_t stream;
@@ -328,75 +459,79 @@ struct Builder {
            stream, args);
   }
 
-  // out[0..n_out) = exclusive scan of in[0..n_in) (zero past n_in).
-  void scan(const int* in, int64_t n_in, int* out, int64_t n_out) {
+  // out[0..n_out) = exclusive scan of in[0..n_in) (zero past n_in); out[n_out - 1] also in *last.
+  void scan(const int* in, int64_t n_in, int* out, int64_t n_out, int64_t* last = nullptr) {
     if (n_out <= 0) return;
     const size_t mark = arena.used;
     const int64_t tiles = tiles_of(n_out);
     int* sums = arena.take<int>(tiles);
-    int* offsets = tiles > 1 ? arena.take<int>(tiles) : nullptr;
+    int* offsets = tiles > kFewTiles ? arena.take<int>(tiles) : nullptr;
     if (module) {
       void* a[] = {&in, &n_in, &out, &n_out, &sums};
       run("scan_tiles", blocks_of(n_out, kTile), a);
     }
-    if (tiles > 1) {
-      int64_t t = tiles;
-      scan(sums, t, offsets, t);
-      if (module) {
-        void* b[] = {&out, &n_out, &offsets};
-        run("scan_add", blocks_of(n_out, 256), b);
-      }
+    if (offsets) scan(sums, tiles, offsets, tiles);
+    if (module && (tiles > 1 || last)) {
+      void* b[] = {&out, &n_out, &offsets, &sums, &last};
+      run("scan_add", blocks_of(n_out, 256), b);
     }
     arena.used = mark;
   }
 
-  // Stable sort of (keys, vals) by the low `bits` of keys; vals == null means
-  // the element index.  The sorted values land in vals_out (keys_out, if
-  // given, receives the sorted keys).  keys is consumed.
-  void sort(uint32_t* keys, const int* vals, int64_t n, int bits, int* vals_out, uint32_t* keys_out) {
-    if (n <= 0) return;
+  struct Sort {
+    uint32_t* keys;      // consumed
+    const int* vals;     // null: the element index
+    int64_t n;
+    int* vals_out;
+    uint32_t* keys_out = nullptr;  // the sorted keys, if wanted
+  };
+
+  // Stable sorts (up to three in each launch) by the low `bits` of the keys, in
+  // 8-bit digits; at least one digit, so that vals_out is always written.
+  void sort(std::initializer_list<Sort> sorts, int bits) {
     const size_t mark = arena.used;
-    const int64_t tiles = tiles_of(n);
-    uint32_t* k_tmp = arena.take<uint32_t>(n);
-    uint32_t* k_tmp2 = arena.take<uint32_t>(n);
-    int* v_tmp = arena.take<int>(n);
-    int* hist = arena.take<int>(kDigits * tiles);
-    int* offsets = arena.take<int>(kDigits * tiles);
-    if (!module) {
-      scan(hist, kDigits * tiles, offsets, kDigits * tiles);
-      arena.used = mark;
-      return;
+    const int passes = std::max(1, (bits + 7) / 8);
+    struct Buffers {
+      uint32_t* keys[2];
+      int *vals, *hist;
+    };
+    std::vector<Buffers> bufs;
+    unsigned most = 0;
+    for (const Sort& q : sorts) {
+      const int64_t tiles = sort_tiles(q.n);
+      Buffers f;
+      f.keys[0] = arena.take<uint32_t>(passes > 1 ? q.n : 0);
+      f.keys[1] = arena.take<uint32_t>(passes > 2 ? q.n : 0);
+      f.vals = arena.take<int>(passes > 1 ? q.n : 0);
+      f.hist = arena.take<int>((tiles + 1) * kDigits);
+      bufs.push_back(f);
+      most = std::max(most, (unsigned)tiles);
     }
-    const int passes = (bits + 3) / 4;
-    uint32_t* k_in = keys;
-    const int* v_in = vals;
-    // Pass p writes buffer (passes - 1 - p) % 2, so the last pass writes
-    // vals_out (and its keys to k_tmp); the input is read by pass 0 only.
-    uint32_t* k_buf[2] = {k_tmp, k_tmp2};
-    int* v_buf[2] = {vals_out, v_tmp};
-    int t = (int)tiles;
-    for (int p = 0; p < passes; ++p) {
-      const int which = (passes - 1 - p) % 2;
-      uint32_t* k_out = k_buf[which];
-      int* v_out = v_buf[which];
-      int shift = 4 * p;
-      void* a[] = {&k_in, &n, &shift, &hist, &t};
-      run("radix_count", blocks_of(n, kTile), a);
-      scan(hist, kDigits * tiles, offsets, kDigits * tiles);
-      void* b[] = {&k_in, &v_in, &k_out, &v_out, &n, &shift, &offsets, &t};
-      run("radix_scatter", blocks_of(n, kTile), b);
-      k_in = k_out;
-      v_in = v_out;
-    }
-    if (passes == 0) {
-      if (vals) fail("luna_graph_build: internal (zero-pass sort with values)");
-      void* a[] = {&vals_out, &n};
-      run("iota", blocks_of(n, 256), a);
-    }
-    if (keys_out && passes > 0) {
-      // The last pass wrote its keys to k_buf[0] == k_tmp.
-      check_hip(hipMemcpyAsync(keys_out, k_tmp, (size_t)n * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream),
-                "hipMemcpyAsync");
+    if (module && most) {
+      for (int p = 0; p < passes; ++p) {
+        GraphJobs jobs{};
+        int n = 0;
+        for (const Sort& q : sorts) {
+          const Buffers& f = bufs[n];
+          GraphJob& j = jobs.job[n++];
+          // The last pass writes vals_out, those before it alternate; the input
+          // buffer of keys is free once pass 0 has read it.
+          const int left = passes - 1 - p;
+          j.keys = p == 0 ? q.keys : f.keys[(p - 1) % 2];
+          j.keys_out = left ? f.keys[p % 2] : q.keys_out;
+          j.vals_out = left % 2 ? f.vals : q.vals_out;
+          j.vals = p == 0 ? q.vals : ((left + 1) % 2 ? f.vals : q.vals_out);
+          j.hist = f.hist;
+          j.n = q.n;
+          j.tiles = (int)sort_tiles(q.n);
+        }
+        int shift = 8 * p;
+        void* a[] = {&jobs, &shift};
+        run("radix_count", dim3(most, (unsigned)n), a);
+        void* c[] = {&jobs};
+        run("radix_columns", dim3(kDigits, (unsigned)n), c);
+        run("radix_scatter", dim3(most, (unsigned)n), a);
+      }
     }
     arena.used = mark;
   }
@@ -413,87 +548,102 @@ struct Outputs {
       *source_node_order, *node_tiers, *seg_rowptr, *seg_nodes, *seg_begin, *seg_end, *seg_order;
 };
 
-// One pass with module == null sizes the workspace; a second one launches.
-void build(hipModule_t module, hipStream_t stream, Arena& arena, const void* src, const void* dst, int is64,
-           int64_t N, int64_t E, Outputs o) {
+// A call with module == null sizes the workspace; with one it launches.
+
+// Tables known before any sort, and status = min, max, unsorted, segments,
+// largest in- and out-degree, 0, 0.
+// Any indices sort and search without fault, so the caller may read the
+// validation after all of it.
+void scan_half(hipModule_t module, hipStream_t stream, Arena& arena, const void* src, const void* dst, int is64,
+               int64_t N, int64_t E, Outputs o, int64_t* status) {
   Builder b{module, stream, arena};
-  const int64_t seg_cap = N + E / kSegment + 1;
-  uint32_t* keys = arena.take<uint32_t>(std::max(std::max(E, N), seg_cap));
-  int* sorted_src = arena.take<int>(E);
-  int* work = arena.take<int>(std::max(N + 1, seg_cap));
-  uint32_t* keys2 = arena.take<uint32_t>(seg_cap);
-  int* perm = arena.take<int>(seg_cap);
-  int Ni = (int)N, Ei = (int)E;
+  uint32_t* sorted = arena.take<uint32_t>(E);
+  int* count = arena.take<int>(N);
+  int Ni = (int)N;
   if (module) {
-    void* a[] = {(void*)&src, &is64, &o.src32, &E};
-    b.run("narrow", blocks_of(E, 256), a);
-    void* c[] = {(void*)&dst, &is64, &o.dst32, &E};
-    b.run("narrow", blocks_of(E, 256), c);
-    void* d[] = {&o.edge_ids_by_dst, &E};
-    b.run("iota", blocks_of(E, 256), d);
-    void* r[] = {&o.dst32, &E, &Ni, &o.dst_rowptr};
-    b.run("rowptr", blocks_of(N + 1, 256), r);
-    void* k[] = {&o.src32, &keys, &E};
-    b.run("keys_from", blocks_of(E, 256), k);
+    void* a[] = {&status};
+    b.run("scan_init", dim3(1), a);
+    if (E > 0) {
+      void* c[] = {(void*)&src, (void*)&dst, &is64, &E, &o.src32, &o.dst32, &o.edge_ids_by_dst, &status};
+      b.run("edges", (unsigned)std::min<int64_t>(1024, (E + 255) / 256), c);
+    }
   }
-  // Edge ids by source (stable), then the source CSR from the sorted keys.
-  b.sort(keys, nullptr, E, bits_for(N > 0 ? N - 1 : 0), o.edge_ids_by_src, (uint32_t*)sorted_src);
+  if (E > 0)
+    b.sort({{(uint32_t*)o.src32, nullptr, E, o.edge_ids_by_src, sorted}}, bits_for(N > 0 ? N - 1 : 0));
   if (module) {
-    if (bits_for(N > 0 ? N - 1 : 0) == 0 && E > 0) {
-      // Every source is node 0: the keys are already "sorted".
-      void* k[] = {&o.src32, &keys, &E};
-      b.run("keys_from", blocks_of(E, 256), k);
-      check_hip(hipMemcpyAsync(sorted_src, keys, (size_t)E * 4, hipMemcpyDeviceToDevice, stream), "hipMemcpyAsync");
-    }
-    void* r[] = {&sorted_src, &E, &Ni, &o.src_rowptr};
-    b.run("rowptr", blocks_of(N + 1, 256), r);
+    void* r[] = {&o.dst32, &sorted, &E, &Ni, &o.dst_rowptr, &o.src_rowptr};
+    b.run("rowptr", dim3(blocks_of(N + 1, 256), 2), r);
   }
-  // Node orders: descending degree, ties by node id.
-  const int deg_bits = bits_for(E);
-  for (int which = 0; which < 2; ++which) {
-    const int32_t* rowptr = which == 0 ? o.dst_rowptr : o.src_rowptr;
-    int32_t* order = which == 0 ? o.node_order : o.source_node_order;
-    if (module && N > 0) {
-      void* a[] = {&rowptr, &Ni, &Ei, &keys};
-      b.run("degree_keys", blocks_of(N, 256), a);
-    }
-    b.sort(keys, nullptr, N, deg_bits, order, nullptr);
-  }
-  // Node tiers from the degrees in node order.
   if (module && N > 0) {
-    void* a[] = {&o.node_order, &o.dst_rowptr, &Ni, &perm};
+    void* a[] = {&o.dst_rowptr, &o.src_rowptr, &Ni, &count, &status};
+    b.run("segment_counts", blocks_of(N, 256), a);
+  }
+  b.scan(count, N, o.seg_rowptr, N + 1, status ? status + 3 : nullptr);
+}
+
+// Node orders, tiers and segments.  `most`: a bound of every degree; segments:
+// their number, or -1 to sort the upper bound N + E/32 + 1 with padding keys
+// past the real ones (then the tables must have room for it).
+void node_half(hipModule_t module, hipStream_t stream, Arena& arena, int64_t N, int64_t E, int64_t most64,
+               int64_t segments, Outputs o) {
+  Builder b{module, stream, arena};
+  const int64_t S = N == 0 ? 0 : segments >= 0 ? segments : N + E / kSegment + 1;
+  uint32_t* in_key = arena.take<uint32_t>(N);
+  uint32_t* out_key = arena.take<uint32_t>(N);
+  uint32_t* seg_key = arena.take<uint32_t>(S);
+  int* perm = arena.take<int>(S);
+  int* work = arena.take<int>(N + 1);
+  int* degrees = arena.take<int>(N);
+  int Ni = (int)N, most = (int)most64;
+  if (module && N > 0) {
+    void* a[] = {&o.dst_rowptr, &o.src_rowptr, &o.seg_rowptr, &Ni, &most, &in_key, &out_key,
+                 &o.seg_nodes, &o.seg_begin, &o.seg_end, &seg_key};
+    b.run("node_keys", blocks_of(N, 256), a);
+    if (segments < 0) {
+      void* p[] = {&o.seg_rowptr, &Ni, (void*)&S, &most, &o.seg_begin, &o.seg_end, &seg_key};
+      b.run("segment_padding", blocks_of(S, 256), p);
+    }
+  }
+  if (N > 0) {
+    b.sort({{in_key, nullptr, N, o.node_order}, {out_key, nullptr, N, o.source_node_order}, {seg_key, nullptr, S, perm}},
+           bits_for(most64 + (segments < 0)));
+    if (module) {
+      void* a[] = {&perm, &o.seg_begin, &o.seg_end, (void*)&S, &seg_key};
+      b.run("length_keys", blocks_of(S, 256), a);
+    }
+    b.sort({{seg_key, perm, S, o.seg_order}}, 6);
+  }
+  if (module && N > 0) {
+    void* a[] = {&o.node_order, &o.dst_rowptr, &Ni, &degrees};
     b.run("gather_degree", blocks_of(N, 256), a);
   }
-  b.scan(perm, N, work, N + 1);
+  b.scan(degrees, N, work, N + 1);
   if (module) {
     void* a[] = {&work, &Ni, &E, &o.node_tiers};
     b.run("tiers", blocks_of(std::max<int64_t>(N, 3), 256), a);
   }
-  // Source segments.
-  if (module && N > 0) {
-    void* a[] = {&o.src_rowptr, &Ni, &perm};
-    b.run("segment_counts", blocks_of(N, 256), a);
-  }
-  b.scan(perm, N, o.seg_rowptr, N + 1);
-  if (module && N > 0) {
-    void* a[] = {&o.src_rowptr, &o.seg_rowptr, &Ni, &Ei, &o.seg_nodes, &o.seg_begin, &o.seg_end, &keys, &keys2};
-    b.run("segments", blocks_of(N, 256), a);
-  }
-  // The segment count is only known on the device: sort the upper bound
-  // seg_cap, with padding keys past the real segments that sort last.  The
-  // real ones are a prefix of the result, because padding keys exceed every
-  // real key (degree key E - d <= E < E + 1, length key 32 - len <= 31 < 32).
-  int64_t S = N > 0 ? seg_cap : 0;
-  if (module && S > 0) {
-    void* a[] = {&o.seg_rowptr, &Ni, &S, &Ei, &keys, &keys2};
-    b.run("segment_padding", blocks_of(S, 256), a);
-  }
-  b.sort(keys, nullptr, S, bits_for(E + 1), perm, nullptr);
-  if (module && S > 0) {
-    void* a[] = {&perm, &keys2, &S, &keys};
-    b.run("gather_keys", blocks_of(S, 256), a);
-  }
-  b.sort(keys, perm, S, 6, o.seg_order, nullptr);
+}
+
+// The halves use the workspace one after the other (and nothing of an earlier
+// one), behind the status words.
+void build(hipModule_t module, hipStream_t stream, Arena& arena, const void* src, const void* dst, int is64,
+           int64_t N, int64_t E, Outputs o) {
+  int64_t* status = arena.take<int64_t>(8);
+  const size_t mark = arena.used;
+  scan_half(module, stream, arena, src, dst, is64, N, E, o, status);
+  arena.used = mark;
+  node_half(module, stream, arena, N, E, E, -1, o);
+}
+
+size_t workspace_bytes_of(int64_t N, int64_t E) {
+  Arena arena{nullptr, 0};
+  build(nullptr, nullptr, arena, nullptr, nullptr, 0, N, E, Outputs{});
+  return arena.peak;
+}
+
+void check_graph(int64_t N, int64_t E, const char* what) {
+  if (N < 0 || E < 0) fail(std::string(what) + ": negative size");
+  if (N >= (1LL << 31) || E >= (1LL << 31) - 1) fail("graph exceeds int32 indexing");
 }
 
 }  // namespace
@@ -515,7 +665,7 @@ int luna_graph_bounds(const void* src, const void* dst, int index_bits, int64_t 
     launch("graph_bounds_init", function_for(module, "luna_graph_bounds_init"), dim3(1), dim3(64), s, a);
     if (num_edges > 0) {
       void* b[] = {(void*)&src, (void*)&dst, &num_edges, &status};
-      const unsigned grid = (unsigned)std::min<int64_t>(2048, (num_edges + 255) / 256);
+      const unsigned grid = (unsigned)std::min<int64_t>(512, (num_edges + 255) / 256);
       launch("graph_bounds", function_for(module, index_bits == 64 ? "luna_graph_bounds64" : "luna_graph_bounds32"),
              dim3(grid), dim3(256), s, b);
     }
@@ -525,12 +675,8 @@ int luna_graph_bounds(const void* src, const void* dst, int index_bits, int64_t 
 int luna_graph_workspace(int64_t num_nodes, int64_t num_edges, size_t* bytes) {
   return guard_call([&] {
     if (!bytes) fail("luna_graph_workspace: null argument");
-    if (num_nodes < 0 || num_edges < 0) fail("luna_graph_workspace: negative size");
-    if (num_nodes >= (1LL << 31) || num_edges >= (1LL << 31) - 1) fail("graph exceeds int32 indexing");
-    Arena arena{nullptr, 0};
-    Outputs o{};
-    build(nullptr, nullptr, arena, nullptr, nullptr, 0, num_nodes, num_edges, o);
-    *bytes = arena.peak;
+    check_graph(num_nodes, num_edges, "luna_graph_workspace");
+    *bytes = workspace_bytes_of(num_nodes, num_edges);
   });
 }
 
@@ -542,25 +688,63 @@ int luna_graph_build(const void* src, const void* dst, int index_bits, int64_t n
                      size_t workspace_bytes, LunaStream stream) {
   return guard_call([&] {
     if (index_bits != 32 && index_bits != 64) fail("luna_graph_build: index_bits must be 32 or 64");
-    if (num_nodes < 0 || num_edges < 0) fail("luna_graph_build: negative size");
-    if (num_nodes >= (1LL << 31) || num_edges >= (1LL << 31) - 1) fail("graph exceeds int32 indexing");
+    check_graph(num_nodes, num_edges, "luna_graph_build");
     if (!dst_rowptr || !src_rowptr || !node_tiers || !seg_rowptr) fail("luna_graph_build: null table");
     if (num_edges > 0 && (!src || !dst || !src32 || !dst32 || !edge_ids_by_src || !edge_ids_by_dst))
       fail("luna_graph_build: null edge table");
     if (num_nodes > 0 && (!node_order || !source_node_order || !seg_nodes || !seg_begin || !seg_end || !seg_order))
       fail("luna_graph_build: null node table");
-    size_t need = 0;
-    {
-      Arena sizing{nullptr, 0};
-      Outputs none{};
-      build(nullptr, nullptr, sizing, nullptr, nullptr, 0, num_nodes, num_edges, none);
-      need = sizing.peak;
-    }
-    if (!workspace || workspace_bytes < need) fail("luna_graph_build: workspace too small");
+    if (!workspace || workspace_bytes < workspace_bytes_of(num_nodes, num_edges))
+      fail("luna_graph_build: workspace too small");
     Arena arena{(char*)workspace, workspace_bytes};
     Outputs o{src32, dst32, dst_rowptr, src_rowptr, edge_ids_by_src, edge_ids_by_dst, node_order,
               source_node_order, node_tiers, seg_rowptr, seg_nodes, seg_begin, seg_end, seg_order};
     build(graph_module(nullptr), (hipStream_t)stream, arena, src, dst, index_bits == 64, num_nodes, num_edges, o);
+  });
+}
+
+int luna_graph_scan(const void* src, const void* dst, int index_bits, int64_t num_nodes, int64_t num_edges,
+                    int32_t* src32, int32_t* dst32, int32_t* dst_rowptr, int32_t* src_rowptr,
+                    int32_t* edge_ids_by_src, int32_t* edge_ids_by_dst, int32_t* seg_rowptr, int64_t* status,
+                    void* workspace, size_t workspace_bytes, LunaStream stream) {
+  return guard_call([&] {
+    if (index_bits != 32 && index_bits != 64) fail("luna_graph_scan: index_bits must be 32 or 64");
+    check_graph(num_nodes, num_edges, "luna_graph_scan");
+    if (!dst_rowptr || !src_rowptr || !seg_rowptr || !status) fail("luna_graph_scan: null table");
+    if (num_edges > 0 && (!src || !dst || !src32 || !dst32 || !edge_ids_by_src || !edge_ids_by_dst))
+      fail("luna_graph_scan: null edge table");
+    if (!workspace || workspace_bytes < workspace_bytes_of(num_nodes, num_edges))
+      fail("luna_graph_scan: workspace too small");
+    Arena arena{(char*)workspace, workspace_bytes};
+    Outputs o{};
+    o.src32 = src32, o.dst32 = dst32, o.dst_rowptr = dst_rowptr, o.src_rowptr = src_rowptr;
+    o.edge_ids_by_src = edge_ids_by_src, o.edge_ids_by_dst = edge_ids_by_dst, o.seg_rowptr = seg_rowptr;
+    scan_half(graph_module(nullptr), (hipStream_t)stream, arena, src, dst, index_bits == 64, num_nodes, num_edges, o,
+              status);
+  });
+}
+
+int luna_graph_finish(const int32_t* dst_rowptr, const int32_t* src_rowptr, const int32_t* seg_rowptr,
+                      int64_t num_nodes, int64_t num_edges, int64_t largest_degree, int64_t segments,
+                      int32_t* node_order, int32_t* source_node_order, int32_t* node_tiers, int32_t* seg_nodes,
+                      int32_t* seg_begin, int32_t* seg_end, int32_t* seg_order, void* workspace,
+                      size_t workspace_bytes, LunaStream stream) {
+  return guard_call([&] {
+    check_graph(num_nodes, num_edges, "luna_graph_finish");
+    if (largest_degree < 0 || largest_degree > num_edges || segments < 0 || segments > num_nodes + num_edges / kSegment + 1)
+      fail("luna_graph_finish: degree or segment count out of range");
+    if (!dst_rowptr || !src_rowptr || !seg_rowptr || !node_tiers) fail("luna_graph_finish: null table");
+    if (num_nodes > 0 && (!node_order || !source_node_order || !seg_nodes || !seg_begin || !seg_end || !seg_order))
+      fail("luna_graph_finish: null node table");
+    if (!workspace || workspace_bytes < workspace_bytes_of(num_nodes, num_edges))
+      fail("luna_graph_finish: workspace too small");
+    Arena arena{(char*)workspace, workspace_bytes};
+    Outputs o{};
+    o.dst_rowptr = const_cast<int32_t*>(dst_rowptr), o.src_rowptr = const_cast<int32_t*>(src_rowptr);
+    o.seg_rowptr = const_cast<int32_t*>(seg_rowptr), o.node_order = node_order;
+    o.source_node_order = source_node_order, o.node_tiers = node_tiers, o.seg_nodes = seg_nodes;
+    o.seg_begin = seg_begin, o.seg_end = seg_end, o.seg_order = seg_order;
+    node_half(graph_module(nullptr), (hipStream_t)stream, arena, num_nodes, num_edges, largest_degree, segments, o);
   });
 }
 

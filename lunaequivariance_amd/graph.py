@@ -236,10 +236,11 @@ def _check_nodes(num_nodes, required, num_edges):
 
 def _make_graph_device(src: torch.Tensor, dst: torch.Tensor, num_nodes) -> LunaTPGraph:
     """Tables of a device graph from the HIP kernels of the C-ABI library
-    (``luna_graph_bounds`` / ``luna_graph_build``; the reference's topology
+    (``luna_graph_scan`` / ``luna_graph_finish``; the reference's topology
     extension, ``src/lunatp/utils/graph.py:142-846``).  The indices are always
-    validated (one read-back of min, max and sortedness), also when
-    ``num_nodes`` is given, because every later kernel indexes with them."""
+    validated (one read-back of min, max and sortedness, together with the
+    segment count and the largest degrees), also when ``num_nodes`` is given,
+    because every later kernel indexes with them."""
     import ctypes
 
     from . import _native
@@ -248,56 +249,66 @@ def _make_graph_device(src: torch.Tensor, dst: torch.Tensor, num_nodes) -> LunaT
         dst = dst.to(src.dtype)
     src, dst = src.contiguous(), dst.contiguous()
     bits = 64 if src.dtype == torch.int64 else 32
-    num_edges = src.numel()
+    E = num_edges = src.numel()
     if wide_offsets(num_nodes or 0, num_edges):
         return _make_graph_torch(src, dst, num_nodes)
     device = src.device
     lib = _native.lib()
     _native.check(lib.luna_graph_precompile(_native.cache_dir().encode()), "luna_graph_precompile")
     stream = torch.cuda.current_stream(device).cuda_stream
-    required = 0
-    if num_edges:
-        status = torch.empty(4, dtype=torch.int64, device=device)
-        _native.check(lib.luna_graph_bounds(src.data_ptr(), dst.data_ptr(), bits, num_edges, status.data_ptr(),
-                                            stream), "luna_graph_bounds")
-        low, high, unsorted, _ = status.tolist()
+    status = torch.empty(8, dtype=torch.int64, device=device)
+
+    def validated(low, high, unsorted):
+        """The nodes the indices require."""
         if low < 0:
             raise ValueError("graph indices must be nonnegative.")
         if unsorted:
             raise ValueError(
                 "dst must be sorted in ascending order; src and edge data must follow the same order.")
-        required = high + 1
-    num_nodes = _check_nodes(num_nodes, required, num_edges)
-    if wide_offsets(num_nodes, num_edges):
-        # int64 edge offsets: torch's sorts and scans on the device (the HIP
-        # builder's radix sort carries int32 edge ids).
-        return _make_graph_torch(src, dst, num_nodes)
-    i32 = torch.int32
-    E, N = num_edges, num_nodes
-    cap = N + E // SOURCE_SEGMENT_EDGES + 1
-    new = lambda n: torch.empty(n, dtype=i32, device=device)
+        return high + 1
+
+    if num_nodes is None:
+        required = 0
+        if num_edges:
+            _native.check(lib.luna_graph_bounds(src.data_ptr(), dst.data_ptr(), bits, num_edges, status.data_ptr(),
+                                                stream), "luna_graph_bounds")
+            required = validated(*status[:3].tolist())
+        num_nodes = _check_nodes(None, required, num_edges)
+        if wide_offsets(num_nodes, num_edges):
+            # int64 edge offsets: torch's sorts and scans on the device (the HIP
+            # builder's radix sort carries int32 edge ids).
+            return _make_graph_torch(src, dst, num_nodes)
+    elif num_nodes < 0:
+        return _check_nodes(num_nodes, 0, num_edges)
+    N = num_nodes
+    new = lambda n: torch.empty(n, dtype=torch.int32, device=device)  # noqa: E731
     t = {name: new(n) for name, n in (
         ("src", E), ("dst", E), ("dst_rowptr", N + 1), ("src_rowptr", N + 1), ("edge_ids_by_src", E),
         ("edge_ids_by_dst", E), ("node_order", N), ("source_node_order", N), ("node_tiers", 3),
-        ("seg_rowptr", N + 1), ("seg_nodes", cap), ("seg_begin", cap), ("seg_end", cap), ("seg_order", cap))}
+        ("seg_rowptr", N + 1))}
     size = ctypes.c_size_t()
     _native.check(lib.luna_graph_workspace(N, E, ctypes.byref(size)), "luna_graph_workspace")
     workspace = torch.empty(max(size.value, 1), dtype=torch.uint8, device=device)
-    order = ("src", "dst", "dst_rowptr", "src_rowptr", "edge_ids_by_src", "edge_ids_by_dst", "node_order",
-             "source_node_order", "node_tiers", "seg_rowptr", "seg_nodes", "seg_begin", "seg_end", "seg_order")
-    _native.check(lib.luna_graph_build(
+    scratch = (workspace.data_ptr(), size.value, stream)
+    address = lambda *names: (t[name].data_ptr() if t[name].numel() else None for name in names)  # noqa: E731
+    _native.check(lib.luna_graph_scan(
         src.data_ptr() if E else None, dst.data_ptr() if E else None, bits, N, E,
-        *(t[name].data_ptr() if t[name].numel() else None for name in order),
-        workspace.data_ptr(), size.value, stream), "luna_graph_build")
-    segments = int(t["seg_rowptr"][N].item()) if N else 0
+        *address("src", "dst", "dst_rowptr", "src_rowptr", "edge_ids_by_src", "edge_ids_by_dst", "seg_rowptr"),
+        status.data_ptr(), *scratch), "luna_graph_scan")
+    low, high, unsorted, segments, most_in, most_out, _, _ = status.tolist()
+    _check_nodes(N, validated(low, high, unsorted) if E else 0, num_edges)
+    t.update({name: new(segments) for name in ("seg_nodes", "seg_begin", "seg_end", "seg_order")})
+    _native.check(lib.luna_graph_finish(
+        *address("dst_rowptr", "src_rowptr", "seg_rowptr"), N, E, max(most_in, most_out), segments,
+        *address("node_order", "source_node_order", "node_tiers", "seg_nodes", "seg_begin", "seg_end", "seg_order"),
+        *scratch), "luna_graph_finish")
     return LunaTPGraph(
         src=t["src"], dst=t["dst"], num_nodes=N,
         dst_rowptr=t["dst_rowptr"], src_rowptr=t["src_rowptr"],
         edge_ids_by_src=t["edge_ids_by_src"], edge_ids_by_dst=t["edge_ids_by_dst"],
         node_order=t["node_order"], source_node_order=t["source_node_order"], node_tiers=t["node_tiers"],
         source_segments=SourceSegmentTables(
-            t["seg_nodes"][:segments], t["seg_begin"][:segments], t["seg_end"][:segments], t["seg_rowptr"],
-            t["seg_order"][:segments]),
+            t["seg_nodes"], t["seg_begin"], t["seg_end"], t["seg_rowptr"], t["seg_order"]),
     )
 
 
