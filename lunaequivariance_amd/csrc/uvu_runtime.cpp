@@ -180,7 +180,7 @@ int luna_uvu_plan_info(const LunaUvuPlan* plan, LunaUvuPlanInfo* info) {
 int luna_uvu_plan_precompile(LunaUvuPlan* plan) {
   return guard_call([&] {
     if (!plan) fail("luna_uvu_plan_precompile: null plan");
-    for (const char* v : {"fwd00", "fws00", "bwd00111"})
+    for (const char* v : {"fwd00", "bwd00111"})
       plan->plan.kernels.code_for(v, [&] { return source_for(plan->plan, v); });
   });
 }
