@@ -144,6 +144,19 @@ hipModule_t ModuleCache::module_for(const std::string& variant, const std::funct
   return module;
 }
 
+hipFunction_t ModuleCache::find(uint64_t code, int device) {
+  std::lock_guard<std::mutex> guard(lock);
+  for (const Known& k : known)
+    if (k.code == code && k.device == device) return k.function;
+  return nullptr;
+}
+
+hipFunction_t ModuleCache::remember(uint64_t code, int device, hipFunction_t function) {
+  std::lock_guard<std::mutex> guard(lock);
+  known.push_back({code, device, function});
+  return function;
+}
+
 hipFunction_t function_for(hipModule_t module, const std::string& name) {
   hipFunction_t function;
   check_hip(hipModuleGetFunction(&function, module, name.c_str()), ("hipModuleGetFunction " + name).c_str());

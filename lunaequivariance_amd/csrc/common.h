@@ -31,9 +31,32 @@ struct ModuleCache {
   ~ModuleCache();
   const std::vector<char>& code_for(const std::string& variant, const std::function<std::string()>& source);
   hipModule_t module_for(const std::string& variant, const std::function<std::string()>& source);
+
+  // Kernels looked up before, by the caller's code for (variant, kernel): a
+  // launch then builds no names and does not search the module again.
+  struct Known {
+    uint64_t code;
+    int device;
+    hipFunction_t function;
+  };
+  std::vector<Known> known;
+  hipFunction_t find(uint64_t code, int device);
+  hipFunction_t remember(uint64_t code, int device, hipFunction_t function);
+  // `variant`, `source` and `name` (callables) are asked on the first use only.
+  template <typename V, typename S, typename N>
+  hipFunction_t function(uint64_t code, V variant, S source, N name);
 };
 
 hipFunction_t function_for(hipModule_t module, const std::string& name);
+
+template <typename V, typename S, typename N>
+hipFunction_t ModuleCache::function(uint64_t code, V variant, S source, N name) {
+  int device = 0;
+  check_hip(hipGetDevice(&device), "hipGetDevice");
+  if (hipFunction_t f = find(code, device)) return f;
+  const std::string v = variant();
+  return remember(code, device, function_for(module_for(v, [&] { return source(v); }), name()));
+}
 
 // Launch on `stream`; while profiling is enabled the launch is bracketed by
 // HIP events recorded under `name`.

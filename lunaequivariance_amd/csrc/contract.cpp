@@ -496,8 +496,11 @@ std::string emit(const CPlan& p) {
   return s;
 }
 
-hipModule_t module_of(CPlan& p) {
-  return p.kernels.module_for("all", [&] { return emit(p); });
+hipFunction_t kernel_of(CPlan& p, int which) {
+  static const char* const names[] = {"luna_con_fwd", "luna_con_ga", "luna_con_gw", "luna_con_gw_reduce"};
+  return p.kernels.function(
+      which, [] { return std::string("all"); }, [&](const std::string&) { return emit(p); },
+      [&] { return std::string(names[which]); });
 }
 
 unsigned grid_x(int64_t tiles) {
@@ -516,7 +519,7 @@ void product(CPlan& p, const void* in, const void* wt, void* out, int64_t rows, 
     tiles += ceil_div(rows, tile_nodes(p.bits, b, mn)) * ceil_div(ceil_div(mn, tile_m(mn)), group);
   }
   void* args[] = {&in, &wt, &out, &rows, &group};
-  launch(swap ? "con_ga" : "con_fwd", function_for(module_of(p), swap ? "luna_con_ga" : "luna_con_fwd"),
+  launch(swap ? "con_ga" : "con_fwd", kernel_of(p, swap),
          dim3(grid_x(tiles)), dim3(256), s, args);
 }
 
@@ -591,14 +594,13 @@ int luna_con_grad_w(const LunaConPlan* cplan, const void* a, const void* g, void
       groups += ceil_div(rows, grad_rows(p, b, span)) * grad_tiles(b);
       tiles += grad_tiles(b);
     }
-    hipModule_t module = module_of(p);
     hipStream_t s = (hipStream_t)stream;
     if (rows > 0) {
       void* args[] = {&a, &g, &workspace, &rows, &span};
-      launch("con_gw", function_for(module, "luna_con_gw"), dim3(grid_x(groups)), dim3(256), s, args);
+      launch("con_gw", kernel_of(p, 2), dim3(grid_x(groups)), dim3(256), s, args);
     }
     void* args[] = {&workspace, &gw, &rows, &span};
-    launch("con_gw_reduce", function_for(module, "luna_con_gw_reduce"), dim3(grid_x(tiles * 64)), dim3(256), s, args);
+    launch("con_gw_reduce", kernel_of(p, 3), dim3(grid_x(tiles * 64)), dim3(256), s, args);
   });
 }
 

@@ -855,8 +855,13 @@ int luna_uuu_conv_fwd(const LunaUuuPlan* cplan, const void* x, const void* y, co
     if (!x || !out || !dst_rowptr || !node_order) fail("luna_uuu_conv_fwd: null tensor");
     if (num_edges > 0 && (!y || !src || (p.spec.wnum > 0 && !w))) fail("luna_uuu_conv_fwd: null edge tensor");
     if (l0 && p.spec.l0 == 0) l0 = nullptr;
-    const std::string v = std::string("fwd") + (env ? '1' : '0') + (l0 ? '1' : '0');
-    hipModule_t module = p.kernels.module_for(v, [&] { return source_for(p, v); });
+    auto kernel = [&](size_t gi) {
+      return p.kernels.function(
+          (uint64_t)gi << 8 | (uint64_t)(env != nullptr) << 1 | (uint64_t)(l0 != nullptr),
+          [&] { return std::string("fwd") + (env ? '1' : '0') + (l0 ? '1' : '0'); },
+          [&](const std::string& v) { return source_for(p, v); },
+          [&] { return "luna_uuu_fwd_g" + std::to_string(gi); });
+    };
     for (size_t gi = 0; gi < p.fwd.size(); ++gi) {
       const UGroup& g = p.fwd[gi];
       const int64_t items = num_nodes * g.chunks;
@@ -864,7 +869,7 @@ int luna_uuu_conv_fwd(const LunaUuuPlan* cplan, const void* x, const void* y, co
       for (int b : g.obs) accs += p.spec.oblocks[b].d;
       int split = split_for(items, accs, p.spec.bits);
       void* args[] = {&x, &y, &w, &env, &src, &dst_rowptr, &node_order, &out, &l0, &split};
-      launch("uuu_fwd", function_for(module, "luna_uuu_fwd_g" + std::to_string(gi)), dim3(blocks_for(items)),
+      launch("uuu_fwd", kernel(gi), dim3(blocks_for(items)),
              dim3(64 * split), (hipStream_t)stream, args, (unsigned)lds_bytes(split, accs, p.spec.bits));
     }
   });
@@ -909,10 +914,20 @@ int luna_uuu_conv_bwd(const LunaUuuPlan* cplan, const void* x, const void* y, co
       }
     }
     const hipStream_t s = (hipStream_t)stream;
-    const std::string flags = std::string() + (env ? '1' : '0') + (gl0 ? '1' : '0') + (gx ? '1' : '0') +
-                              (gy ? '1' : '0') + (gw ? '1' : '0') + (genv ? '1' : '0');
-    const std::string v = "bwd" + flags;
-    hipModule_t module = p.kernels.module_for(v, [&] { return source_for(p, v); });
+    const void* const flags[] = {env, gl0, gx, gy, gw, genv};
+    uint64_t code = 1 << 7;
+    for (int n = 0; n < 6; ++n) code |= (uint64_t)(flags[n] != nullptr) << n;
+    auto kernel = [&](size_t gi, const char* name) {
+      return p.kernels.function(
+          (uint64_t)gi << 8 | code,
+          [&] {
+            std::string v = "bwd";
+            for (const void* f : flags) v += f ? '1' : '0';
+            return v;
+          },
+          [&](const std::string& v) { return source_for(p, v); },
+          [&] { return gi == p.bwd.size() ? std::string(name) : name + std::to_string(gi); });
+    };
     for (size_t gi = 0; gi < p.bwd.size(); ++gi) {
       const UGroup& grp = p.bwd[gi];
       const int64_t items = num_nodes * grp.chunks;
@@ -922,12 +937,12 @@ int luna_uuu_conv_bwd(const LunaUuuPlan* cplan, const void* x, const void* y, co
       int split = split_for(items, accs, p.spec.bits);
       void* args[] = {&x, &y, &w, &env, &g, &gl0, &dst, &src_rowptr, &edge_ids_by_src, &source_node_order,
                       &gx, &gy, &gw, &part, &split, &E};
-      launch("uuu_bwd", function_for(module, "luna_uuu_bwd_g" + std::to_string(gi)), dim3(blocks_for(items)),
+      launch("uuu_bwd", kernel(gi, "luna_uuu_bwd_g"), dim3(blocks_for(items)),
              dim3(64 * split), s, args, (unsigned)lds_bytes(split, accs, p.spec.bits));
     }
     if (genv && p.genv_slots > 1) {
       void* args[] = {&part, &genv, &E};
-      launch("uuu_genv_reduce", function_for(module, "luna_uuu_genv_reduce"), dim3((unsigned)((E + 255) / 256)),
+      launch("uuu_genv_reduce", kernel(p.bwd.size(), "luna_uuu_genv_reduce"), dim3((unsigned)((E + 255) / 256)),
              dim3(256), s, args);
     }
   });

@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 
 #include "../../include/lunaeq_amd.h"
 #include "uvu_plan.h"
@@ -19,8 +20,20 @@ std::string source_for(const Plan& plan, const std::string& variant) {
   return emit_backward(plan, flag(3), flag(4), flag(5), flag(6), flag(7));
 }
 
-hipModule_t module_for(Plan& plan, const std::string& variant) {
-  return plan.kernels.module_for(variant, [&] { return source_for(plan, variant); });
+// Kernel `name` of variant <kind><flags...>; `kind` 0 fwd, 1 fws, 2 bwd.
+template <typename N>
+hipFunction_t kernel_of(Plan& plan, int kind, std::initializer_list<bool> flags, int which, N name) {
+  uint64_t code = (uint64_t)which << 8 | (uint64_t)kind << 6;
+  int bit = 0;
+  for (bool f : flags) code |= (uint64_t)f << bit++;
+  return plan.kernels.function(
+      code,
+      [&] {
+        std::string v = kind == 0 ? "fwd" : kind == 1 ? "fws" : "bwd";
+        for (bool f : flags) v += f ? '1' : '0';
+        return v;
+      },
+      [&](const std::string& v) { return source_for(plan, v); }, name);
 }
 
 // Workspace layout: gy/genv partials, then the per-edge gx messages.
@@ -95,20 +108,21 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
       fail("luna_uvu_conv_bwd: workspace too small");
     void* part = want_parts ? workspace : nullptr;
     void* msg = want_msg ? (void*)((char*)workspace + pbytes) : nullptr;
-    std::string variant = std::string("bwd") + (env ? '1' : '0') + (gl0 ? '1' : '0') + (gw ? '1' : '0') +
-                          (want_msg ? '1' : '0') + (want_parts ? '1' : '0');
-    hipModule_t module = module_for(plan, variant);
+    auto kernel = [&](int which, const char* name, int phase) {
+      return kernel_of(plan, 2, {env != nullptr, gl0 != nullptr, gw != nullptr, want_msg, want_parts}, which,
+                       [&] { return phase < 0 ? std::string(name) : name + std::to_string(phase); });
+    };
     hipStream_t s = (hipStream_t)stream;
     if (want_msg && plan.bwd_gx_needs_zero) {
       int64_t n = E * (int64_t)plan.spec.in1;
       if ((n + 255) / 256 > 0xffffffffLL) fail("luna_uvu_conv_bwd: message fill exceeds the launch grid");
       void* args[] = {&msg, &n};
-      launch("uvu_fill", function_for(module, "luna_uvu_fill"), dim3((unsigned)((n + 255) / 256)), dim3(256), s,
+      launch("uvu_fill", kernel(0, "luna_uvu_fill", -1), dim3((unsigned)((n + 255) / 256)), dim3(256), s,
              args);
     }
     if (E > 0 && (gw || want_parts || want_msg)) {
       for (int phase = 0; phase < plan.bwd_phases; ++phase) {
-        hipFunction_t f = function_for(module, "luna_uvu_bwd_p" + std::to_string(phase));
+        hipFunction_t f = kernel(3 + phase, "luna_uvu_bwd_p", phase);
         void* args[] = {&x, &y, &w, &env, &g, &gl0, &src, &dst_rowptr, &node_order, &gw, &msg, &part, &E};
         dim3 grid = grid_for(num_nodes, plan.bwd_phase_slots[phase], plan.bwd_block_waves[phase]);
         grid.z = edge_split(plan.bwd_groups, phase, num_nodes * plan.bwd_phase_slots[phase], num_nodes, E,
@@ -119,7 +133,7 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
     }
     if (want_parts) {
       void* args[] = {&part, &gy, &genv, &E};
-      launch("uvu_bwd_reduce", function_for(module, "luna_uvu_bwd_reduce"), dim3((unsigned)((E + 255) / 256)),
+      launch("uvu_bwd_reduce", kernel(1, "luna_uvu_bwd_reduce", -1), dim3((unsigned)((E + 255) / 256)),
              dim3(256), s, args);
     }
     if (gx) {
@@ -127,7 +141,7 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
       void* args[] = {&msg, &src_rowptr, &edge_ids_by_src, &gx};
       const int vec = gather_vector_width(plan);
       const int64_t per_block = (int64_t)gather_columns(plan) * vec;
-      launch("uvu_bwd_gather", function_for(module, "luna_uvu_bwd_gather"),
+      launch("uvu_bwd_gather", kernel(2, "luna_uvu_bwd_gather", -1),
              dim3((unsigned)num_nodes, (unsigned)((plan.spec.in1 + per_block - 1) / per_block)),
              dim3(gather_columns(plan) * gather_teams(plan)), s, args);
     }
@@ -202,9 +216,8 @@ int luna_uvu_conv_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
                              kForwardWaves);
       const size_t wave_lds = split_forward_lds(plan, phase) * (plan.spec.dtype_bits / 8);
       while (split > 1 && split * wave_lds > 65536) split /= 2;
-      const std::string variant = std::string(split > 1 ? "fws" : "fwd") + (env ? '1' : '0') + (l0 ? '1' : '0');
-      hipModule_t module = module_for(plan, variant);
-      hipFunction_t f = function_for(module, "luna_uvu_fwd_p" + std::to_string(phase));
+      hipFunction_t f = kernel_of(plan, split > 1, {env != nullptr, l0 != nullptr}, phase,
+                                  [&] { return "luna_uvu_fwd_p" + std::to_string(phase); });
       void* args[] = {&x, &y, &w, &env, &src, &dst_rowptr, &node_order, &out, &l0};
       if (split > 1) {
         launch("uvu_fwd_p" + std::to_string(phase), f, dim3((unsigned)num_nodes, (unsigned)plan.phase_slots[phase]),

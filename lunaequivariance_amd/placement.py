@@ -148,12 +148,12 @@ def run_with_workspace(device: torch.device, nbytes: int, avoid, launch, place: 
     may overwrite parts of it before ``launch`` fills it) or None; ``place``
     False takes an ordinary allocation.
     """
-    stream = torch.cuda.current_stream(device)
-    if (not place or not _enabled() or nbytes < PLACE_MIN_BYTES
+    if (not place or nbytes < PLACE_MIN_BYTES or not _enabled()
             or torch.cuda.is_current_stream_capturing()):
         scratch = torch.empty(nbytes, device=device, dtype=torch.uint8)
         launch(scratch.data_ptr())
         return
+    stream = torch.cuda.current_stream(device)
     if avoid is not None and (not avoid.is_contiguous() or _nbytes(avoid) < PROBE_BYTES):
         avoid = None
     index = device.index if device.index is not None else torch.cuda.current_device()

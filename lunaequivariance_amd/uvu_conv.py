@@ -147,6 +147,12 @@ class NativePlan:
         _native.check(lib.luna_uvu_plan_info(handle, ctypes.byref(info)), "luna_uvu_plan_info")
         self.info = info
 
+    def bwd_workspace_bytes(self, nodes: int, edges: int) -> int:
+        size = ctypes.c_size_t()
+        _native.check(_native.lib().luna_uvu_conv_bwd_workspace(self.handle, nodes, edges, ctypes.byref(size)),
+                      "luna_uvu_conv_bwd_workspace")
+        return size.value
+
     def precompile(self):
         _native.check(_native.lib().luna_uvu_plan_precompile(self.handle), "luna_uvu_plan_precompile")
 
@@ -231,11 +237,12 @@ class LunaTPUVUConv:
 def edge_index_bits(graph) -> int:
     """32 or 64: the width of the graph's edge-offset tables (dst_rowptr,
     src_rowptr, edge_ids_by_src must agree; node ids are int32)."""
-    widths = {t.dtype for t in (graph.dst_rowptr, graph.src_rowptr, graph.edge_ids_by_src)}
-    if widths == {torch.int32}:
-        return 32
-    if widths == {torch.int64}:
-        return 64
+    width = graph.dst_rowptr.dtype
+    if graph.src_rowptr.dtype is width and graph.edge_ids_by_src.dtype is width:
+        if width is torch.int32:
+            return 32
+        if width is torch.int64:
+            return 64
     raise TypeError("graph edge-offset tables must all be int32 or all int64")
 
 
@@ -259,8 +266,7 @@ def create_uvu_conv_operator(tp_or_meta, *, dtype=None):
 # Kernel calls (no autograd)
 # ---------------------------------------------------------------------------
 
-def _stream(tensor) -> int:
-    return torch.cuda.current_stream(tensor.device).cuda_stream
+_stream = _native.stream_of
 
 
 def _check_device(op, graph, *tensors):
@@ -269,11 +275,11 @@ def _check_device(op, graph, *tensors):
             continue
         if not t.is_cuda:
             raise RuntimeError("convolution kernels run on the GPU; got a CPU tensor")
-        if t.dtype != op.compute_dtype:
+        if t.dtype is not op.compute_dtype:
             raise TypeError(f"expected {op.compute_dtype}, got {t.dtype}")
     if not graph.src.is_cuda:
         raise RuntimeError("graph tables must live on the GPU; build the graph from GPU tensors")
-    if any(t.dtype != torch.int32 for t in (graph.src, graph.dst, graph.node_order, graph.source_node_order)):
+    if not (graph.src.dtype is graph.dst.dtype is graph.node_order.dtype is graph.source_node_order.dtype is torch.int32):
         raise TypeError("graph node-id tables (src, dst, node_order, source_node_order) must be int32")
 
 
@@ -294,7 +300,7 @@ def run_forward(op, x, y, w, graph, env=None, want_l0=False):
         l0 = torch.empty((E, op.l0_dim), device=x.device, dtype=x.dtype)
     if N:
         _native.check(_native.lib().luna_uvu_conv_fwd(
-            plan.handle, x.data_ptr(), _native.ptr(y), _native.ptr(w), _native.ptr(env),
+            plan.handle, x.data_ptr(), y.data_ptr(), w.data_ptr(), _native.ptr(env),
             graph.src.data_ptr(), graph.dst_rowptr.data_ptr(), graph.node_order.data_ptr(),
             out.data_ptr(), _native.ptr(l0) if (l0 is not None and l0.numel()) else None,
             N, E, _stream(x)), "luna_uvu_conv_fwd")
@@ -321,23 +327,19 @@ def run_backward(op, x, y, w, graph, g, env=None, gl0=None, needs=(True, True, T
         genv = torch.empty((E,), device=x.device, dtype=x.dtype)
     if N and (need_x or ((need_y or need_w or need_env) and E)):
         lib = _native.lib()
-        size = ctypes.c_size_t()
-        _native.check(lib.luna_uvu_conv_bwd_workspace(plan.handle, N, E, ctypes.byref(size)),
-                      "luna_uvu_conv_bwd_workspace")
+        size = plan.bwd_workspace_bytes(N, E) if (need_x or need_y or need_env) and E else 0
 
         def launch(workspace):
             _native.check(lib.luna_uvu_conv_bwd(
-                plan.handle, x.data_ptr(), _native.ptr(y), _native.ptr(w), _native.ptr(env),
+                plan.handle, x.data_ptr(), y.data_ptr(), w.data_ptr(), _native.ptr(env),
                 g.data_ptr(), _native.ptr(gl0) if (gl0 is not None and gl0.numel()) else None,
                 graph.src.data_ptr(), graph.dst_rowptr.data_ptr(), graph.node_order.data_ptr(),
                 graph.src_rowptr.data_ptr(), graph.edge_ids_by_src.data_ptr(),
                 _native.ptr(gx), _native.ptr(gy), _native.ptr(gw), _native.ptr(genv),
-                workspace, size.value if workspace is not None else 0,
-                N, E, _stream(x)), "luna_uvu_conv_bwd")
+                workspace, size, N, E, _stream(x)), "luna_uvu_conv_bwd")
 
-        if (need_x or need_y or need_env) and E:
-            run_with_workspace(x.device, size.value, gw if gw is not None else gx, launch,
-                               place=x.dtype == torch.float32)
+        if size:
+            run_with_workspace(x.device, size, gw if gw is not None else gx, launch, place=x.dtype is torch.float32)
         else:
             launch(None)
     if gy is not None and not E:

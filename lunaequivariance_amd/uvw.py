@@ -170,8 +170,7 @@ class LunaTPUVW:
         return state
 
 
-def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+_stream = _native.stream_of
 
 
 def _check(op, *tensors):

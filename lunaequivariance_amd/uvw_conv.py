@@ -122,7 +122,7 @@ class NativeContraction:
         """"out": (A, W) -> out; "a": (g, W) -> gA; "w": (A, g) -> gW."""
         self._check(a, b)
         a, b = a.contiguous(), b.contiguous()
-        lib, rows, stream = _native.lib(), a.shape[0], torch.cuda.current_stream(a.device).cuda_stream
+        lib, rows, stream = _native.lib(), a.shape[0], _native.stream_of(a)
         like = dict(device=a.device, dtype=a.dtype)
         if kind == "w":
             out = torch.empty((self.weight_numel,), **like)
