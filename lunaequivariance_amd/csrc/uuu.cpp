@@ -584,6 +584,21 @@ std::string emit_forward(const UuuPlan& plan, bool env, bool l0) {
   return c.s.str();
 }
 
+// Backward groups held to three waves per SIMD (168 registers).  Left alone, the
+// compiler hoists every load of the lmax-3 group and takes 251 registers, two
+// waves: 64 channels, 2,083 nodes, 109,000 edges, step 769 us, at three waves
+// with 8 registers spilled 686 us.  Blocks wider than 7 components spill 46 to
+// 240 registers at three waves, fp64 groups up to 31: left as they are, like the
+// groups whose estimate says that they fit by themselves (lmax 2: 56, 95
+// registers, which the hint would raise to 124).
+bool three_waves(const USpec& s, const UGroup& g) {
+  bool narrow = s.bits == 32 && cost(s, g.paths, true) > 80;
+  for (int b : g.xbs) narrow = narrow && s.xblocks[b].d <= 7;
+  for (int b : g.ybs) narrow = narrow && s.yblocks[b].d <= 7;
+  for (int b : g.obs) narrow = narrow && s.oblocks[b].d <= 7;
+  return narrow;
+}
+
 std::string emit_backward(const UuuPlan& plan, bool env, bool gl0, bool want_gx, bool want_gy,
                           bool want_gw, bool want_genv) {
   const USpec& s = plan.spec;
@@ -593,7 +608,8 @@ std::string emit_backward(const UuuPlan& plan, bool env, bool gl0, bool want_gx,
     const UGroup& g = plan.bwd[gi];
     const Uses use = uses_of(s, g);
     const int nsub = 64 / g.cw;
-    c.line("extern \"C\" __global__ void __launch_bounds__(512) luna_uuu_bwd_g%d(", (int)gi);
+    c.line("extern \"C\" __global__ void __launch_bounds__(512) %sluna_uuu_bwd_g%d(",
+           three_waves(s, g) ? "__attribute__((amdgpu_waves_per_eu(3))) " : "", (int)gi);
     c.line("    const real* __restrict__ x, const real* __restrict__ y, const real* __restrict__ w,");
     c.line("    const real* __restrict__ env, const real* __restrict__ g, const real* __restrict__ gl0,");
     c.line("    const int* __restrict__ dst, const eix* __restrict__ rowptr, const eix* __restrict__ edge_ids,");
