@@ -150,6 +150,26 @@ int luna_uvu_conv_bwd(const LunaUvuPlan* plan,
                       int64_t num_nodes, int64_t num_edges, LunaStream stream);
 
 /*
+ * Row-wise product: luna_uvu_conv_fwd with row b as node b, edge b and the
+ * source of edge b (no graph tables, no env and l0).  shared_w: w is one row
+ * [1, weight_numel] for all rows (always so with a w_broadcast plan).
+ * out must be zero-filled where the plan's fwd_needs_zero says so.
+ * replaces: the row-wise uvu forward (src/lunatp/interface.py:265-285)
+ */
+int luna_uvu_rows_fwd(const LunaUvuPlan* plan, const void* x, const void* y, const void* w, int shared_w,
+                      void* out, int64_t rows, LunaStream stream);
+/* Bytes of device workspace luna_uvu_rows_bwd needs where it writes gy, or gw of a shared row. */
+int luna_uvu_rows_bwd_workspace(const LunaUvuPlan* plan, int shared_w, int64_t rows, size_t* bytes);
+/*
+ * Its first-order backward: gx [rows, in1], gy [rows, in2] and gw [rows,
+ * weight_numel], or with shared_w [1, weight_numel] summed over the rows; each
+ * may be NULL.  gw must be NULL with a w_broadcast plan.
+ */
+int luna_uvu_rows_bwd(const LunaUvuPlan* plan, const void* x, const void* y, const void* w, int shared_w,
+                      const void* g, void* gx, void* gy, void* gw, void* workspace, size_t workspace_bytes,
+                      int64_t rows, LunaStream stream);
+
+/*
  * Device buffer of `bytes` (at least 1 GB) placed outside the HBM region of
  * `avoid` (a device buffer of avoid_bytes >= 2 GB whose contents the probe
  * overwrites; NULL: outside the region the allocator is filling now).

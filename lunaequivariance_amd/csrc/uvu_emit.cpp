@@ -535,6 +535,104 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
   c.line("    }");
 }
 
+// Loop over the rows of a row-wise product, where node, edge and source are the
+// same row: rows blockIdx.x, + gridDim.x, ... (64 / cw rows at once in a packed
+// group, lanes past the last row repeating it with ok == false).  The operands
+// of the next row are in flight while the current one is computed; a weight row
+// shared by every row is loaded once, before the loop.  `seeds`: also the rows'
+// output seeds, loaded where they are used (requested a row ahead they take up to
+// twice the registers, at the same time: 183 us either way at 64 channels, lmax 2,
+// 50,000 rows).  Bound by memory: that backward moves 0.89 GB (4.9 TB/s), its
+// forward 0.77 GB in 157 us.
+void emit_row_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& use, bool shared, bool nt_w, bool seeds,
+                   const std::function<void()>& body) {
+  const int np = (int)g.paths.size(), nsub = 64 / g.cw;
+  const bool packed = nsub > 1;
+  struct Operand {
+    std::string name, address;
+    char cls;
+    bool nt;
+  };
+  std::vector<Operand> ops, direct;
+  auto at = [&](const char* base, const char* row, long off, int stride) {
+    return std::string(base) + " + rn * " + row + " + (" + std::to_string(off) + " + uc * " + std::to_string(stride) + ")";
+  };
+  for (int i = 0; i < g.d1; ++i) ops.push_back({"x" + std::to_string(i), at("x", "IN1", g.x_off + i, g.d1), 'v', false});
+  for (int n = 0; n < np; ++n) {
+    const Path& q = spec.paths[g.paths[n]];
+    if (shared)
+      c.line("    const real w%d = w[%d + uc * %d];", n, q.w_off, q.w_stride);
+    else
+      ops.push_back({"w" + std::to_string(n), at("w", "WNUM", q.w_off, q.w_stride), 'v', nt_w});
+  }
+  if (seeds)
+    for (size_t b = 0; b < g.blocks.size(); ++b)
+      for (int k = 0; k < g.blocks[b].d3; ++k)
+        direct.push_back({"G" + std::to_string(b) + "_" + std::to_string(k),
+                       at("g", "OUTD", g.blocks[b].out_off + k, g.blocks[b].d3), 'v', false});
+  for (int yi : use.ys)
+    ops.push_back({"y" + std::to_string(yi), "y + rn * IN2 + " + std::to_string(yi), packed ? 'v' : 's', false});
+  auto load = [&](const std::string& row) {
+    c.line("      {");
+    const std::string mine = packed ? "(" + row + " + sub)" : row;
+    c.line("        const i64 rn = %s < end ? %s : end - 1;", mine.c_str(), mine.c_str());
+    for (const auto& o : ops)
+      c.line(o.nt ? "        n%s = __builtin_nontemporal_load(%s);" : "        n%s = *(%s);", o.name.c_str(),
+             o.address.c_str());
+    c.line("      }");
+  };
+  auto waits = [&]() {
+    for (const auto& o : ops) c.line("      asm volatile(\"\" :: \"%c\"(n%s));", o.cls, o.name.c_str());
+  };
+  c.line("    const i64 end = E, first = (i64)blockIdx.x * %d, step = (i64)gridDim.x * %d;", nsub, nsub);
+  c.line("    if (first < end) {");
+  for (const auto& o : ops) c.line("      real n%s;", o.name.c_str());
+  load("first");
+  waits();
+  c.line("      int it = 0;");
+  c.line("      for (i64 e0 = first; e0 < end; e0 += step, ++it) {");
+  c.line("      const i64 e = %s;", packed ? "e0 + sub < end ? e0 + sub : end - 1" : "e0");
+  if (packed) c.line("      const bool ok = e0 + sub < end;");
+  for (const auto& o : ops) c.line("      real %s = n%s;", o.name.c_str(), o.name.c_str());
+  if (!direct.empty()) {
+    c.line("      const i64 rn = e;");
+    for (const auto& o : direct) c.line("      const real %s = *(%s);", o.name.c_str(), o.address.c_str());
+  }
+  load("e0 + step");
+  body();
+  waits();
+  c.line("      }");
+  c.line("    }");
+}
+
+// Leaves values `names` (d per lane) of the current rows at dst[row, off + u * d + k]:
+// through the per-wave buffer `lds`, so that a wave stores consecutive values.
+void emit_row_store(Code& c, const Group& g, const std::vector<std::string>& names, const char* lds, const char* dst,
+                    const char* width, int off, bool accumulate) {
+  const int d = (int)names.size(), nsub = 64 / g.cw, per = g.cw * d;
+  c.line("      {");
+  for (int k = 0; k < d; ++k) c.line("        %s[lane * %d + %d] = %s;", lds, d, k, names[k].c_str());
+  c.line("        asm volatile(\"\" ::: \"memory\");");
+  c.line("        real* const ob = %s + e0 * %s + (%d + c0 * %d);", dst, width, off, d);
+  for (int m = 0; m < d; ++m) {
+    std::string cond, at = "ob + " + std::to_string(m * 64) + " + lane";
+    const std::string idx = std::to_string(m * 64) + " + lane";
+    if (nsub > 1) {
+      c.line("        const int q%d = (%s) / %d, i%d = (%s) - q%d * %d;", m, idx.c_str(), per, m, idx.c_str(), m, per);
+      cond = "if (i" + std::to_string(m) + " < nch * " + std::to_string(d) + " && e0 + q" + std::to_string(m) + " < end) ";
+      at = "ob + (i64)q" + std::to_string(m) + " * " + width + " + i" + std::to_string(m);
+    } else if (g.channels % 64) {
+      cond = "if (" + idx + " < nch * " + std::to_string(d) + ") ";
+    }
+    if (accumulate)
+      c.line("        %s*(%s) += %s[%s];", cond.c_str(), at.c_str(), lds, idx.c_str());
+    else
+      c.line("        %s__builtin_nontemporal_store(%s[%s], %s);", cond.c_str(), lds, idx.c_str(), at.c_str());
+  }
+  c.line("        asm volatile(\"\" ::: \"memory\");");
+  c.line("      }");
+}
+
 // Channel u (uc: clamped to the last) of this lane, and the edge of the wave it
 // works on (`sub`) in a packed group.
 void emit_lanes(Code& c, const Group& g, int slot_base, int subsets) {
@@ -550,16 +648,11 @@ void emit_lanes(Code& c, const Group& g, int slot_base, int subsets) {
   c.line("    const int uc = active ? u : %d;", g.channels - 1);
 }
 
-void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt,
-                        bool split) {
+// The products of one edge (or row) added to the accumulators A<block>_<k>.
+void emit_forward_body(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt) {
   const int bits = spec.dtype_bits;
-  GroupUse use = group_use(spec, g);
   const int np = (int)g.paths.size();
   const bool packed = g.cw < 64;
-  emit_lanes(c, g, g.slot_base, 1);
-  for (size_t b = 0; b < g.blocks.size(); ++b)
-    for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
-  auto body = [&]() {
   if (packed) c.line("      if (ok) {");
   // l0 columns are summed over the paths (edge copies) sharing them.
   std::map<int, std::vector<int>> l0_cols;
@@ -635,7 +728,16 @@ void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, boo
   for (const auto& col : l0_cols)
     c.line("      l0[(i64)e * L0DIM + %d + uc] = L%d;", col.first, col.first);
   if (packed) c.line("      }");
-  };
+}
+
+void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt,
+                        bool split) {
+  GroupUse use = group_use(spec, g);
+  const bool packed = g.cw < 64;
+  emit_lanes(c, g, g.slot_base, 1);
+  for (size_t b = 0; b < g.blocks.size(); ++b)
+    for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
+  auto body = [&]() { emit_forward_body(c, spec, g, env, l0, opt); };
   emit_edge_loop(c, spec, g, use, env, opt, {}, body, split);
   if (packed || split) {
     // The sums of a wave's edges, and of the waves sharing the node, meet in
@@ -716,6 +818,29 @@ void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, boo
   c.line("    }");
 }
 
+// First channel of this wave's chunk and the number of channels in it.
+void emit_chunk(Code& c, const Group& g, int subsets) {
+  c.line("    const int c0 = (slot - %d) / %d * %d;", g.slot_base, subsets, g.cw);
+  c.line("    const int nch = %d - c0 < %d ? %d - c0 : %d;", g.channels, g.cw, g.channels, g.cw);
+}
+
+void emit_rows_forward_group(Code& c, const Spec& spec, const Group& g, bool shared, const Options& opt) {
+  GroupUse use = group_use(spec, g);
+  emit_lanes(c, g, g.slot_base, 1);
+  emit_chunk(c, g, 1);
+  emit_row_loop(c, spec, g, use, shared, opt.fwd_nt_w, false, [&] {
+    for (size_t b = 0; b < g.blocks.size(); ++b)
+      for (int k = 0; k < g.blocks[b].d3; ++k) c.line("      real A%zu_%d = 0;", b, k);
+    emit_forward_body(c, spec, g, false, false, opt);
+    for (size_t b = 0; b < g.blocks.size(); ++b) {
+      const AccBlock& blk = g.blocks[b];
+      std::vector<std::string> names;
+      for (int k = 0; k < blk.d3; ++k) names.push_back("A" + std::to_string(b) + "_" + std::to_string(k));
+      emit_row_store(c, g, names, "obuf", "out", "OUTD", blk.out_off, blk.accumulate);
+    }
+  });
+}
+
 // Backward, destination-owned: the wave keeps the output seeds g[t] of its
 // group in registers and streams the node's in-edges, writing gw and the gy
 // partials per edge and the per-edge gx message msg[e, x block]; a second
@@ -724,9 +849,13 @@ void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, boo
 // a split group (`g` is then the subset's view, sub its index).
 Group subset_view(const Group& g, int sub);
 
+// What a backward wave streams: a node's edges, or the rows of a row-wise
+// product with a weight row each or one shared by all of them.
+enum class Rows { none, own, shared };
+
 void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, bool gl0, bool want_gw,
                         bool want_msg, bool want_part, const Options& opt, int sub, bool cmajor,
-                        const Group* whole) {
+                        const Group* whole, Rows rows) {
   const int bits = spec.dtype_bits;
   GroupUse use = group_use(spec, g);
   const int np = (int)g.paths.size();
@@ -734,8 +863,12 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   const bool packed = g.cw < 64;
   const int nsub = 64 / g.cw;
   emit_lanes(c, g, g.slot_base, g.subsets);
+  if (rows != Rows::none) emit_chunk(c, g, g.subsets);
+  const bool sum_gw = rows == Rows::shared && want_gw;
+  if (sum_gw)
+    for (int n = 0; n < np; ++n) c.line("    real GW%d = 0;", n);
   std::vector<std::string> seeds;
-  for (size_t b = 0; b < g.blocks.size(); ++b) {
+  for (size_t b = 0; b < g.blocks.size() && rows == Rows::none; ++b) {
     const AccBlock& blk = g.blocks[b];
     c.line("    const real* g%zu = g + (i64)t * OUTD + (%d + uc * %d);", b, blk.out_off, blk.d3);
     for (int k = 0; k < blk.d3; ++k) {
@@ -774,7 +907,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
       }
     }
     const int per_value = bits / 32;
-    int budget = opt.hoist_regs >= 0 ? opt.hoist_regs : 36;
+    int budget = rows != Rows::none ? -1 : opt.hoist_regs >= 0 ? opt.hoist_regs : 36;  // (rows: no node to hoist to)
     std::map<std::string, int> left = users;  // classes per seed not yet hoisted
     int extra = 0;                            // registers: hoisted values minus freed seeds
     auto cost = [&](const Candidate& cd) {
@@ -837,8 +970,10 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
       c.line("    const int r%d = %s;", s2, chain.c_str());
     }
   }
+  // Alternates between the iterations of the loop: the half of a shared LDS buffer.
+  const std::string parity = packed || rows != Rows::none ? "it & 1" : "(e - beg) & 1";
   auto body = [&]() {
-  if (!opt.hoist) {
+  if (!opt.hoist && rows == Rows::none) {
     // Opaque to the optimiser: keeps the edge-invariant q_ij inside the loop
     // instead of holding all of them in registers across it.
     for (const auto& name : seeds) c.line("      asm volatile(\"\" : \"+v\"(%s));", name.c_str());
@@ -878,7 +1013,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     if (g.pair_partials) {
       // Chunk 1 hands its sums to chunk 0 (two buffers by edge parity: one
       // barrier per edge orders both uses).
-      c.line("        const int par = (e - beg) & 1;");
+      c.line("        const int par = %s;", parity.c_str());
       c.line("        if (slot - %d == 1) {", g.slot_base);
       c.line("          if (own) gy_share[par][%d + col] = %s;", column[values[0]], total.c_str());
       c.line("          __syncthreads();");
@@ -980,7 +1115,9 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     } else {
       c.line("        const real ws = wv;");
     }
-    if (want_gw) {
+    if (sum_gw) {
+      c.line("        GW%d += gwv;", n);
+    } else if (want_gw) {
       if (opt.nt_gw)
         c.line("        __builtin_nontemporal_store(gwv, gw + (i64)e * WNUM + %d + uc * %d);", q.w_off, q.w_stride);
       else
@@ -991,7 +1128,6 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     c.line("      }");
   }
   if (packed) c.line("      }");
-  const std::string parity = packed ? "it & 1" : "(e - beg) & 1";
   std::vector<std::string> values;
   for (int yi : use.ys) values.push_back("GY" + std::to_string(yi));
   if (env) values.push_back("GE");
@@ -1020,7 +1156,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     std::string total = lds_reduce ? emit_lds_reduce(c, values, tag.c_str(), &shift, &low)
                                    : emit_butterfly(c, values, tag.c_str(), &shift, &low);
     c.line("        const int col = lane >> %d;", shift);
-    c.line("        if ((lane & %d) == 0 && col < %zu) gy_sub[%d][(e - beg) & 1][col] = %s;", low, values.size(), sub,
+    c.line("        if ((lane & %d) == 0 && col < %zu) gy_sub[%d][%s][col] = %s;", low, values.size(), sub, parity.c_str(),
            total.c_str());
     c.line("      }");
   };
@@ -1041,7 +1177,12 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     }
     c.line("      }");
   }
-  if (want_msg && sub == 0) {
+  if (want_msg && sub == 0 && rows != Rows::none) {
+    // The row's only message is its gx.
+    std::vector<std::string> names;
+    for (int i = 0; i < g.d1; ++i) names.push_back("M" + std::to_string(i));
+    emit_row_store(c, g, names, "red", "msg", "IN1", g.x_off, g.gx_accumulate);
+  } else if (want_msg && sub == 0) {
     // Lanes past the last channel repeat channel C-1 exactly, so their stores
     // write identical values; only the cross-lane sums below must mask them.
     // Component-major messages: component i of the 64 channels of a chunk is
@@ -1082,7 +1223,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   } else if (combine && sub == 0) {
     reduce_to_lds();
     c.line("      {");
-    c.line("        const int par = (e - beg) & 1;");
+    c.line("        const int par = %s;", parity.c_str());
     c.line("        if (r0 >= 0 || r1 >= 0)");
     c.line("          part[((i64)(%d + (slot - %d) / 2) * E + e) * PART_W + lane] =", whole->gy_slot_base,
            whole->slot_base);
@@ -1092,7 +1233,19 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   }
   if (!combine) flush(values);
   };
-  emit_edge_loop(c, spec, g, use, env, opt, seeds, body);
+  if (rows == Rows::none) {
+    emit_edge_loop(c, spec, g, use, env, opt, seeds, body);
+    return;
+  }
+  emit_row_loop(c, spec, g, use, rows == Rows::shared, opt.nt_w, true, body);
+  if (!sum_gw) return;
+  // The gradient of the shared weight row over this workgroup's rows.
+  for (int n = 0; n < np; ++n) {
+    const Path& q = spec.paths[g.paths[n]];
+    for (int m = g.cw; m < 64; m *= 2) c.line("    GW%d += xchg<%d>(GW%d);", n, m, n);
+    c.line("    if (active%s) gw[(i64)blockIdx.x * WNUM + %d + u * %d] = GW%d;", packed ? " && sub == 0" : "", q.w_off,
+           q.w_stride, n);
+  }
 }
 
 // The paths of subset `sub` of a split group, as a group of their own.
@@ -1116,16 +1269,16 @@ Group subset_view(const Group& g, int sub) {
 }
 
 void emit_backward_group(Code& c, const Spec& spec, const Group& g, bool env, bool gl0, bool want_gw,
-                         bool want_msg, bool want_part, const Options& opt, bool cmajor) {
+                         bool want_msg, bool want_part, const Options& opt, bool cmajor, Rows rows) {
   if (g.subsets == 1) {
-    emit_backward_wave(c, spec, g, env, gl0, want_gw, want_msg, want_part, opt, 0, cmajor, nullptr);
+    emit_backward_wave(c, spec, g, env, gl0, want_gw, want_msg, want_part, opt, 0, cmajor, nullptr, rows);
     return;
   }
   c.line("    const int sub = (slot - %d) %% %d;", g.slot_base, g.subsets);
   for (int sub = 0; sub < g.subsets; ++sub) {
     c.line("    %sif (sub == %d) {", sub ? "else " : "", sub);
     emit_backward_wave(c, spec, subset_view(g, sub), env, gl0, want_gw, want_msg, want_part, opt, sub, cmajor,
-                       &g);
+                       &g, rows);
     c.line("    }");
   }
 }
@@ -1203,7 +1356,8 @@ std::string emit_forward(const Plan& plan, bool env, bool l0, bool split) {
   return c.s.str();
 }
 
-std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bool want_msg, bool want_part) {
+static std::string backward_source(const Plan& plan, bool env, bool gl0, bool want_gw, bool want_msg, bool want_part,
+                                   Rows rows) {
   const Spec& spec = plan.spec;
   Options opt = options();
   opt.prefetch = opt.bwd_prefetch;
@@ -1216,11 +1370,15 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
   c.raw(prelude(spec, plan.edge_index_bits));
   for (int phase = 0; phase < plan.bwd_phases; ++phase) {
     const int waves = plan.bwd_block_waves[phase], slots = plan.bwd_phase_slots[phase];
-    c.line("extern \"C\" __global__ void __launch_bounds__(%d) %sluna_uvu_bwd_p%d(", 64 * std::max(waves, 1),
-           kernel_attributes(opt.bwd_wpe).c_str(), phase);
+    c.line("extern \"C\" __global__ void __launch_bounds__(%d) %sluna_uvu_%s_p%d(", 64 * std::max(waves, 1),
+           kernel_attributes(opt.bwd_wpe).c_str(), rows == Rows::none ? "bwd" : "rows_bwd", phase);
     c.line("    const real* __restrict__ x, const real* __restrict__ y, const real* __restrict__ w,");
-    c.line("    const real* __restrict__ env, const real* __restrict__ g, const real* __restrict__ gl0,");
-    c.line("    const int* __restrict__ src, const eix* __restrict__ rowptr, const int* __restrict__ order,");
+    if (rows == Rows::none) {
+      c.line("    const real* __restrict__ env, const real* __restrict__ g, const real* __restrict__ gl0,");
+      c.line("    const int* __restrict__ src, const eix* __restrict__ rowptr, const int* __restrict__ order,");
+    } else {
+      c.line("    const real* __restrict__ g,");
+    }
     c.line("    real* __restrict__ gw, real* __restrict__ msg, real* __restrict__ part, i64 E) {");
     int share_d1 = 0;
     for (const Group& g : plan.bwd_groups)
@@ -1239,17 +1397,25 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
     }
     bool packed = false;
     for (const Group& g : plan.bwd_groups) packed = packed || (g.phase == phase && g.cw < 64);
-    if (want_part && (packed || opt.lds_reduce != 0)) {
-      // Per-wave table of the LDS reduction of the gy partials.
-      int most = 1;
-      for (const Group& g : plan.bwd_groups)
-        if (g.phase == phase) most = std::max(most, (int)group_use(spec, g).ys.size() + (env ? 1 : 0));
-      const int pitch = reduce_pitch(most);
+    const bool stores = rows != Rows::none && want_msg;
+    if ((want_part && (packed || opt.lds_reduce != 0)) || stores) {
+      // Per-wave table of the LDS reduction of the gy partials; rows leave gx
+      // through it too.
+      int most = 1, widest = 1;
+      for (const Group& g : plan.bwd_groups) {
+        if (g.phase != phase) continue;
+        most = std::max(most, (int)group_use(spec, g).ys.size() + (env ? 1 : 0));
+        widest = std::max(widest, g.d1);
+      }
+      const int pitch = std::max(want_part ? reduce_pitch(most) : 1, stores ? widest : 1);
       c.line("  __shared__ real red_lds[%d];", std::max(waves, 1) * 64 * pitch);
       c.line("  real* const red = red_lds + %s * %d;",
              waves > 0 ? "__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)" : "0", 64 * pitch);
     }
-    if (waves == 0) {
+    if (rows != Rows::none) {
+      c.line("  const int lane = threadIdx.x & 63;");
+      c.line("  const int slot = blockIdx.y * %d + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);", std::max(waves, 1));
+    } else if (waves == 0) {
       // One wave per workgroup, the slots of a node on consecutive workgroups.
       c.line("  const int lane = threadIdx.x;");
       c.line("  const int t = order[blockIdx.x / %d];", slots);
@@ -1261,6 +1427,7 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
       c.line("  const int t = order[blockIdx.x];");
       c.line("  const int slot = blockIdx.y * %d + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);", waves);
     }
+    if (rows == Rows::none) {
     // Few nodes: a grid of more than one layer cuts every node's edges into as
     // many runs (nothing is summed over a node's edges here).
     c.line("  eix beg = rowptr[t], end = rowptr[t + 1];");
@@ -1269,6 +1436,7 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
     c.line("    beg += run * (eix)blockIdx.z;");
     c.line("    end = beg + run < end ? beg + run : end;");
     c.line("  }");
+    }
     bool first = true;
     for (const Group& g : plan.bwd_groups) {
       if (g.phase != phase) continue;
@@ -1276,7 +1444,7 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
       c.line("  %sif (slot >= %d && slot < %d) {", first ? "" : "else ", g.slot_base,
              g.slot_base + g.chunks * g.subsets);
       first = false;
-      emit_backward_group(c, spec, g, env, gl0, want_gw, want_msg, want_part, opt, cmajor);
+      emit_backward_group(c, spec, g, env, gl0, want_gw, want_msg, want_part, opt, cmajor, rows);
       c.line("  }");
     }
     c.line("}");
@@ -1381,6 +1549,30 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
   c.line("  const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;");
   c.line("  if (i < n) p[i] = 0;");
   c.line("}");
+  if (rows != Rows::none) {
+    if (rows == Rows::own || !want_gw) return c.s.str();
+    // Sum of the workgroups' gradients of the shared weight row: 32 columns and 32
+    // teams of threads per workgroup, so that few columns still keep many loads
+    // in flight.
+    c.line("extern \"C\" __global__ void __launch_bounds__(1024) luna_uvu_rows_gw(");
+    c.line("    const real* __restrict__ part, real* __restrict__ gw, int n) {");
+    c.line("  __shared__ real share[32][33];");
+    c.line("  const int lane = threadIdx.x & 31, team = threadIdx.x >> 5, col = blockIdx.x * 32 + lane;");
+    c.line("  real v = 0;");
+    c.line("  if (col < WNUM) {");
+    c.line("    #pragma unroll 8");
+    c.line("    for (int r = team; r < n; r += 32) v += part[(i64)r * WNUM + col];");
+    c.line("  }");
+    c.line("  share[team][lane] = v;");
+    c.line("  __syncthreads();");
+    c.line("  for (int h = 16; h; h >>= 1) {");
+    c.line("    if (team < h) share[team][lane] += share[team + h][lane];");
+    c.line("    __syncthreads();");
+    c.line("  }");
+    c.line("  if (team == 0 && col < WNUM) gw[col] = share[0][lane];");
+    c.line("}");
+    return c.s.str();
+  }
   // Segment sum of the gx messages over each source node's out-edges.
   std::vector<std::pair<long, long>> ranges;
   for (const Group& g : plan.bwd_groups) ranges.push_back({g.x_off, g.x_off + (long)g.channels * g.d1});
@@ -1474,6 +1666,41 @@ std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bo
     c.line("  *(vec_t*)(gx + (i64)s * IN1 + col) = acc0;");
   }
   c.line("}");
+  return c.s.str();
+}
+
+std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bool want_msg, bool want_part) {
+  return backward_source(plan, env, gl0, want_gw, want_msg, want_part, Rows::none);
+}
+
+std::string emit_rows_backward(const Plan& plan, bool shared, bool want_gw, bool want_msg, bool want_part) {
+  return backward_source(plan, false, false, want_gw, want_msg, want_part, shared ? Rows::shared : Rows::own);
+}
+
+std::string emit_rows_forward(const Plan& plan, bool shared) {
+  const Spec& spec = plan.spec;
+  const Options opt = options();
+  Code c;
+  c.raw(prelude(spec, plan.edge_index_bits));
+  for (int phase = 0; phase < plan.fwd_phases; ++phase) {
+    const int waves = std::max(plan.fwd_block_waves[phase], 1), per = split_forward_lds(plan, phase);
+    c.line("extern \"C\" __global__ void __launch_bounds__(%d) luna_uvu_rows_fwd_p%d(", 64 * waves, phase);
+    c.line("    const real* __restrict__ x, const real* __restrict__ y, const real* __restrict__ w,");
+    c.line("    real* __restrict__ out, i64 E) {");
+    c.line("  __shared__ __attribute__((aligned(16))) real obuf_lds[%d];", waves * per);
+    c.line("  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;");
+    c.line("  real* const obuf = obuf_lds + wave * %d;", per);
+    c.line("  const int slot = blockIdx.y * %d + wave;", waves);
+    bool first = true;
+    for (const Group& g : plan.fwd_groups) {
+      if (g.phase != phase) continue;
+      c.line("  %sif (slot < %d) {", first ? "" : "else ", g.slot_base + g.chunks);
+      first = false;
+      emit_rows_forward_group(c, spec, g, shared, opt);
+      c.line("  }");
+    }
+    c.line("}");
+  }
   return c.s.str();
 }
 

@@ -115,6 +115,10 @@ std::string emit_forward(const Plan& plan, bool env, bool l0, bool split);
 // LDS reals per wave of the split forward.
 int split_forward_lds(const Plan& plan, int phase);
 std::string emit_backward(const Plan& plan, bool env, bool gl0, bool want_gw, bool want_msg, bool want_part);
+// Row-wise products (row b is node, source and edge b); `shared`: one weight row
+// for every row, whose gradient is summed (a partial per workgroup, then one sum).
+std::string emit_rows_forward(const Plan& plan, bool shared);
+std::string emit_rows_backward(const Plan& plan, bool shared, bool want_gw, bool want_msg, bool want_part);
 
 // The first-order backward launches (luna_uvu_conv_bwd without the plan
 // check), with the caller's workspace of uvu_bwd_workspace_bytes bytes.

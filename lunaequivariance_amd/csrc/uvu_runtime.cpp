@@ -12,24 +12,29 @@ using namespace luna;
 namespace {
 
 std::string source_for(const Plan& plan, const std::string& variant) {
-  // Variant names: fwd<env><l0>, fws<env><l0> (split over waves) and
-  // bwd<env><gl0><gw><msg><part>, each flag '0' or '1'.
+  // Variant names: fwd<env><l0>, fws<env><l0> (split over waves),
+  // bwd<env><gl0><gw><msg><part>, and row-wise rwf<shared> and
+  // rwb<shared><gw><msg><part>, each flag '0' or '1'.
   auto flag = [&](size_t i) { return variant.size() > i && variant[i] == '1'; };
   if (variant.compare(0, 3, "fwd") == 0) return emit_forward(plan, flag(3), flag(4), false);
   if (variant.compare(0, 3, "fws") == 0) return emit_forward(plan, flag(3), flag(4), true);
+  if (variant.compare(0, 3, "rwf") == 0) return emit_rows_forward(plan, flag(3));
+  if (variant.compare(0, 3, "rwb") == 0) return emit_rows_backward(plan, flag(3), flag(4), flag(5), flag(6));
   return emit_backward(plan, flag(3), flag(4), flag(5), flag(6), flag(7));
 }
 
-// Kernel `name` of variant <kind><flags...>; `kind` 0 fwd, 1 fws, 2 bwd.
+// Kernel `name` of variant <kind><flags...>; at most five flags.
+enum Kind { kFwd, kFws, kBwd, kRwf, kRwb };
 template <typename N>
-hipFunction_t kernel_of(Plan& plan, int kind, std::initializer_list<bool> flags, int which, N name) {
-  uint64_t code = (uint64_t)which << 8 | (uint64_t)kind << 6;
+hipFunction_t kernel_of(Plan& plan, Kind kind, std::initializer_list<bool> flags, int which, N name) {
+  uint64_t code = (uint64_t)which << 8 | (uint64_t)kind << 5;
   int bit = 0;
   for (bool f : flags) code |= (uint64_t)f << bit++;
   return plan.kernels.function(
       code,
       [&] {
-        std::string v = kind == 0 ? "fwd" : kind == 1 ? "fws" : "bwd";
+        static const char* const names[] = {"fwd", "fws", "bwd", "rwf", "rwb"};
+        std::string v = names[kind];
         for (bool f : flags) v += f ? '1' : '0';
         return v;
       },
@@ -72,6 +77,33 @@ int edge_split(const std::vector<Group>& groups, int phase, int64_t waves, int64
 }
 constexpr int64_t kForwardWaves = 4096, kBackwardWaves = 8192;
 
+// Workgroups along the rows of a row-wise product: every wave loops over rows,
+// which keeps the next row's operands in flight and a shared weight row (and its
+// gradient) in registers.  64 channels, lmax 2, 50,000 rows, forward + backward +
+// weight sum: 2,048 waves 168 + 167 + 7 us, 4,096 156 + 198 + 8, 8,192 157 + 183 +
+// 13, 16,384 153 + 177 + 20, 40,000 150 + 175 + 40; fp64 uvw rows 313, 306, 301,
+// 300 and 302 us a step.  (Through the convolution kernels, with the weight row
+// expanded, per-row weight gradients summed by a library reduction and gx
+// messages gathered: 179 + 240 + 67 + 53 us and the expansion, step 557 us.)
+constexpr int64_t kRowWaves = 8192;
+unsigned row_blocks(const std::vector<Group>& groups, int phase, int slots, int64_t rows) {
+  int at_once = 64;
+  for (const Group& g : groups)
+    if (g.phase == phase) at_once = std::min(at_once, 64 / g.cw);
+  return (unsigned)std::max<int64_t>(1, std::min((rows + at_once - 1) / at_once, kRowWaves / std::max(slots, 1)));
+}
+// Partials of the shared weight row's gradient: a row per workgroup of the
+// largest launch (zeros where a launch has no rows left).
+int64_t row_gw_blocks(const Plan& p, int64_t rows) {
+  unsigned n = 1;
+  for (int phase = 0; phase < p.bwd_phases; ++phase)
+    n = std::max(n, row_blocks(p.bwd_groups, phase, p.bwd_phase_slots[phase], rows));
+  return n;
+}
+size_t row_gw_bytes(const Plan& p, int64_t rows) {
+  return align256((size_t)row_gw_blocks(p, rows) * (size_t)p.spec.wnum * (p.spec.dtype_bits / 8));
+}
+
 void check_sizes(const Plan& plan, int64_t num_nodes, int64_t num_edges) {
   if (num_nodes < 0 || num_edges < 0) fail("negative problem size");
   if (num_nodes > 0x7fffffffLL) fail("graph node count exceeds signed int32 capacity");
@@ -109,7 +141,7 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
     void* part = want_parts ? workspace : nullptr;
     void* msg = want_msg ? (void*)((char*)workspace + pbytes) : nullptr;
     auto kernel = [&](int which, const char* name, int phase) {
-      return kernel_of(plan, 2, {env != nullptr, gl0 != nullptr, gw != nullptr, want_msg, want_parts}, which,
+      return kernel_of(plan, kBwd, {env != nullptr, gl0 != nullptr, gw != nullptr, want_msg, want_parts}, which,
                        [&] { return phase < 0 ? std::string(name) : name + std::to_string(phase); });
     };
     hipStream_t s = (hipStream_t)stream;
@@ -216,7 +248,7 @@ int luna_uvu_conv_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
                              kForwardWaves);
       const size_t wave_lds = split_forward_lds(plan, phase) * (plan.spec.dtype_bits / 8);
       while (split > 1 && split * wave_lds > 65536) split /= 2;
-      hipFunction_t f = kernel_of(plan, split > 1, {env != nullptr, l0 != nullptr}, phase,
+      hipFunction_t f = kernel_of(plan, split > 1 ? kFws : kFwd, {env != nullptr, l0 != nullptr}, phase,
                                   [&] { return "luna_uvu_fwd_p" + std::to_string(phase); });
       void* args[] = {&x, &y, &w, &env, &src, &dst_rowptr, &node_order, &out, &l0};
       if (split > 1) {
@@ -252,6 +284,88 @@ int luna_uvu_conv_bwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
     uvu_conv_bwd(const_cast<LunaUvuPlan*>(cplan)->plan, x, y, w, env, g, gl0, src, dst_rowptr, node_order,
                  src_rowptr, edge_ids_by_src, gx, gy, gw, genv, workspace, workspace_bytes, num_nodes, num_edges,
                  stream);
+  });
+}
+
+int luna_uvu_rows_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, const void* w, int shared_w, void* out,
+                      int64_t rows, LunaStream stream) {
+  return guard_call([&] {
+    if (!cplan) fail("luna_uvu_rows_fwd: null plan");
+    Plan& plan = const_cast<LunaUvuPlan*>(cplan)->plan;
+    check_sizes(plan, rows, rows);
+    if (rows == 0) return;
+    if (!x || !y || !w || !out) fail("luna_uvu_rows_fwd: null tensor");
+    const bool shared = shared_w || plan.spec.w_broadcast;
+    for (int phase = 0; phase < plan.fwd_phases; ++phase) {
+      hipFunction_t f = kernel_of(plan, kRwf, {shared}, phase,
+                                  [&] { return "luna_uvu_rows_fwd_p" + std::to_string(phase); });
+      const int waves = std::max(plan.fwd_block_waves[phase], 1), slots = plan.phase_slots[phase];
+      void* args[] = {&x, &y, &w, &out, &rows};
+      launch("uvu_rows_fwd", f, dim3(row_blocks(plan.fwd_groups, phase, slots, rows), (unsigned)((slots + waves - 1) / waves)),
+             dim3(64 * waves), (hipStream_t)stream, args);
+    }
+  });
+}
+
+int luna_uvu_rows_bwd_workspace(const LunaUvuPlan* plan, int shared_w, int64_t rows, size_t* bytes) {
+  return guard_call([&] {
+    if (!plan || !bytes) fail("luna_uvu_rows_bwd_workspace: null argument");
+    check_sizes(plan->plan, rows, rows);
+    *bytes = part_bytes(plan->plan, rows) + (shared_w ? row_gw_bytes(plan->plan, rows) : 0);
+  });
+}
+
+int luna_uvu_rows_bwd(const LunaUvuPlan* cplan, const void* x, const void* y, const void* w, int shared_w, const void* g,
+                      void* gx, void* gy, void* gw, void* workspace, size_t workspace_bytes, int64_t rows,
+                      LunaStream stream) {
+  return guard_call([&] {
+    if (!cplan) fail("luna_uvu_rows_bwd: null plan");
+    Plan& plan = const_cast<LunaUvuPlan*>(cplan)->plan;
+    check_sizes(plan, rows, rows);
+    if (rows == 0) {
+      if (gw && shared_w) fail("luna_uvu_rows_bwd: the gradient of a shared weight row needs at least one row");
+      return;
+    }
+    if (!x || !y || !w || !g) fail("luna_uvu_rows_bwd: null tensor");
+    if (gw && plan.spec.w_broadcast) fail("luna_uvu_rows_bwd: a broadcast weight row has no gradient");
+    if (!gx && !gy && !gw) return;
+    const bool shared = shared_w || plan.spec.w_broadcast, sum_gw = shared && gw;
+    const size_t pbytes = part_bytes(plan, rows);
+    if ((gy || sum_gw) && (!workspace || workspace_bytes < pbytes + (sum_gw ? row_gw_bytes(plan, rows) : 0)))
+      fail("luna_uvu_rows_bwd: workspace too small");
+    void* part = gy ? workspace : nullptr;
+    void* gw_out = sum_gw ? (void*)((char*)workspace + pbytes) : gw;
+    hipStream_t s = (hipStream_t)stream;
+    auto kernel = [&](int which, const char* name, int phase) {
+      return kernel_of(plan, kRwb, {shared, gw != nullptr, gx != nullptr, gy != nullptr}, which,
+                       [&] { return phase < 0 ? std::string(name) : name + std::to_string(phase); });
+    };
+    if (gx && plan.bwd_gx_needs_zero) {
+      int64_t n = rows * (int64_t)plan.spec.in1;
+      if ((n + 255) / 256 > 0xffffffffLL) fail("luna_uvu_rows_bwd: gx fill exceeds the launch grid");
+      void* args[] = {&gx, &n};
+      launch("uvu_fill", kernel(0, "luna_uvu_fill", -1), dim3((unsigned)((n + 255) / 256)), dim3(256), s, args);
+    }
+    for (int phase = 0; phase < plan.bwd_phases; ++phase) {
+      const int waves = std::max(plan.bwd_block_waves[phase], 1), slots = plan.bwd_phase_slots[phase];
+      // With several launches every workgroup row of the partials is written by all of them.
+      const unsigned blocks = sum_gw ? (unsigned)row_gw_blocks(plan, rows) : row_blocks(plan.bwd_groups, phase, slots, rows);
+      void* args[] = {&x, &y, &w, &g, &gw_out, &gx, &part, &rows};
+      launch("uvu_rows_bwd", kernel(3 + phase, "luna_uvu_rows_bwd_p", phase),
+             dim3(blocks, (unsigned)((slots + waves - 1) / waves)), dim3(64 * waves), s, args);
+    }
+    if (gy) {
+      void* genv = nullptr;
+      void* args[] = {&part, &gy, &genv, &rows};
+      launch("uvu_bwd_reduce", kernel(1, "luna_uvu_bwd_reduce", -1), dim3((unsigned)((rows + 255) / 256)), dim3(256), s,
+             args);
+    }
+    if (sum_gw) {
+      int n = (int)row_gw_blocks(plan, rows);
+      void* args[] = {&gw_out, &gw, &n};
+      launch("uvu_rows_gw", kernel(2, "luna_uvu_rows_gw", -1), dim3((unsigned)((plan.spec.wnum + 31) / 32)), dim3(1024), s,
+             args);
+    }
   });
 }
 

@@ -3,10 +3,11 @@
 A row-wise product (``TensorProduct``, ``src/modules/tensorproduct.py:19-116``;
 the reference's ``LunaTPUVU`` / ``LunaTPUUU``, ``src/lunatp/interface.py:265-307``)
 is the convolution over the identity graph: row b is node b, edge b and the
-destination of edge b, so the HIP convolution kernels compute it with every
-segment holding one edge.  Shared weights ``[weight_numel]`` are broadcast to
-every row.  UVU takes matrices ``[B, dim]``; UUU also broadcasts leading batch
-dimensions of x, y and per-row weights, as the reference does.
+destination of edge b.  UVU runs row kernels of the same plan, which read a
+shared weight row once and sum its gradient; UUU runs the convolution kernels
+with every segment holding one edge and shared weights ``[weight_numel]``
+broadcast to every row.  UVU takes matrices ``[B, dim]``; UUU also broadcasts
+leading batch dimensions of x, y and per-row weights, as the reference does.
 """
 
 from __future__ import annotations
@@ -78,7 +79,12 @@ class LunaTPRows:
             forward = getattr(torch.ops.lunatp, f"{self.mode}_forward").default
             return forward(x.contiguous(), y.contiguous(), weight.contiguous(), self.torch_config)
         rows = x.shape[0]
-        if weight is not None and weight.shape in ((self.weight_numel,), (1, self.weight_numel)):
+        shared = weight is not None and weight.shape in ((self.weight_numel,), (1, self.weight_numel))
+        if self.mode == "uvu":
+            from .uvu_conv import Rows
+
+            return self.conv.run(x, y, weight.reshape(1, -1) if shared else weight, graph=Rows(rows))
+        if shared:
             weight = weight.reshape(1, -1).expand(rows, -1)
         graph = self.identity_graph(rows, x.device)
         return self.conv.run(x, y, weight, graph=graph)

@@ -269,7 +269,7 @@ def create_uvu_conv_operator(tp_or_meta, *, dtype=None):
 _stream = _native.stream_of
 
 
-def _check_device(op, graph, *tensors):
+def _check_tensors(op, *tensors):
     for t in tensors:
         if t is None:
             continue
@@ -277,14 +277,74 @@ def _check_device(op, graph, *tensors):
             raise RuntimeError("convolution kernels run on the GPU; got a CPU tensor")
         if t.dtype is not op.compute_dtype:
             raise TypeError(f"expected {op.compute_dtype}, got {t.dtype}")
+
+
+def _check_device(op, graph, *tensors):
+    _check_tensors(op, *tensors)
     if not graph.src.is_cuda:
         raise RuntimeError("graph tables must live on the GPU; build the graph from GPU tensors")
     if not (graph.src.dtype is graph.dst.dtype is graph.node_order.dtype is graph.source_node_order.dtype is torch.int32):
         raise TypeError("graph node-id tables (src, dst, node_order, source_node_order) must be int32")
 
 
+class Rows:
+    """In the place of a graph: a row-wise product, whose row b is node b, edge b and that
+    edge's source.  The weight is a row per row, or one [1, weight_numel] shared by all."""
+
+    __slots__ = ("num_nodes", "num_edges")
+
+    def __init__(self, rows):
+        self.num_nodes = self.num_edges = rows
+
+
+def _rows_checked(op, x, y, w, graph, *more):
+    """Checks the operands; True for a shared weight row."""
+    _check_tensors(op, x, y, w, *more)
+    rows = graph.num_nodes
+    if x.shape != (rows, op.in1_dim):
+        raise ValueError(f"x must have shape ({rows}, {op.in1_dim}); got {tuple(x.shape)}")
+    shared = w.shape == (1, op.weight_numel)
+    if y.shape != (rows, op.in2_dim) or not (shared or w.shape == (rows, op.weight_numel)):
+        raise ValueError("edge_attr/weight rows must match the rows of x")
+    return shared
+
+
+def run_rows_forward(op, x, y, w, graph):
+    shared = _rows_checked(op, x, y, w, graph)
+    rows, plan = graph.num_nodes, op.plan
+    factory = torch.zeros if plan.info.fwd_needs_zero else torch.empty
+    out = factory((rows, op.out_dim), device=x.device, dtype=x.dtype)
+    _native.check(_native.lib().luna_uvu_rows_fwd(plan.handle, x.data_ptr(), y.data_ptr(), w.data_ptr(), shared,
+                                                  out.data_ptr(), rows, _stream(x)), "luna_uvu_rows_fwd")
+    return out
+
+
+def run_rows_backward(op, x, y, w, graph, g, needs):
+    shared = _rows_checked(op, x, y, w, graph, g)
+    rows, plan = graph.num_nodes, op.plan
+    if needs[2] and op.meta.get("broadcast_weights"):
+        raise ValueError("a broadcast weight row has no per-edge gradient")
+    if g.shape != (rows, op.out_dim):
+        raise ValueError(f"the output gradient must have shape ({rows}, {op.out_dim}); got {tuple(g.shape)}")
+    gx, gy, gw = (torch.empty_like(t) if n else None for t, n in zip((x, y, w), needs))
+    if not rows:
+        return gx, gy, gw if gw is None else gw.zero_(), None
+    size = ctypes.c_size_t()
+    lib = _native.lib()
+    if needs[1] or (needs[2] and shared):
+        _native.check(lib.luna_uvu_rows_bwd_workspace(plan.handle, shared, rows, ctypes.byref(size)),
+                      "luna_uvu_rows_bwd_workspace")
+    workspace = torch.empty((size.value,), device=x.device, dtype=torch.uint8) if size.value else None
+    _native.check(lib.luna_uvu_rows_bwd(plan.handle, x.data_ptr(), y.data_ptr(), w.data_ptr(), shared, g.data_ptr(),
+                                        _native.ptr(gx), _native.ptr(gy), _native.ptr(gw), _native.ptr(workspace),
+                                        size.value, rows, _stream(x)), "luna_uvu_rows_bwd")
+    return gx, gy, gw, None
+
+
 def run_forward(op, x, y, w, graph, env=None, want_l0=False):
     """out [N, out_dim] (and l0 [E, l0_dim]) from the forward kernel."""
+    if isinstance(graph, Rows):
+        return run_rows_forward(op, x, y, w, graph), None
     _check_device(op, graph, x, y, w, env)
     N, E = graph.num_nodes, graph.num_edges
     if x.shape != (N, op.in1_dim):
@@ -309,6 +369,8 @@ def run_forward(op, x, y, w, graph, env=None, want_l0=False):
 
 def run_backward(op, x, y, w, graph, g, env=None, gl0=None, needs=(True, True, True, True)):
     """(gx, gy, gw, genv) from the first-order backward kernels."""
+    if isinstance(graph, Rows):
+        return run_rows_backward(op, x, y, w, graph, g, needs[:3])
     _check_device(op, graph, x, y, w, env, g, gl0)
     N, E = graph.num_nodes, graph.num_edges
     plan = op.plan_for(graph)
@@ -486,6 +548,6 @@ def lunatp_uvu_conv_func(op, x, edge_attr, weight, *, graph: LunaTPGraph, env=No
 # The reference's names for the same autograd nodes.
 UVUConvForward, UVUConvBackward = ConvForward, ConvBackward
 
-__all__ = ["ConvForward", "ConvBackward", "build_uvu_conv_metadata", "l0_feature_layout", "spec_text", "LunaTPUVUConv",
+__all__ = ["ConvForward", "ConvBackward", "build_uvu_conv_metadata", "l0_feature_layout", "spec_text", "LunaTPUVUConv", "Rows",
            "create_uvu_conv_operator", "lunatp_uvu_conv_func", "run_forward", "run_backward",
            "NativePlan"]

@@ -9,10 +9,9 @@ forward and two backward kernels whose contractions over ``(u, v)`` and over
 rows run on ``v_mfma_f32_32x32x2f32``.  Autograd composes higher orders from
 the forward and backward kernels, as for the convolution.
 
-fp64 and per-row weights (``shared_weights=False``) take the UVW convolution
-over the identity graph (row b is node b and edge b): the CG products of each
-row on the HIP UVU kernels, the weight contraction as library GEMMs (on the
-fp64 matrix cores for fp64).
+fp64 and per-row weights (``shared_weights=False``) take the row form of the
+UVW convolution (row b is node b and edge b): the CG products of each row on
+the HIP UVU row kernels, then the contraction with the weights.
 """
 
 from __future__ import annotations
@@ -109,7 +108,6 @@ class LunaTPUVW:
         self.weight_mode = self.meta["weight_mode"]
         self.out_dim = self.meta["out_dim"]
         self._plan = None
-        self._identity = {}
         # fp32 with shared weights: the matrix-core kernels; otherwise the row form
         # of the convolution.
         self.rows_op = None
@@ -141,32 +139,19 @@ class LunaTPUVW:
             return self._run_rows(x, y, weight)
         return lunatp_uvw_func(self, x, y, weight)
 
-    def identity_graph(self, rows, device):
-        """Row b is node b and edge b (cached per size and device)."""
-        key = (rows, str(device))
-        if key not in self._identity:
-            from .graph import make_graph
-
-            ids = torch.arange(rows, device=device)
-            graph = make_graph(ids, ids, rows)
-            graph._tables["identity"] = True
-            self._identity = {key: graph}
-        return self._identity[key]
-
     def _run_rows(self, x, y, weight):
         if weight is None:
             raise TypeError("UVW requires a weight tensor")
         if x.ndim != 2 or y.ndim != 2 or y.shape[0] != x.shape[0]:
             raise ValueError("UVW x and edge_attr must be matrices with the same rows")
+        from .uvu_conv import Rows
         from .uvw_conv import lunatp_uvw_conv_func
 
-        graph = self.identity_graph(x.shape[0], x.device)
-        return lunatp_uvw_conv_func(self.rows_op, x, y, weight, graph=graph)
+        return lunatp_uvw_conv_func(self.rows_op, x, y, weight, graph=Rows(x.shape[0]))
 
     def __getstate__(self):
         state = dict(self.__dict__)
         state["_plan"] = None
-        state["_identity"] = {}
         return state
 
 

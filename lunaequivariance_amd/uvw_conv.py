@@ -40,7 +40,7 @@ from .tracing import recording
 from .cg import sparse_terms
 from .graph import LunaTPGraph, make_graph
 from .layout import TensorProductPaths
-from .uvu_conv import LunaTPUVUConv, ConvForward
+from .uvu_conv import LunaTPUVUConv, ConvForward, Rows
 
 
 # Reductions over fewer rows than this stay one library GEMM.
@@ -394,7 +394,7 @@ def lunatp_uvw_conv_func(op, x, edge_attr, weight=None, *, graph: LunaTPGraph, e
     if op.weight_mode == "shared":
         aggregated = op._aggregate(x, edge_attr, env, graph)
         return op._contract(aggregated, weight, N)
-    if graph._tables.get("identity"):
+    if isinstance(graph, Rows):
         # Every edge is its own destination (the row-wise product): no edge graph, no sum.
         return op._contract(op._aggregate(x, edge_attr, env, graph), weight.contiguous(), E)
     edges = op._edge_graph(graph)
