@@ -195,6 +195,21 @@ GroupUse group_use(const Spec& spec, const Group& g) {
   return use;
 }
 
+// Where one weight row serves every edge, weights and coupling coefficients leave
+// the edge loop: a node's edges only meet in the products P_ij = sum_e x_i y_j
+// (forward), or meet its seeds in Q_ij = sum_paths w sum_k c_ijk G_k (backward:
+// gx messages Q y, gy partials Q^T x), so an edge costs one FMA per product instead of one
+// per coefficient, component and product (lmax 3: forward 686 -> 234 FMAs, backward
+// 1,233 -> 535 with the lane sums).  64 channels, lmax 3, 2,083 nodes, 109,000 edges,
+// where both were bound by those: forward 125 -> 81 us, 69 with the whole next edge
+// in flight; backward 198 -> 134 us, now bound by its x gathers and messages
+// (0.9 GB, 6.7 TB/s from the caches and to memory).  The sums are kept in
+// registers, hence the limit: 120 leave three waves per SIMD (lmax 3 has 112 in
+// fp32; fp64 at lmax 3 would have 224 and keeps the per-edge form).
+bool folds_weights(const Spec& spec, const GroupUse& use) {
+  return spec.w_broadcast && (int)use.products.size() * spec.dtype_bits / 32 <= 120;
+}
+
 // Reduce-scatter of `names` over the 64 lanes: log2(P) halving steps leave
 // every lane with one value index summed over a subset of lanes, then full
 // exchanges finish the sum.  Lane L then holds value index L >> shift, and
@@ -361,11 +376,11 @@ struct YCopies {
 // channels ran half of its lanes idle and its weight rows as 128-byte requests:
 // 1,000 nodes, 52,000 edges, lmax 2, 32 channels, forward 76 -> 31 us (100 MB of
 // weights, 3.4 TB/s), backward 81 -> 64 us (4.2 TB/s).  `split`: the workgroup's
-// waves take the iterations in turn.
+// waves take the iterations in turn.  `weights` off: the body uses none per edge.
 void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& use, bool env,
                     const Options& opt, const std::vector<std::string>& resident,
-                    const std::function<void()>& body, bool split = false) {
-  const int np = (int)g.paths.size();
+                    const std::function<void()>& body, bool split = false, bool weights = true) {
+  const int np = weights ? (int)g.paths.size() : 0;
   const int nsub = 64 / g.cw;
   const bool packed = nsub > 1;
   const bool full = opt.prefetch >= 2;
@@ -730,15 +745,55 @@ void emit_forward_body(Code& c, const Spec& spec, const Group& g, bool env, bool
   if (packed) c.line("      }");
 }
 
+// The group's accumulators A<block>_<k> from the node's product sums (folds_weights).
+void emit_folded_sums(Code& c, const Spec& spec, const Group& g, const GroupUse& use, bool env, const Options& opt,
+                      bool split) {
+  const int bits = spec.dtype_bits;
+  for (const auto& p : use.products) c.line("    real P%d_%d = 0;", p.first, p.second);
+  emit_edge_loop(c, spec, g, use, env, opt, {}, [&] {
+    if (g.cw < 64) c.line("      if (ok) {");
+    std::set<int> is;
+    for (const auto& p : use.products) is.insert(p.first);
+    for (int i : is) c.line(env ? "      const real z%d = ev * x%d;" : "      const real z%d = x%d;", i, i);
+    YCopies ycopy{opt.y_vgpr < 0 ? bits == 32 : opt.y_vgpr != 0, {}};
+    for (const auto& p : use.products) {
+      ycopy.need(c, p.second);
+      c.line("      P%d_%d = FMA(z%d, y%d, P%d_%d);", p.first, p.second, p.first, p.second, p.first, p.second);
+    }
+    if (g.cw < 64) c.line("      }");
+  }, split, false);
+  for (size_t b = 0; b < g.blocks.size(); ++b)
+    for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
+  for (size_t n = 0; n < g.paths.size(); ++n) {
+    const Path& q = spec.paths[g.paths[n]];
+    c.line("    {");
+    c.line("      const real wv = w[%d + uc * %d];", q.w_off, q.w_stride);
+    std::set<int> done;
+    for (const Term& t : q.terms) {
+      const std::string c0 = literal(t.c, bits);
+      if (done.insert(t.k).second)
+        c.line("      real t%d = %s * P%d_%d;", t.k, c0.c_str(), t.i, q.y_off + t.j);
+      else
+        c.line("      t%d = FMA(%s, P%d_%d, t%d);", t.k, c0.c_str(), t.i, q.y_off + t.j, t.k);
+    }
+    for (int k : done) c.line("      A%d_%d = FMA(wv, t%d, A%d_%d);", g.path_block[n], k, k, g.path_block[n], k);
+    c.line("    }");
+  }
+}
+
 void emit_forward_group(Code& c, const Spec& spec, const Group& g, bool env, bool l0, const Options& opt,
                         bool split) {
   GroupUse use = group_use(spec, g);
   const bool packed = g.cw < 64;
   emit_lanes(c, g, g.slot_base, 1);
-  for (size_t b = 0; b < g.blocks.size(); ++b)
-    for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
-  auto body = [&]() { emit_forward_body(c, spec, g, env, l0, opt); };
-  emit_edge_loop(c, spec, g, use, env, opt, {}, body, split);
+  if (!l0 && folds_weights(spec, use)) {
+    emit_folded_sums(c, spec, g, use, env, opt, split);
+  } else {
+    for (size_t b = 0; b < g.blocks.size(); ++b)
+      for (int k = 0; k < g.blocks[b].d3; ++k) c.line("    real A%zu_%d = 0;", b, k);
+    auto body = [&]() { emit_forward_body(c, spec, g, env, l0, opt); };
+    emit_edge_loop(c, spec, g, use, env, opt, {}, body, split);
+  }
   if (packed || split) {
     // The sums of a wave's edges, and of the waves sharing the node, meet in
     // LDS: piece q (wave and edge of the wave) holds its cw * d3 values in the
@@ -876,6 +931,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
       seeds.push_back("G" + std::to_string(b) + "_" + std::to_string(k));
     }
   }
+  const bool fold = rows == Rows::none && !gl0 && !want_gw && folds_weights(spec, use);
   // Some q classes are computed once per node, before the edge loop, within
   // a register budget: classes of two or more terms first (each saves that
   // many instructions per edge), then single-term ones, cheapest first (a
@@ -907,7 +963,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
       }
     }
     const int per_value = bits / 32;
-    int budget = rows != Rows::none ? -1 : opt.hoist_regs >= 0 ? opt.hoist_regs : 36;  // (rows: no node to hoist to)
+    int budget = rows != Rows::none || fold ? -1 : opt.hoist_regs >= 0 ? opt.hoist_regs : 36;
     std::map<std::string, int> left = users;  // classes per seed not yet hoisted
     int extra = 0;                            // registers: hoisted values minus freed seeds
     auto cost = [&](const Candidate& cd) {
@@ -953,6 +1009,33 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     for (const auto& kv : hoisted) resident.push_back(kv.second);
     seeds = resident;
   }
+  if (fold) {
+    std::set<std::pair<int, int>> begun;
+    std::vector<std::string> sums;
+    for (int n = 0; n < np; ++n) {
+      const Path& q = spec.paths[g.paths[n]];
+      c.line("    const real wn%d = w[%d + uc * %d];", n, q.w_off, q.w_stride);
+      for (const SignedClass& cls : path_classes[n]) {
+        std::string expr;
+        for (const auto& kc : cls.coefficients) {
+          const std::string seed = "G" + std::to_string(g.path_block[n]) + "_" + std::to_string(kc.first);
+          expr = expr.empty() ? literal(kc.second, bits) + " * " + seed
+                              : "FMA(" + literal(kc.second, bits) + ", " + seed + ", " + expr + ")";
+        }
+        for (const auto& m : cls.members) {
+          const int yi = q.y_off + m.j;
+          const std::string name = "Q" + std::to_string(m.i) + "_" + std::to_string(yi);
+          if (begun.insert({m.i, yi}).second) {
+            c.line("    real %s = %swn%d * (%s);", name.c_str(), m.sign > 0 ? "" : "-", n, expr.c_str());
+            sums.push_back(name);
+          } else {
+            c.line("    %s = FMA(%swn%d, %s, %s);", name.c_str(), m.sign > 0 ? "" : "-", n, expr.c_str(), name.c_str());
+          }
+        }
+      }
+    }
+    seeds = sums;
+  }
   // Combined subsets: lane c of the first subset's wave adds column c (y
   // index, env last) of both subsets' partials; r0 / r1 are that column's
   // positions in the two subsets' value lists (-1: not there).
@@ -973,7 +1056,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   // Alternates between the iterations of the loop: the half of a shared LDS buffer.
   const std::string parity = packed || rows != Rows::none ? "it & 1" : "(e - beg) & 1";
   auto body = [&]() {
-  if (!opt.hoist && rows == Rows::none) {
+  if (!opt.hoist && rows == Rows::none && !fold) {
     // Opaque to the optimiser: keeps the edge-invariant q_ij inside the loop
     // instead of holding all of them in registers across it.
     for (const auto& name : seeds) c.line("      asm volatile(\"\" : \"+v\"(%s));", name.c_str());
@@ -1031,7 +1114,23 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     c.line("      }");
   };
   if (packed) c.line("      if (ok) {");
-  for (int n = 0; n < np; ++n) {
+  if (fold) {
+    YCopies copies{opt.y_vgpr < 0 ? bits == 32 : opt.y_vgpr != 0, {}};
+    std::set<int> is;
+    for (const auto& p : use.products) {
+      is.insert(p.first);
+      copies.need(c, p.second);
+      c.line("      M%d = FMA(y%d, Q%d_%d, M%d);", p.first, p.second, p.first, p.second, p.first);
+    }
+    for (int i : is) {
+      if (env) c.line("      GE = FMA(x%d, M%d, GE);", i, i);
+      if (env) c.line("      M%d *= ev;", i);
+      c.line(env ? "      const real z%d = ev * x%d;" : "      const real z%d = x%d;", i, i);
+    }
+    for (const auto& p : use.products)
+      c.line("      GY%d = FMA(z%d, Q%d_%d, GY%d);", p.second, p.first, p.first, p.second, p.second);
+  }
+  for (int n = 0; n < np && !fold; ++n) {
     const Path& q = spec.paths[g.paths[n]];
     const int b = g.path_block[n];
     const bool scalar_seed = gl0 && q.l0_col >= 0;
@@ -1234,7 +1333,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
   if (!combine) flush(values);
   };
   if (rows == Rows::none) {
-    emit_edge_loop(c, spec, g, use, env, opt, seeds, body);
+    emit_edge_loop(c, spec, g, use, env, opt, seeds, body, false, !fold);
     return;
   }
   emit_row_loop(c, spec, g, use, rows == Rows::shared, opt.nt_w, true, body);
@@ -1347,7 +1446,7 @@ std::string emit_forward(const Plan& plan, bool env, bool l0, bool split) {
       c.line("  %sif (slot < %d) {", first ? "" : "else ", g.slot_base + g.chunks);
       first = false;
       Options own = opt;
-      if (g.cw < 64 || split) own.prefetch = opt.packed_prefetch;
+      if (g.cw < 64 || split || (!l0 && folds_weights(spec, group_use(spec, g)))) own.prefetch = opt.packed_prefetch;
       emit_forward_group(c, spec, g, env, l0, own, split);
       c.line("  }");
     }
