@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <functional>
 #include <map>
 #include <memory>
 #include <set>
@@ -48,7 +49,6 @@ struct UvwSpec {
   bool vec = true;
   int wide = 2;
   bool wdma = true;
-  int bcy = -1;  // LUNAEQ_AMD_UVW_BCY: gx/gy contraction as (c y) dZ (1) or c (y dZ) (0); -1: by occupancy
   // LUNAEQ_AMD_UVW_GPAD: seed-row padding in the gx/gy staging (1: scalar LDS
   // writes, 2: pairs, 4: 16-byte writes).  With rows 32 d3 + 2 floats apart,
   // the B-operand reads of one half-wave (16 rows x two w) fall in 32
@@ -296,6 +296,26 @@ std::set<int> term_js(const UvwPath& q) {
   return r;
 }
 
+// c<i>_<k> = sum_j c_ijk y_j of the lane's row: the coupling matrix of one path between
+// x_i and output component k.  Formed once per row, it takes one FMA per (i, k)
+// and channel where the terms take two per (i, j, k).
+void emit_coupling(Code& c, const UvwPath& q, const std::function<std::string(int)>& y) {
+  std::set<std::pair<int, int>> begun;
+  for (const auto& t : q.terms) {
+    const std::string name = "c" + std::to_string(t.i) + "_" + std::to_string(t.k);
+    if (begun.insert({t.i, t.k}).second)
+      c.line("        real %s = %s * %s;", name.c_str(), flit(t.c).c_str(), y(t.j).c_str());
+    else
+      c.line("        %s = FMA(%s, %s, %s);", name.c_str(), flit(t.c).c_str(), y(t.j).c_str(), name.c_str());
+  }
+}
+// Distinct (i, k) of a path's terms.
+std::set<std::pair<int, int>> term_iks(const UvwPath& q) {
+  std::set<std::pair<int, int>> r;
+  for (const auto& t : q.terms) r.insert({t.i, t.k});
+  return r;
+}
+
 // s_waitcnt immediate that waits until at most n vector-memory operations of
 // the wave are outstanding (gfx9 encoding: vmcnt bits 3:0 and 15:14; expcnt
 // and lgkmcnt left at their maxima, i.e. not waited for).
@@ -444,6 +464,7 @@ void emit_forward_wide(Code& c, const UvwSpec& s, const Unit& u, int nt) {
 // arguments: inlined, every copy and every LDS read carries the alias scope of
 // its buffer, and the compiler waits before a read only for the copies into
 // that buffer (without the scopes it waits for every copy in flight).
+constexpr int kLateRegisters = 192;
 void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
   const UvwPath& head = s.paths[u.paths[0]];
   const int d3 = head.d3, mul3 = head.mul3, T = dma_tiles(s, u), wq = 8 * T;  // wq: 16-byte pieces per K row
@@ -454,6 +475,15 @@ void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
     c.line("  {");
     c.line("    const real* ys = y + (i64)brow * %d + %d;", s.in2, q.y_off);
     for (int j : js) c.line("    const real y%d = ys[%d];", j, j);
+    emit_coupling(c, q, [](int j) { return "y" + std::to_string(j); });
+    const std::set<std::pair<int, int>> iks = term_iks(q);
+    // Fewer input than output components: contract x with the weights first
+    // (2 l1 + 1 matrix steps instead of 2 l3 + 1) and couple the results, where
+    // both accumulators leave two waves per SIMD without spills.  200,000 rows, 64
+    // channels, lmax 2, forward: 621 us without, 616 / 600 / 560 us with up to 96 /
+    // 128 / 192 registers of accumulators, 547 us with 256 (37 spilled); 100,000 rows,
+    // lmax 1: 110 -> 92 us; 32 channels, lmax 2: 119 -> 115 us.
+    const bool late = d1 < d3 && 16 * T * (d1 + d3) <= kLateRegisters;
     c.line("    const real* xrow = x + (i64)rrow * %d + %d + (lane >> 5) * 4;", s.in1, q.x_off);
     c.line("    const real* wrow = wt + %d + (i64)(lane / %d) * %d + wl;", q.w_off, wq, mul3);
     auto copy = [&](const char* chunk, const char* X, const char* W) {
@@ -486,9 +516,15 @@ void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
           c.line("          const real x%d = q%d.%c;", i, (st * d1 + i) / 4, "xyzw"[(st * d1 + i) % 4]);
         for (int t = 0; t < T; ++t)
           c.line("          const real a%d = %s[(%d + 4 * hk) * %d + %d + col];", t, W, st, 32 * T, 32 * t);
+        if (late) {
+          for (int i : is)
+            for (int t = 0; t < T; ++t) c.line("          xw[%d][%d] = mfma32(a%d, x%d, xw[%d][%d]);", t, i, t, i, t, i);
+          c.line("        }");
+          continue;
+        }
         for (int k = 0; k < d3; ++k) c.line("          real z%d = 0;", k);
-        for (const auto& t : q.terms)
-          c.line("          z%d = FMA(%s, x%d * y%d, z%d);", t.k, flit(t.c).c_str(), t.i, t.j, t.k);
+        for (const auto& ik : iks)
+          c.line("          z%d = FMA(x%d, c%d_%d, z%d);", ik.second, ik.first, ik.first, ik.second, ik.second);
         for (int k = 0; k < d3; ++k)
           for (int t = 0; t < T; ++t) c.line("          acc[%d][%d] = mfma32(a%d, z%d, acc[%d][%d]);", t, k, t, k, t, k);
         c.line("        }");
@@ -496,6 +532,11 @@ void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
       c.line("      }");
     };
     const int ncopy = d1 + T;
+    if (late) {
+      c.line("    floatx16 xw[%d][%d];", T, d1);
+      for (int t = 0; t < T; ++t)
+        for (int i = 0; i < d1; ++i) c.line("    xw[%d][%d] = (floatx16)(0.0f);", t, i);
+    }
     c.line("    {");
     copy("0", "X0", "W0");
     c.line("    }");
@@ -512,6 +553,15 @@ void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
     c.line("      }");
     compute("X1", "W1");
     c.line("    }");
+    // The next path's copies refill these buffers: nothing may move them above this
+    // path's LDS reads (with two chunks the loop is straight-line code, and the
+    // scheduler does not order a copy after earlier reads of its buffer).
+    c.line("    asm volatile(\"\" ::: \"memory\");");
+    c.line("    __builtin_amdgcn_sched_barrier(0);");
+    if (late)
+      for (const auto& ik : iks)
+        for (int t = 0; t < T; ++t)
+          c.line("    acc[%d][%d] += c%d_%d * xw[%d][%d];", t, ik.second, ik.first, ik.second, t, ik.first);
     c.line("  }");
   }
 }
@@ -781,7 +831,6 @@ __device__ __forceinline__ void lds_copy16(const void* src, lvoid* dst) {
       const int estimate = 8 * head.d1 + 4 * d3 + 2 * (int)ycols.size() + 48;
       if (estimate > 128) four = false;
     }
-    const bool cy_form = s.bcy < 0 ? four : s.bcy != 0;
     int stage_d3 = 0, cw = s.bcw;  // w per staged chunk
     bool dma = s.bdma < 0 ? !four : s.bdma != 0;
     for (const Unit& u : units)
@@ -1051,7 +1100,7 @@ __device__ __forceinline__ void lds_copy16(const void* src, lvoid* dst) {
             // (c y) dZ shares the products c y across the four K rows (one
             // VALU op per term and row); c (y dZ) keeps no products live (two
             // ops), for kernels short of registers.
-            if (cy_form) {
+            if (four) {
               c.line("      gxa%d_%d = FMA(%s * y%d_%d, dz%d[%d], gxa%d_%d);", qd, t.i, flit(t.c).c_str(), v, t.j, t.k,
                      r, qd, t.i);
               c.line("      gp%d_%d = FMA(%s * x%d_%d, dz%d[%d], gp%d_%d);", v, t.j, flit(t.c).c_str(), r, t.i, t.k, r,
@@ -1205,6 +1254,7 @@ void emit_bw_dma(Code& c, const UvwSpec& s, int chunk_rows) {
     const int d2 = q.d2;
     const int nch = chunk_rows / s.wrows;
     const std::set<int> is = term_is(q), js = term_js(q);
+    const std::set<std::pair<int, int>> iks = term_iks(q);
     c.line("  if (path == %d) {", p);
     for (int m = 0; m < mt; ++m)
       for (int n = 0; n < nt; ++n) c.line("    floatx16 acc%d_%d = (floatx16)(0.0f);", m, n);
@@ -1258,20 +1308,38 @@ void emit_bw_dma(Code& c, const UvwSpec& s, int chunk_rows) {
         for (int j : js) c.line("        const real y%d_%d = %s[(%d + hk) * %d + %d];", sp, j, Y, 2 * sp, d2, j);
         c.line("        const lreal* xl = %s + (%d + hk) * %d;", X, 2 * sp, px);
         c.line("        const lreal* gl = %s + (%d + hk) * %d;", G, 2 * sp, pg);
-        for (int m = 0; m < mt; ++m) {
-          for (int i : is) c.line("        const real x%d_%d = xl[xu%d + %d];", m, i, m, i);
-          for (int k = 0; k < d3; ++k) c.line("        real z%d_%d = 0;", m, k);
-          for (const auto& t : q.terms)
-            c.line("        z%d_%d = FMA(%s, x%d_%d * y%d_%d, z%d_%d);", m, t.k, flit(t.c).c_str(), m, t.i, sp, t.j, m,
-                   t.k);
-          for (int k = 0; k < d3; ++k) c.line("        z%d_%d = (rok && kok%d) ? z%d_%d : 0.0f;", m, k, m, m, k);
-        }
+        emit_coupling(c, q, [&](int j) { return "y" + std::to_string(sp) + "_" + std::to_string(j); });
+        // The shorter of the two forms: sum_k z_k g_k with z_k = sum_i x_i c_ik, or
+        // sum_i x_i h_i with h_i = sum_k c_ik g_k (2 l1 + 1 < 2 l3 + 1 matrix steps).
+        // Bound by the matrix instructions: at 64 channels, lmax 2, 108 of 140 remain
+        // per pair of rows; 200,000 rows, beside the gx/gy kernel: step 1,998 -> 1,851 us.
+        const bool seeds = d1 < d3;
+        for (int m = 0; m < mt; ++m)
+          for (int i : is)
+            c.line("        const real x%d_%d = %sxl[xu%d + %d]%s;", m, i,
+                   seeds ? ("(rok && kok" + std::to_string(m) + ") ? ").c_str() : "", m, i, seeds ? " : 0.0f" : "");
         for (int n = 0; n < nt; ++n)
           for (int k = 0; k < d3; ++k) c.line("        const real g%d_%d = wok%d ? gl[gw%d + %d] : 0.0f;", n, k, n, n, k);
-        for (int k = 0; k < d3; ++k)
+        auto contract = [&](const char* to, const char* from, int tiles, int width, bool over_i) {
+          for (int m = 0; m < tiles; ++m) {
+            for (int v = 0; v < width; ++v) c.line("        real %s%d_%d = 0;", to, m, v);
+            for (const auto& ik : iks)
+              c.line("        %s%d_%d = FMA(%s%d_%d, c%d_%d, %s%d_%d);", to, m, over_i ? ik.second : ik.first, from, m,
+                     over_i ? ik.first : ik.second, ik.first, ik.second, to, m, over_i ? ik.second : ik.first);
+            for (int v = 0; v < width; ++v)
+              c.line("        %s%d_%d = (rok%s) ? %s%d_%d : 0.0f;", to, m, v,
+                     over_i ? (" && kok" + std::to_string(m)).c_str() : "", to, m, v);
+          }
+        };
+        if (seeds)
+          contract("h", "g", nt, d1, false);
+        else
+          contract("z", "x", mt, d3, true);
+        for (int v = 0; v < std::min(d1, d3); ++v)
           for (int m = 0; m < mt; ++m)
             for (int n = 0; n < nt; ++n)
-              c.line("        acc%d_%d = mfma32(z%d_%d, g%d_%d, acc%d_%d);", m, n, m, k, n, k, m, n);
+              c.line("        acc%d_%d = mfma32(%s%d_%d, %s%d_%d, acc%d_%d);", m, n, seeds ? "x" : "z", m, v,
+                     seeds ? "h" : "g", n, v, m, n);
         c.line("      }");
       }
     };
@@ -1341,6 +1409,7 @@ std::string emit_backward_w(const UvwSpec& s, int chunk_rows) {
     const UvwPath& q = s.paths[p];
     const int K = q.mul1 * q.mul2, mt = ktiles(q), nt = (q.mul3 + 31) / 32, d3 = q.d3;
     const std::set<int> is = term_is(q), js = term_js(q);
+    const std::set<std::pair<int, int>> iks = term_iks(q);
     c.line("  if (path == %d) {", p);
     for (int m = 0; m < mt; ++m)
       for (int n = 0; n < nt; ++n) c.line("    floatx16 acc%d_%d = (floatx16)(0.0f);", m, n);
@@ -1521,7 +1590,6 @@ int luna_uvw_plan_create(const char* spec, const char* cache_dir, LunaUvwPlan** 
     p.spec.wide = wide ? std::atoi(wide) : 2;
     p.spec.wdma = !wdma || std::atoi(wdma) != 0;
     if (const char* wr = std::getenv("LUNAEQ_AMD_UVW_WROWS")) p.spec.wrows = std::atoi(wr) == 4 ? 4 : 2;
-    if (const char* cy = std::getenv("LUNAEQ_AMD_UVW_BCY")) p.spec.bcy = std::atoi(cy);
     if (const char* gp = std::getenv("LUNAEQ_AMD_UVW_GPAD")) {
       const int v = std::atoi(gp);
       p.spec.gpad = v == 1 || v == 4 ? v : 2;
