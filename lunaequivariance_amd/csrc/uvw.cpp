@@ -1094,23 +1094,28 @@ __device__ __forceinline__ void lds_copy16(const void* src, lvoid* dst) {
           for (int k = 0; k < d3; ++k) c.line("        dz%d = mfma16(a, gr[sc * %d + %d], dz%d);", k, d3, k, k);
           c.line("      }");
         }
-        for (int r = 0; r < 4; ++r) {
-          const int v = r % m2, qd = r / m2;
-          for (const auto& t : q.terms) {
-            // (c y) dZ shares the products c y across the four K rows (one
-            // VALU op per term and row); c (y dZ) keeps no products live (two
-            // ops), for kernels short of registers.
-            if (four) {
-              c.line("      gxa%d_%d = FMA(%s * y%d_%d, dz%d[%d], gxa%d_%d);", qd, t.i, flit(t.c).c_str(), v, t.j, t.k,
-                     r, qd, t.i);
-              c.line("      gp%d_%d = FMA(%s * x%d_%d, dz%d[%d], gp%d_%d);", v, t.j, flit(t.c).c_str(), r, t.i, t.k, r,
-                     v, t.j);
-            } else {
-              c.line("      gxa%d_%d = FMA(%s, y%d_%d * dz%d[%d], gxa%d_%d);", qd, t.i, flit(t.c).c_str(), v, t.j, t.k,
-                     r, qd, t.i);
-              c.line("      gp%d_%d = FMA(%s, x%d_%d * dz%d[%d], gp%d_%d);", v, t.j, flit(t.c).c_str(), r, t.i, t.k, r,
-                     v, t.j);
+        // Per (i, k), over the lane's K rows: gx_i += c_ik dZ_k with c_ik = sum_j c_ijk y_j,
+        // and gy_j += c_ijk s_ik with s_ik = sum x_i dZ_k (8 operations a pair and
+        // 2 a term; term by term it was 13 a term, 83 terms on 79 pairs at lmax 2).
+        // 200,000 rows, 64 channels, lmax 2: step 1,918 -> 1,904 us.
+        for (const auto& ik : term_iks(q)) {
+          const int i = ik.first, k = ik.second;
+          for (int v = 0; v < m2; ++v) {
+            std::string coupling;
+            for (const auto& t : q.terms) {
+              if (t.i != i || t.k != k) continue;
+              const std::string yv = "y" + std::to_string(v) + "_" + std::to_string(t.j);
+              coupling = coupling.empty() ? flit(t.c) + " * " + yv : "FMA(" + flit(t.c) + ", " + yv + ", " + coupling + ")";
             }
+            c.line("      {");
+            c.line("        const real cik = %s;", coupling.c_str());
+            for (int r = v; r < 4; r += m2) c.line("        gxa%d_%d = FMA(cik, dz%d[%d], gxa%d_%d);", r / m2, i, k, r, r / m2, i);
+            c.line("        real sik = x%d_%d * dz%d[%d];", v, i, k, v);
+            for (int r = v + m2; r < 4; r += m2) c.line("        sik = FMA(x%d_%d, dz%d[%d], sik);", r, i, k, r);
+            for (const auto& t : q.terms)
+              if (t.i == i && t.k == k)
+                c.line("        gp%d_%d = FMA(%s, sik, gp%d_%d);", v, t.j, flit(t.c).c_str(), v, t.j);
+            c.line("      }");
           }
         }
         // Sum over the four lane groups that share a batch row.
