@@ -1,4 +1,4 @@
-"""UVW tensor-product convolution as aggregation on the HIP UVU kernels plus per-path GEMMs.
+"""UVW tensor-product convolution as aggregation on the HIP UVU kernels plus a contraction.
 
 For a uvw path p (``src/lunatp/uvw_conv/``, e3nn's uvw connection) and an edge
 e = (s -> t):
@@ -25,7 +25,8 @@ destinations are the edges themselves (``Z`` per edge), the per-edge
 contraction is a batched GEMM, and the messages are summed at destinations.
 
 Every piece is differentiable (the UVU autograd classes for the aggregation,
-the contraction's three bilinear maps, torch for the batched GEMM and the sum), so derivatives of every order follow.
+the contraction's three bilinear maps, torch for the batched GEMM and the sum),
+so derivatives of every order follow.
 """
 
 from __future__ import annotations
@@ -202,7 +203,7 @@ class LunaTPUVWConv:
         a_off = w_off = 0
         max_channels = 1
         # Aggregate blocks in output order, so the paths into one output block are
-        # contiguous columns of A and contract in one GEMM.
+        # contiguous columns of A and contract together.
         w_offsets, at = [], 0
         for ins in paths.instructions:
             w_offsets.append(at)
