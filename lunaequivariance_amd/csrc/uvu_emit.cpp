@@ -150,6 +150,10 @@ std::string prelude(const Spec& spec, int edge_index_bits) {
   s << "#define WROW " << (spec.w_broadcast ? "0LL" : "WNUM") << "\n";
   s << "#define L0DIM " << spec.l0_dim << "LL\n";
   s << "#define PART_W " << spec.in2 + 1 << "LL\n";
+  // Edges are compared by distances: with int32 offsets a position past `end`
+  // wraps to a negative one where a graph has almost 2^31 edges.
+  s << "__device__ __forceinline__ eix edge_at(eix from, int ahead, eix end) {"
+       " return end - from > ahead ? from + ahead : end - 1; }\n";
   if (fp64) {
     // A double literal cannot be an instruction operand: it lives in a scalar
     // register pair.  Left alone, the compiler hoists all of a kernel's
@@ -440,29 +444,31 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
 
   if (packed || split) {
     const std::string step = split ? std::to_string(nsub) + " * split" : std::to_string(nsub);
-    const std::string lane_edge = packed ? " + sub" : "";
-    auto clamped = [&](const std::string& edge) {
-      return "(" + edge + lane_edge + " < end ? " + edge + lane_edge + " : end - 1)";
+    const std::string lane_edge = packed ? " + sub" : "", skip = split ? "part * " + std::to_string(nsub) : "0";
+    // The lane's edge `ahead` after `edge` (which lies before the end), or the last one.
+    auto clamped = [&](const std::string& edge, const std::string& ahead) {
+      return "edge_at(" + edge + ", " + ahead + lane_edge + ", end)";
     };
-    c.line("    const eix first = %s;", split ? ("beg + part * " + std::to_string(nsub)).c_str() : "beg");
-    c.line("    if (first < end) {");
+    c.line("    if (end - beg > %s) {", skip.c_str());
+    c.line("    const eix first = beg + %s;", skip.c_str());
     declare('n');
-    c.line("      int sn = src[%s];", clamped("first").c_str());
-    load_edge(clamped("first").c_str(), "sn", 'n');
-    c.line("      sn = src[%s];", clamped("first + " + step).c_str());
+    c.line("      int sn = src[%s];", clamped("first", "0").c_str());
+    load_edge(clamped("first", "0").c_str(), "sn", 'n');
+    c.line("      sn = src[%s];", clamped("first", step).c_str());
     waits('n');
     resident_waits();
     if (packed) c.line("      int it = 0;");
-    c.line("      for (eix e0 = first; e0 < end; e0 += %s%s) {", step.c_str(), packed ? ", ++it" : "");
-    c.line("      const eix e = %s;", clamped("e0").c_str());
-    if (packed) c.line("      const bool ok = e0 + sub < end;");
+    c.line("      for (eix e0 = first;; e0 += %s%s) {", step.c_str(), packed ? ", ++it" : "");
+    c.line("      const eix e = %s;", clamped("e0", "0").c_str());
+    if (packed) c.line("      const bool ok = end - e0 > sub;");
     bind('n');
-    c.line("      const eix en = %s;", clamped("e0 + " + step).c_str());
+    c.line("      const eix en = %s;", clamped("e0", step).c_str());
     load_edge("en", "sn", 'n');
-    c.line("      sn = src[%s];", clamped("e0 + 2 * " + step).c_str());
+    c.line("      sn = src[%s];", clamped("e0", "2 * " + step).c_str());
     if (!full) inline_y();
     body();
     waits('n');
+    c.line("      if (end - e0 <= %s) break;", step.c_str());
     c.line("      }");
     c.line("    }");
     return;
@@ -526,10 +532,10 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
   load_edge("beg", "sn", 'n');
   c.line("      sn = src[beg + 1 < end ? beg + 1 : last];");
   load_edge("(beg + 1 < end ? beg + 1 : last)", "sn", 'm');
-  c.line("      sn = src[beg + 2 < end ? beg + 2 : last];");
+  c.line("      sn = src[edge_at(beg, 2, end)];");
   waits('n');
   resident_waits();
-  c.line("      for (eix e0 = beg; e0 < end; e0 += 2) {");
+  c.line("      for (eix e0 = beg;; e0 += 2) {");
   for (int half = 0; half < 2; ++half) {
     const char cur = half == 0 ? 'n' : 'm', other = half == 0 ? 'm' : 'n';
     if (half == 0)
@@ -539,13 +545,14 @@ void emit_edge_loop(Code& c, const Spec& spec, const Group& g, const GroupUse& u
     c.line("      const eix e = e0 + %d;", half);
     bind(cur);
     // Refill this buffer with edge e+2 and fetch the source index of e+3.
-    c.line("      const eix en = e + 2 < end ? e + 2 : last;");
+    c.line("      const eix en = edge_at(e, 2, end);");
     load_edge("en", "sn", cur);
     c.line("      sn = src[en + 1 < end ? en + 1 : last];");
     body();
     waits(other);
     c.line("      }");
   }
+  c.line("      if (end - e0 <= 2) break;");
   c.line("      }");
   c.line("    }");
 }
@@ -1081,7 +1088,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     if (packed) {
       emit_packed_reduce(c, values, tag.c_str(), g.cw,
                          [&](const char* edge, const char* rank, const char* total, const char* own) {
-        c.line("          if (%s && e0 + %s < end)", own, edge);
+        c.line("          if (%s && end - e0 > %s)", own, edge);
         c.line("            part[((i64)(%d + (slot - %d)) * E + (e0 + %s)) * PART_W + %d + %s] = %s;", g.gy_slot_base,
                g.slot_base, edge, column[values[0]], rank, total);
       });
@@ -1314,7 +1321,7 @@ void emit_backward_wave(Code& c, const Spec& spec, const Group& g, bool env, boo
     c.line("      for (int o = lane; o < %d * (int)PART_W; o += 64) {", nsub);
     c.line("        const int par = it & 1, edge = o / (int)PART_W, col = o %% (int)PART_W;");
     c.line("        const bool a = %s, b = %s;", present(0).c_str(), present(1).c_str());
-    c.line("        if ((a || b) && e0 + edge < end)");
+    c.line("        if ((a || b) && end - e0 > edge)");
     c.line("          part[((i64)(%d + (slot - %d) / 2) * E + (e0 + edge)) * PART_W + col] =", whole->gy_slot_base,
            whole->slot_base);
     c.line("              (a ? gy_sub[0][par][o] : (real)0) + (b ? gy_sub[1][par][o] : (real)0);");
@@ -1531,9 +1538,10 @@ static std::string backward_source(const Plan& plan, bool env, bool gl0, bool wa
     // many runs (nothing is summed over a node's edges here).
     c.line("  eix beg = rowptr[t], end = rowptr[t + 1];");
     c.line("  if (gridDim.z > 1) {");
-    c.line("    const eix run = (end - beg + (eix)gridDim.z - 1) / (eix)gridDim.z;");
-    c.line("    beg += run * (eix)blockIdx.z;");
-    c.line("    end = beg + run < end ? beg + run : end;");
+    c.line("    const eix n = end - beg, layers = (eix)gridDim.z;");
+    c.line("    const eix run = n / layers + (n %% layers != 0), skip = run * (eix)blockIdx.z;");
+    c.line("    beg += skip < n ? skip : n;");
+    c.line("    if (end - beg > run) end = beg + run;");
     c.line("  }");
     }
     bool first = true;
@@ -1735,13 +1743,14 @@ static std::string backward_source(const Plan& plan, bool env, bool gl0, bool wa
   };
   for (int n = 0; n < un; ++n) c.line("  vec_t acc%d = {};", n);
   c.line("  if (covered(col)) {");
-  c.line("    const eix beg = srow[s]%s, end = srow[s + 1];", teams > 1 ? " + team" : "");
-  c.line("    eix p = beg;");
-  c.line("    for (; p + %d < end; p += %d) {", (un - 1) * teams, un * teams);
+  c.line("    const eix beg = srow[s];");
+  c.line("    eix left = srow[s + 1] - beg%s;", teams > 1 ? " - team" : "");
+  c.line("    const eix* p = ebs + (i64)beg%s;", teams > 1 ? " + team" : "");
+  c.line("    for (; left > %d; left -= %d, p += %d) {", (un - 1) * teams, un * teams, un * teams);
   for (int n = 0; n < un; ++n)
-    c.line("      acc%d += %s;", n, load("ebs[p + " + std::to_string(n * teams) + "]").c_str());
+    c.line("      acc%d += %s;", n, load("p[" + std::to_string(n * teams) + "]").c_str());
   c.line("    }");
-  c.line("    for (; p < end; p += %d) acc0 += %s;", teams, load("ebs[p]").c_str());
+  c.line("    for (; left > 0; left -= %d, p += %d) acc0 += %s;", teams, teams, load("*p").c_str());
   c.line("  }");
   // pairwise sum of the partial accumulators
   for (int width = 1; width < un; width *= 2)
