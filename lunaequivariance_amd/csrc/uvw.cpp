@@ -1318,7 +1318,8 @@ void emit_bw_dma(Code& c, const UvwSpec& s, int chunk_rows) {
         // sum_i x_i h_i with h_i = sum_k c_ik g_k (2 l1 + 1 < 2 l3 + 1 matrix steps).
         // Bound by the matrix instructions: at 64 channels, lmax 2, 108 of 140 remain
         // per pair of rows; 200,000 rows, beside the gx/gy kernel: step 1,998 -> 1,851 us.
-        const bool seeds = d1 < d3;
+        // A path of weight 0 has no terms and takes the first form, whose z are then 0.
+        const bool seeds = d1 < d3 && !q.terms.empty();
         for (int m = 0; m < mt; ++m)
           for (int i : is)
             c.line("        const real x%d_%d = %sxl[xu%d + %d]%s;", m, i,
@@ -1340,7 +1341,7 @@ void emit_bw_dma(Code& c, const UvwSpec& s, int chunk_rows) {
           contract("h", "g", nt, d1, false);
         else
           contract("z", "x", mt, d3, true);
-        for (int v = 0; v < std::min(d1, d3); ++v)
+        for (int v = 0; v < (seeds ? d1 : d3); ++v)
           for (int m = 0; m < mt; ++m)
             for (int n = 0; n < nt; ++n)
               c.line("        acc%d_%d = mfma32(%s%d_%d, %s%d_%d, acc%d_%d);", m, n, seeds ? "x" : "z", m, v,

@@ -107,6 +107,24 @@ def test_uvw_plan_compiles_without_gpu(tmp_path, monkeypatch):
     assert per_row.op.rows_op is not None and per_row.op.weight_mode == "external"
 
 
+@pytest.mark.parametrize("in1,in2,out,weights", [
+    ("64x0e", "1x1o", "64x1o", [0.0]),                                   # one path, l1 < l3
+    ("64x0e", "1x1o", "64x1o", [1.0]),
+    ("16x0e+16x1o", "1x0e+1x1o", "16x0e+16x1o+16x2e", [1.0, 0.0, 0.0, 1.0, 0.0]),  # beside weighted paths
+    ("10x0e+6x1o", "2x1o", "9x0e+7x1o+5x2e", [0.0, 0.0, 0.0]),           # unaligned rows, mul2 = 2
+])
+def test_uvw_plan_compiles_with_paths_of_weight_zero(tmp_path, monkeypatch, in1, in2, out, weights):
+    import lunaequivariance_amd as lunaeq
+
+    monkeypatch.setenv("LUNAEQ_AMD_CACHE", str(tmp_path))
+    paths = uvw_instructions(in1, in2, out)
+    assert len(paths) == len(weights)
+    tp = lunaeq.TensorProduct(in1, in2, out, [(*p, w) for p, w in zip(paths, weights)], shared_weights=True,
+                              internal_weights=False)
+    tp.op.plan.precompile()
+    assert len(list(tmp_path.glob("uvw_*.co"))) == 3
+
+
 # Hand-computed uvw normalisation, the formula of the reference's
 # src/lunatp/utils/layout.py:339-367 with fan = mul1 * mul2 for uvw paths.
 # Config 5 ("64x0e+64x1o+64x2e" x "1x0e+1x1o+1x2e" -> same, fully connected,

@@ -303,3 +303,31 @@ def test_uvw_gx_gy_staging_modes(monkeypatch, copied, in1, in2, out, rows):
             assert_close(a, r, torch.float32, f"{'gx' if n == 0 else 'gy'}, copied={copied}")
     finally:
         itf._cached.cache_clear()
+
+
+@pytest.mark.parametrize("in1,in2,out,zero", [
+    ("64x0e", "1x1o", "64x1o", (0,)),                                    # l1 < l3, no path with terms
+    ("16x0e+16x1o", "1x0e+1x1o", "16x0e+16x1o+16x2e", (1, 2, 4)),
+    ("10x0e+6x1o", "2x1o", "9x0e+7x1o+5x2e", (0, 2)),
+])
+def test_uvw_paths_of_weight_zero(in1, in2, out, zero):
+    """Such a path adds nothing and its weights get gradient 0: the oracle with its weights at 0."""
+    instructions = uvw_instructions(in1, in2, out)
+    weighted = [(*p, float(n not in zero)) for n, p in enumerate(instructions)]
+    tp = lunaeq.TensorProduct(in1, in2, out, weighted, shared_weights=True, internal_weights=False)
+    gen = torch.Generator().manual_seed(len(zero))
+    x = torch.randn(70, tp.irreps_in1.dim, generator=gen, dtype=torch.float64)
+    y = torch.randn(70, tp.irreps_in2.dim, generator=gen, dtype=torch.float64)
+    w = torch.randn(tp.weight_numel, generator=gen, dtype=torch.float64) / 8
+    keep = torch.cat([torch.full((tp.irreps_in1[i].mul * tp.irreps_in2[j].mul * tp.irreps_out[k].mul,),
+                                 float(n not in zero), dtype=torch.float64)
+                      for n, (i, j, k, *_) in enumerate(instructions)])
+    ref_in = [t.clone().requires_grad_() for t in (x, y, w)]
+    ref = uvw_tensor_product(in1, in2, out, instructions, ref_in[0], ref_in[1], ref_in[2] * keep)
+    dev_in = [t.to(DEV, torch.float32).requires_grad_() for t in (x, y, w)]
+    act = tp(*dev_in)
+    assert_close(act, ref, torch.float32, "forward")
+    g = torch.randn(ref.shape, generator=gen, dtype=torch.float64)
+    for name, a, r in zip("xyw", torch.autograd.grad(act, dev_in, g.to(DEV, torch.float32)),
+                          torch.autograd.grad(ref, ref_in, g)):
+        assert_close(a, r, torch.float32, "g" + name)
