@@ -470,7 +470,7 @@ struct Builder {
       void* a[] = {&in, &n_in, &out, &n_out, &sums};
       run("scan_tiles", blocks_of(n_out, kTile), a);
     }
-    if (offsets) scan(sums, tiles, offsets, tiles);
+    if (tiles > kFewTiles) scan(sums, tiles, offsets, tiles);
     if (module && (tiles > 1 || last)) {
       void* b[] = {&out, &n_out, &offsets, &sums, &last};
       run("scan_add", blocks_of(n_out, 256), b);
