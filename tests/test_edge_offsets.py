@@ -176,3 +176,100 @@ def test_last_edges_of_a_graph(emitter, tmp_path, bits, edges, channels):
     if done.returncode == 77:
         pytest.skip(done.stdout)
     assert done.returncode == 0 and done.stdout.strip() == "ok", (done.returncode, done.stdout)
+
+
+# ---- the UUU convolution's loops
+
+EMIT_UUU = r"""
+#include <fstream>
+#include "%s/lunaequivariance_amd/csrc/uuu.cpp"
+int main(int argc, char** argv) {
+  LunaUuuPlan* plan = nullptr;
+  if (luna_uuu_plan_create_ex(argv[1], "", std::stoi(argv[2]), &plan)) return 1;
+  const std::string to = argv[3];
+  std::ofstream(to + "/fwd.h") << luna::emit_forward(plan->plan, false, true);
+  std::ofstream(to + "/bwd.h") << luna::emit_backward(plan->plan, false, false, true, true, true, true);
+}
+"""
+
+# Every edge's own results (scalar features; gy, gw and the env-gradient partials) are written by the
+# lane that takes it; sums over lanes are not formed here.
+RUN_UUU = RUN[:RUN.index('#include "plan.h"')] + r"""
+#define __align__(n) __attribute__((aligned(n)))
+namespace fwd {
+#include "fwd.h"
+}
+namespace bwd {
+#include "bwd.h"
+}
+typedef fwd::eix eix;
+typedef float real;
+""" + RUN[RUN.index("// `n` zeros"):RUN.index("int main()")] + r"""
+int main() {
+  const long long E = EDGES;
+  const int C = CHANNELS;
+  int* other = sparse<int>(E);
+  eix* ids = sparse<eix>(E);
+  real *y = sparse<real>(E * C), *w = sparse<real>(E * C), *l0 = sparse<real>(E * C), *gy = sparse<real>(E * C);
+  real *gw = sparse<real>(E * C), *part = sparse<real>(E);
+  static real x[64], g[64], out[64], gx[64];
+  static int order[1];
+  for (int c = 0; c < C; ++c) x[c] = g[c] = 1;
+  for (long long e = E - MOST; e < E; ++e) {
+    ids[e] = (eix)e;
+    for (int c = 0; c < C; ++c) y[e * C + c] = w[e * C + c] = 1;
+  }
+  for (int k = 0; k <= MOST; k += k < 70 ? 1 : 61) {
+    const eix rowptr[2] = {(eix)(E - k), (eix)E};
+    for (int split = 1; split <= 8; split *= 2) {
+      real* const results[] = {l0, gy, gw};
+      for (real* p : results) memset(p + (E - MOST) * C, 0, sizeof(real) * MOST * C);
+      memset(part + (E - MOST), 0, sizeof(real) * MOST);
+      workgroup(64 * split, [&] { fwd::luna_uuu_fwd_g0(x, y, w, nullptr, other, rowptr, order, out, l0, split); });
+      workgroup(64 * split, [&] {
+        bwd::luna_uuu_bwd_g0(x, y, w, nullptr, g, nullptr, other, rowptr, ids, order, gx, gy, gw, part, split, E);
+      });
+      for (long long e = E - MOST; e < E; ++e) {
+        const bool mine = e >= E - k;
+        for (int c = 0; c < C; ++c) EXPECT(l0[e * C + c] == mine && gy[e * C + c] == mine && gw[e * C + c] == mine);
+        EXPECT(part[e] == mine);
+      }
+    }
+  }
+  puts("ok");
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def uuu_emitter(tmp_path_factory):
+    to = tmp_path_factory.mktemp("emit_uuu")
+    (to / "emit.cpp").write_text(EMIT_UUU % ROOT)
+    library = Path(_native.LIBRARY_PATH)
+    subprocess.run([CLANG, "-std=c++17", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{HIP_INCLUDE}", str(to / "emit.cpp"),
+                    str(library), f"-Wl,-rpath,{library.parent}", "-Wl,--unresolved-symbols=ignore-all", "-o",
+                    str(to / "emit")], check=True)
+    return to / "emit"
+
+
+@pytest.mark.parametrize("channels", [1, 3, 33])  # 64 and 16 edges at once, and one
+@pytest.mark.parametrize("bits,edges", [(32, 2 ** 31 - 1), (64, 2 ** 31 + 2 ** 12)])
+def test_last_edges_of_a_graph_uuu(uuu_emitter, tmp_path, bits, edges, channels):
+    spec = (f"LUNAUUU1 32 {channels} {channels} {channels} {channels} 1 {channels}\n"
+            f"0 0 0 0 {channels} 1 1 1 0 1 0 0 0 1.0\n")
+    subprocess.run([str(uuu_emitter), spec, str(bits), str(tmp_path)], check=True)
+    for name in ("fwd", "bwd"):
+        path = tmp_path / f"{name}.h"
+        text = host_source(path.read_text())
+        path.write_text(re.sub(r"extern __shared__ __align__\(16\) unsigned char lds\[\];",
+                               "static __align__(16) unsigned char lds[1 << 20];", text))
+    most = 2 * 64 * 8 + 3  # two rounds of the widest step and a remainder
+    (tmp_path / "run.cpp").write_text(
+        RUN_UUU.replace("EDGES", f"{edges}LL").replace("CHANNELS", str(channels)).replace("MOST", str(most)))
+    # Signed sums wrap, as on the device.
+    subprocess.run([CLANG, "-std=c++17", "-O1", "-w", "-fwrapv", str(tmp_path / "run.cpp"), "-o", str(tmp_path / "run")],
+                   check=True)
+    done = subprocess.run([str(tmp_path / "run")], capture_output=True, text=True)
+    if done.returncode == 77:
+        pytest.skip(done.stdout)
+    assert done.returncode == 0 and done.stdout.strip() == "ok", (done.returncode, done.stdout)
