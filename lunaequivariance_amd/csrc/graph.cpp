@@ -324,8 +324,10 @@ extern "C" __global__ void __launch_bounds__(256) luna_graph_node_keys(const int
   out_key[n] = (u32)(most - (r1 - r0));
   for (int s = seg_rowptr[n], k = 0; s < seg_rowptr[n + 1]; ++s, ++k) {
     nodes[s] = n;
-    begin[s] = r0 + 32 * k;
-    end[s] = min(r0 + 32 * k + 32, r1);
+    // (what is left, not positions: past the last edge they wrap near 2^31 edges)
+    const int b = r0 + 32 * k;
+    begin[s] = b;
+    end[s] = r1 - b > 32 ? b + 32 : r1;
     seg_key[s] = (u32)(most - (r1 - r0));
   }
 }
@@ -383,7 +385,7 @@ extern "C" __global__ void __launch_bounds__(256) luna_graph_segment_counts(cons
   if (n < N) {
     in = dst_rowptr[n + 1] - dst_rowptr[n];
     out = src_rowptr[n + 1] - src_rowptr[n];
-    count[n] = out > 0 ? (out + 31) / 32 : 1;
+    count[n] = out > 0 ? (out - 1) / 32 + 1 : 1;
   }
   for (int m = 32; m >= 1; m >>= 1) {
     in = max(in, __shfl_xor(in, m, 64));

@@ -273,3 +273,55 @@ def test_last_edges_of_a_graph_uuu(uuu_emitter, tmp_path, bits, edges, channels)
     if done.returncode == 77:
         pytest.skip(done.stdout)
     assert done.returncode == 0 and done.stdout.strip() == "ok", (done.returncode, done.stdout)
+
+
+# ---- the graph tables' source segments
+
+RUN_SEGMENTS = r"""
+#include <cstdio>
+struct Dim { unsigned x, y, z; } threadIdx, blockIdx;
+typedef long long i64;
+typedef unsigned u32;
+#define __global__
+#define __launch_bounds__(n)
+#define __shfl_xor(v, m, w) (v)
+#define __hip_atomic_load(p, order, scope) (*(p))
+inline void atomicMax(long long* p, long long v) { if (v > *p) *p = v; }
+inline int max(int a, int b) { return a > b ? a : b; }
+inline int min(int a, int b) { return a < b ? a : b; }
+KERNELS
+int main() {
+  const int E = 2147483646;  // the most edges of the builder
+  for (int degree = 1; degree <= 100; ++degree) {
+    const int rowptr[2] = {E - degree, E};
+    int count, nodes[4], begin[4], end[4];
+    u32 in_key, out_key, seg_key[4];
+    i64 status[8] = {};
+    luna_graph_segment_counts(rowptr, rowptr, 1, &count, status);
+    if (count != (degree + 31) / 32 || status[5] != degree) { printf("count of %d\n", degree); return 1; }
+    const int seg_rowptr[2] = {0, count};
+    luna_graph_node_keys(rowptr, rowptr, seg_rowptr, 1, degree, &in_key, &out_key, nodes, begin, end, seg_key);
+    for (int s = 0; s < count; ++s)
+      if (begin[s] != E - degree + 32 * s || end[s] != (s + 1 < count ? begin[s] + 32 : E)) { printf("segment of %d\n", degree); return 1; }
+  }
+  // One node with every edge.
+  const int hub[2] = {0, E};
+  int count;
+  i64 status[8] = {};
+  luna_graph_segment_counts(hub, hub, 1, &count, status);
+  if (count != E / 32 + 1) { puts("count of the hub"); return 1; }
+  puts("ok");
+}
+"""
+
+
+def test_segments_of_the_last_edges(tmp_path):
+    source = (ROOT / "lunaequivariance_amd" / "csrc" / "graph.cpp").read_text()
+    kernels = "\n".join(
+        re.search(r'extern "C" __global__ void __launch_bounds__\(256\) ' + name + r"\(.*?\n}\n", source, re.S).group(0)
+        for name in ("luna_graph_segment_counts", "luna_graph_node_keys"))
+    (tmp_path / "run.cpp").write_text(RUN_SEGMENTS.replace("KERNELS", kernels))
+    subprocess.run([CLANG, "-std=c++17", "-O1", "-w", "-fwrapv", str(tmp_path / "run.cpp"), "-o", str(tmp_path / "run")],
+                   check=True)
+    done = subprocess.run([str(tmp_path / "run")], capture_output=True, text=True)
+    assert done.returncode == 0 and done.stdout.strip() == "ok", (done.returncode, done.stdout)
