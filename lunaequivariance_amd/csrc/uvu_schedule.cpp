@@ -107,21 +107,19 @@ namespace {
 
 // Channels per chunk.  Up to 32 channels would leave half of a wave's lanes
 // idle or more, so such chunks are a power of two wide and a wave takes several
-// edges at once (at most eight).  `halves`: also cut wider blocks by 32 where
-// that saves more than an eighth of the lanes (65-96 and 129-160 channels).
-int chunk_width(int channels, bool halves) {
-  if (channels <= 32) {
-    int w = 8;
-    while (w < channels) w *= 2;
-    return w;
-  }
-  const int whole = (channels + 63) / 64 * 64, half = (channels + 31) / 32 * 32;
-  return halves && 8 * (whole - half) > whole ? 32 : kWave;
+// edges at once (at most eight).  Wider blocks keep whole waves: 96 channels as
+// three chunks of 32 took 347 us instead of 242 (lmax 2, 40,000 nodes of two
+// edges), 202 instead of 190 us (3,000 nodes of 50).
+int chunk_width(int channels) {
+  if (channels > 32) return kWave;
+  int w = 8;
+  while (w < channels) w *= 2;
+  return w;
 }
 
 // Split the paths sharing one input block into groups whose output blocks fit
 // the accumulator budget.  Paths writing the same output block stay together.
-std::vector<Group> make_groups(const Spec& spec, int budget, bool halves) {
+std::vector<Group> make_groups(const Spec& spec, int budget) {
   std::map<std::tuple<int, int, int>, std::vector<int>> by_input;
   std::vector<std::tuple<int, int, int>> key_order;
   for (int p = 0; p < (int)spec.paths.size(); ++p) {
@@ -163,7 +161,7 @@ std::vector<Group> make_groups(const Spec& spec, int budget, bool halves) {
       g.x_off = std::get<0>(key);
       g.d1 = std::get<1>(key);
       g.channels = std::get<2>(key);
-      g.cw = chunk_width(g.channels, halves);
+      g.cw = chunk_width(g.channels);
       g.chunks = (g.channels + g.cw - 1) / g.cw;
       // Keep the original block order inside the bin.
       for (const auto& b : blocks) {
@@ -254,7 +252,7 @@ void build_schedule(Plan& plan) {
   // have to accumulate their gx messages.
   int acc_regs = kAccumulatorRegisters;
   if (const char* e = std::getenv("LUNAEQ_AMD_FACC")) acc_regs = std::max(8, std::atoi(e));
-  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32), true);
+  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32));
   auto out_ranges = [](const Group& g) {
     std::vector<std::pair<long, long>> r;
     for (const auto& b : g.blocks) r.push_back({b.out_off, b.out_off + (long)g.channels * b.d3});
@@ -347,7 +345,7 @@ void build_schedule(Plan& plan) {
     if (s > 65535) fail("too many channel chunks for one launch");
 
   // ---- backward ----
-  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters, false);
+  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters);
   auto in_ranges = [](const Group& g) {
     return std::vector<std::pair<long, long>>{{g.x_off, g.x_off + (long)g.channels * g.d1}};
   };
@@ -410,8 +408,6 @@ void build_schedule(Plan& plan) {
   int bwd_limit = limit;
   if (const char* e = std::getenv("LUNAEQ_AMD_BWG")) bwd_limit = std::max(0, std::min(16, std::atoi(e)));
   for (int s : plan.bwd_phase_slots) plan.bwd_block_waves.push_back(any_split ? 2 : std::min(s, bwd_limit));
-  // (Blocks of 65-96 channels keep two chunks here: three of 32 would need a
-  // partial slot each, a larger workspace.)
   // A group whose two chunks are the two waves of one workgroup adds their gy
   // partials through LDS and writes one slot (half the partial traffic).
   bool pair = true;

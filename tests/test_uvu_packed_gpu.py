@@ -1,8 +1,7 @@
 """UVU kernels that take several edges per wave (narrow channel blocks) or several waves per node
 (few nodes, many edges each) against the fp64 oracle.
 
-Channel counts stand at the edges of the chunk widths (8, 16, 32, 64, and 32-wide chunks of 65-96
-and 129-160 channels); graphs have a node without edges and row lengths that are no multiple of
+Channel counts stand at the edges of the chunk widths (8, 16, 32, 64) and of two and three chunks; graphs have a node without edges and row lengths that are no multiple of
 the edges taken at once.
 """
 

@@ -1,0 +1,53 @@
+"""Which lanes the UVU kernels give to channels and to edges, read from the built plans (no GPU)."""
+
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from lunaequivariance_amd import _native
+
+ROOT = Path(__file__).resolve().parents[1]
+CLANG = shutil.which("clang++") or "/opt/rocm/llvm/bin/clang++"
+HIP_INCLUDE = Path("/opt/rocm/include")
+
+pytestmark = pytest.mark.skipif(not (Path(CLANG).exists() and HIP_INCLUDE.exists()), reason="needs clang++ and HIP headers")
+
+
+def run(tmp_path, body):
+    (tmp_path / "plan.cpp").write_text(
+        f'#include <cstdio>\n#include "{ROOT}/include/lunaeq_amd.h"\n'
+        f'#include "{ROOT}/lunaequivariance_amd/csrc/uvu_plan.h"\n' + body)
+    library = Path(_native.LIBRARY_PATH)
+    subprocess.run([CLANG, "-std=c++17", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{HIP_INCLUDE}", str(tmp_path / "plan.cpp"),
+                    str(library), f"-Wl,-rpath,{library.parent}", "-Wl,--unresolved-symbols=ignore-all", "-o",
+                    str(tmp_path / "plan")], check=True)
+    return subprocess.run([str(tmp_path / "plan")], capture_output=True, text=True, check=True).stdout.split()
+
+
+PLAN = r"""
+// One scalar path of `channels` channels.
+LunaUvuPlan* plan_of(int channels) {
+  char spec[128];
+  snprintf(spec, sizeof(spec), "LUNAUVU1 32 %d 1 %d %d 1 %d\n0 0 0 0 1 %d 1 1 1 0 1 0 0 0 1.0\n", channels, channels,
+           channels, channels, channels);
+  LunaUvuPlan* plan = nullptr;
+  if (luna_uvu_plan_create(spec, "", &plan)) puts("failed");
+  return plan;
+}
+"""
+
+
+def test_chunk_widths(tmp_path):
+    """Up to 32 channels in chunks of a power of two from 8 on; more in whole waves only."""
+    channels = [1, 8, 9, 16, 17, 32, 33, 64, 65, 80, 96, 129, 160]
+    out = run(tmp_path, PLAN + r"""
+int main() {
+  for (int channels : {%s}) {
+    LunaUvuPlan* plan = plan_of(channels);
+    printf("%%d:%%d:%%d\n", plan->plan.fwd_groups[0].cw, plan->plan.fwd_groups[0].chunks, plan->plan.bwd_groups[0].cw);
+  }
+}""" % ",".join(map(str, channels)))
+    width = [8, 8, 16, 16, 32, 32] + 7 * [64]
+    assert out == [f"{w}:{-(-c // w)}:{w}" for c, w in zip(channels, width)]
