@@ -59,7 +59,7 @@ int luna_uvu_conv_bwd_noalloc(const LunaUvuPlan* cplan, const void* x, const voi
   return luna::guard_call([&] {
     if (!cplan) luna::fail("luna_uvu_conv_bwd_noalloc: null plan");
     if (num_nodes < 0 || num_edges < 0) luna::fail("luna_uvu_conv_bwd_noalloc: negative problem size");
-    luna::Plan& plan = const_cast<LunaUvuPlan*>(cplan)->plan;
+    luna::Plan& plan = const_cast<LunaUvuPlan*>(cplan)->of(num_nodes, num_edges);
     const size_t need = luna::uvu_bwd_workspace_bytes(plan, num_edges);
     if (need > LUNA_UVU_NOALLOC_SCRATCH_BYTES)
       luna::fail("luna_uvu_conv_bwd_noalloc: " + std::to_string(num_edges) + " edges need " +

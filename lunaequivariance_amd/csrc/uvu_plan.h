@@ -89,6 +89,8 @@ struct Plan {
   // Width of the edge-offset graph tables (dst_rowptr, src_rowptr,
   // edge_ids_by_src) the kernels read: 32, or 64 for 2^31 or more edges.
   int edge_index_bits = 32;
+  // Narrow blocks one edge at a time too (see LunaUvuPlan::sparse).
+  bool one_edge = false;
   ModuleCache kernels;  // emitted modules per variant and device
 };
 
@@ -135,4 +137,15 @@ void uvu_conv_bwd(Plan& plan, const void* x, const void* y, const void* w, const
 // The C-ABI's opaque plan handle (include/lunaeq_amd.h).
 struct LunaUvuPlan {
   luna::Plan plan;
+  // For graphs of few edges per node, where a wave that takes several edges of a
+  // node at once finds too few (null where the plan takes one at a time anyway): at
+  // most two per node, three where the plan takes two at once.  Forward + backward
+  // of 40,000 nodes, lmax 2, at 1 / 2 / 3 edges per node, several at once and one:
+  // 8 channels 206 / 224 / 240 and 144 / 196 / 256 us, 16 channels 230 / 254 / 274 and 165 /
+  // 221 / 285 us, 32 channels 282 / 308 / 388 and 217 / 281 / 349 us (20,000 nodes of four:
+  // 213 and 211 us).
+  std::unique_ptr<luna::Plan> sparse;
+  int sparse_degree = 2;
+  bool few(int64_t nodes, int64_t edges) const { return sparse && edges <= sparse_degree * nodes; }
+  luna::Plan& of(int64_t nodes, int64_t edges) { return few(nodes, edges) ? *sparse : plan; }
 };

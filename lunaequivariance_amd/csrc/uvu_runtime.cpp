@@ -197,6 +197,24 @@ int luna_uvu_plan_create_ex(const char* spec, const char* cache_dir, int edge_in
     holder->plan.kernels.cache_dir = cache_dir ? cache_dir : "";
     holder->plan.kernels.tag = "uvu";
     build_schedule(holder->plan);
+    int narrow = 64;
+    for (const auto* groups : {&holder->plan.fwd_groups, &holder->plan.bwd_groups})
+      for (const Group& g : *groups) narrow = std::min(narrow, g.cw);
+    if (narrow < 64) {
+      holder->sparse_degree = narrow == 32 ? 3 : 2;
+      holder->sparse = std::make_unique<Plan>();
+      Plan& one = *holder->sparse;
+      one.edge_index_bits = edge_index_bits;
+      one.spec = holder->plan.spec;
+      one.kernels.cache_dir = holder->plan.kernels.cache_dir;
+      one.kernels.tag = "uvu";
+      one.one_edge = true;
+      build_schedule(one);
+      // One workspace size and one plan info hold for both.
+      if (one.gy_parts != holder->plan.gy_parts || one.fwd_needs_zero != holder->plan.fwd_needs_zero ||
+          one.bwd_gx_needs_zero != holder->plan.bwd_gx_needs_zero)
+        holder->sparse.reset();
+    }
     *out = holder.release();
   });
 }
@@ -237,7 +255,7 @@ int luna_uvu_conv_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
                       int64_t num_edges, LunaStream stream) {
   return guard_call([&] {
     if (!cplan) fail("luna_uvu_conv_fwd: null plan");
-    Plan& plan = const_cast<LunaUvuPlan*>(cplan)->plan;
+    Plan& plan = const_cast<LunaUvuPlan*>(cplan)->of(num_nodes, num_edges);
     check_sizes(plan, num_nodes, num_edges);
     if (num_nodes == 0) return;
     if (!x || !out || !dst_rowptr || !node_order) fail("luna_uvu_conv_fwd: null tensor");
@@ -281,9 +299,9 @@ int luna_uvu_conv_bwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
                       LunaStream stream) {
   return guard_call([&] {
     if (!cplan) fail("luna_uvu_conv_bwd: null plan");
-    uvu_conv_bwd(const_cast<LunaUvuPlan*>(cplan)->plan, x, y, w, env, g, gl0, src, dst_rowptr, node_order,
-                 src_rowptr, edge_ids_by_src, gx, gy, gw, genv, workspace, workspace_bytes, num_nodes, num_edges,
-                 stream);
+    uvu_conv_bwd(const_cast<LunaUvuPlan*>(cplan)->of(num_nodes, num_edges), x, y, w, env, g, gl0, src, dst_rowptr,
+                 node_order, src_rowptr, edge_ids_by_src, gx, gy, gw, genv, workspace, workspace_bytes, num_nodes,
+                 num_edges, stream);
   });
 }
 

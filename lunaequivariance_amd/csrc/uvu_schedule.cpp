@@ -110,8 +110,8 @@ namespace {
 // edges at once (at most eight).  Wider blocks keep whole waves: 96 channels as
 // three chunks of 32 took 347 us instead of 242 (lmax 2, 40,000 nodes of two
 // edges), 202 instead of 190 us (3,000 nodes of 50).
-int chunk_width(int channels) {
-  if (channels > 32) return kWave;
+int chunk_width(int channels, bool one_edge) {
+  if (channels > 32 || one_edge) return kWave;
   int w = 8;
   while (w < channels) w *= 2;
   return w;
@@ -119,7 +119,7 @@ int chunk_width(int channels) {
 
 // Split the paths sharing one input block into groups whose output blocks fit
 // the accumulator budget.  Paths writing the same output block stay together.
-std::vector<Group> make_groups(const Spec& spec, int budget) {
+std::vector<Group> make_groups(const Spec& spec, int budget, bool one_edge) {
   std::map<std::tuple<int, int, int>, std::vector<int>> by_input;
   std::vector<std::tuple<int, int, int>> key_order;
   for (int p = 0; p < (int)spec.paths.size(); ++p) {
@@ -161,7 +161,7 @@ std::vector<Group> make_groups(const Spec& spec, int budget) {
       g.x_off = std::get<0>(key);
       g.d1 = std::get<1>(key);
       g.channels = std::get<2>(key);
-      g.cw = chunk_width(g.channels);
+      g.cw = chunk_width(g.channels, one_edge);
       g.chunks = (g.channels + g.cw - 1) / g.cw;
       // Keep the original block order inside the bin.
       for (const auto& b : blocks) {
@@ -239,7 +239,7 @@ int gather_columns(const Plan& plan) {
 }
 int gather_teams(const Plan& plan) {
   const int row = (plan.spec.in1 + plan.gather_vec - 1) / plan.gather_vec;
-  return row > 128 ? 1 : std::min(16, 256 / gather_columns(plan));
+  return row > 128 || plan.one_edge ? 1 : std::min(16, 256 / gather_columns(plan));
 }
 
 void build_schedule(Plan& plan) {
@@ -252,7 +252,7 @@ void build_schedule(Plan& plan) {
   // have to accumulate their gx messages.
   int acc_regs = kAccumulatorRegisters;
   if (const char* e = std::getenv("LUNAEQ_AMD_FACC")) acc_regs = std::max(8, std::atoi(e));
-  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32));
+  plan.fwd_groups = make_groups(spec, acc_regs / (spec.dtype_bits / 32), plan.one_edge);
   auto out_ranges = [](const Group& g) {
     std::vector<std::pair<long, long>> r;
     for (const auto& b : g.blocks) r.push_back({b.out_off, b.out_off + (long)g.channels * b.d3});
@@ -345,7 +345,7 @@ void build_schedule(Plan& plan) {
     if (s > 65535) fail("too many channel chunks for one launch");
 
   // ---- backward ----
-  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters);
+  plan.bwd_groups = make_groups(spec, kAccumulatorRegisters, plan.one_edge);
   auto in_ranges = [](const Group& g) {
     return std::vector<std::pair<long, long>>{{g.x_off, g.x_off + (long)g.channels * g.d1}};
   };

@@ -1,8 +1,8 @@
 """UVU kernels that take several edges per wave (narrow channel blocks) or several waves per node
 (few nodes, many edges each) against the fp64 oracle.
 
-Channel counts stand at the edges of the chunk widths (8, 16, 32, 64) and of two and three chunks; graphs have a node without edges and row lengths that are no multiple of
-the edges taken at once.
+Channel counts stand at the edges of the chunk widths (8, 16, 32, 64) and of two and three chunks;
+graphs have a node without edges and row lengths that are no multiple of the edges taken at once.
 """
 
 import pytest
@@ -36,6 +36,21 @@ def test_options_and_higher_orders(channels, nodes, edges, dtype):
     instructions = all_uvu_instructions(in1, sh, out)
     conv = make_conv(in1, sh, out, instructions, dtype)
     src, dst = random_graph(nodes, edges, gen)
+    x, y, w = inputs(conv, nodes, edges, dtype, gen)
+    env = torch.rand(edges, generator=gen, dtype=torch.float64)
+    check_orders(conv, in1, sh, out, instructions, x, y, w, src, dst, nodes, dtype, gen, env=env, l0=True, orders=2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("channels,degree", [(8, 2), (12, 2), (32, 3)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_both_sides_of_few_edges_per_node(channels, degree, more, dtype):
+    """The most edges that are taken one at a time, and one more."""
+    nodes, gen = 30, torch.Generator().manual_seed(channels + more)
+    edges = degree * nodes + more
+    in1, sh, out, instructions = mace_irreps(channels, 2)
+    conv = make_conv(in1, sh, out, instructions, dtype)
+    src, dst = random_graph(nodes - 1, edges, gen)
     x, y, w = inputs(conv, nodes, edges, dtype, gen)
     env = torch.rand(edges, generator=gen, dtype=torch.float64)
     check_orders(conv, in1, sh, out, instructions, x, y, w, src, dst, nodes, dtype, gen, env=env, l0=True, orders=2)

@@ -51,3 +51,20 @@ int main() {
 }""" % ",".join(map(str, channels)))
     width = [8, 8, 16, 16, 32, 32] + 7 * [64]
     assert out == [f"{w}:{-(-c // w)}:{w}" for c, w in zip(channels, width)]
+
+
+def test_few_edges_per_node_are_taken_one_at_a_time(tmp_path):
+    """Up to two per node, three where the plan takes two at once; the workspace is the same."""
+    out = run(tmp_path, PLAN + r"""
+int main() {
+  for (int channels : {8, 12, 16, 17, 32, 33}) {
+    LunaUvuPlan* plan = plan_of(channels);
+    int most = 0;
+    while (most < 8 && plan->few(1000, 1000 * (most + 1))) ++most;
+    const bool exact = !plan->sparse || !plan->few(1000, 1000 * most + 1);
+    const bool same = !plan->sparse || (luna::uvu_bwd_workspace_bytes(*plan->sparse, 999) == luna::uvu_bwd_workspace_bytes(plan->plan, 999) &&
+                                        plan->sparse->fwd_groups[0].cw == 64 && plan->sparse->bwd_groups[0].cw == 64);
+    printf("%d:%d:%d:%d\n", channels, most, exact, same);
+  }
+}""")
+    assert out == ["8:2:1:1", "12:2:1:1", "16:2:1:1", "17:3:1:1", "32:3:1:1", "33:0:1:1"]
