@@ -78,26 +78,27 @@ int edge_split(const std::vector<Group>& groups, int phase, int64_t waves, int64
 constexpr int64_t kForwardWaves = 4096, kBackwardWaves = 8192;
 
 // Workgroups along the rows of a row-wise product: every wave loops over rows,
-// which keeps the next row's operands in flight and a shared weight row (and its
-// gradient) in registers.  64 channels, lmax 2, 50,000 rows, forward + backward +
-// weight sum: 2,048 waves 168 + 167 + 7 us, 4,096 156 + 198 + 8, 8,192 157 + 183 +
-// 13, 16,384 153 + 177 + 20, 40,000 150 + 175 + 40; fp64 uvw rows 313, 306, 301,
-// 300 and 302 us a step.  (Through the convolution kernels, with the weight row
-// expanded, per-row weight gradients summed by a library reduction and gx
-// messages gathered: 179 + 240 + 67 + 53 us and the expansion, step 557 us.)
-constexpr int64_t kRowWaves = 8192;
-unsigned row_blocks(const std::vector<Group>& groups, int phase, int slots, int64_t rows) {
+// with the next row's operands in flight, a shared weight row in registers and,
+// in its gradient's kernel (`sum_gw`), the sums over the wave's rows too.  That
+// one keeps to 8,192 waves, each of which writes a partial row: 64 channels,
+// lmax 2, 50,000 rows, shared weights, forward + backward 341 us, 356 with
+// 32,768 waves, 475 with a wave per row.  The others take a wave per row up to 2^20
+// (forward 128 us with 8,192 waves, 121 so; a weight row per row: forward 170 and
+// 149 us, forward + backward 409 and 388 us).
+constexpr int64_t kGradientWaves = 8192, kRowWaves = 1 << 20;
+unsigned row_blocks(const std::vector<Group>& groups, int phase, int slots, int64_t rows, bool sum_gw) {
   int at_once = 64;
   for (const Group& g : groups)
     if (g.phase == phase) at_once = std::min(at_once, 64 / g.cw);
-  return (unsigned)std::max<int64_t>(1, std::min((rows + at_once - 1) / at_once, kRowWaves / std::max(slots, 1)));
+  const int64_t waves = sum_gw ? kGradientWaves : kRowWaves;
+  return (unsigned)std::max<int64_t>(1, std::min((rows + at_once - 1) / at_once, waves / std::max(slots, 1)));
 }
 // Partials of the shared weight row's gradient: a row per workgroup of the
 // largest launch (zeros where a launch has no rows left).
 int64_t row_gw_blocks(const Plan& p, int64_t rows) {
   unsigned n = 1;
   for (int phase = 0; phase < p.bwd_phases; ++phase)
-    n = std::max(n, row_blocks(p.bwd_groups, phase, p.bwd_phase_slots[phase], rows));
+    n = std::max(n, row_blocks(p.bwd_groups, phase, p.bwd_phase_slots[phase], rows, true));
   return n;
 }
 size_t row_gw_bytes(const Plan& p, int64_t rows) {
@@ -319,7 +320,7 @@ int luna_uvu_rows_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
                                   [&] { return "luna_uvu_rows_fwd_p" + std::to_string(phase); });
       const int waves = std::max(plan.fwd_block_waves[phase], 1), slots = plan.phase_slots[phase];
       void* args[] = {&x, &y, &w, &out, &rows};
-      launch("uvu_rows_fwd", f, dim3(row_blocks(plan.fwd_groups, phase, slots, rows), (unsigned)((slots + waves - 1) / waves)),
+      launch("uvu_rows_fwd", f, dim3(row_blocks(plan.fwd_groups, phase, slots, rows, false), (unsigned)((slots + waves - 1) / waves)),
              dim3(64 * waves), (hipStream_t)stream, args);
     }
   });
@@ -367,7 +368,7 @@ int luna_uvu_rows_bwd(const LunaUvuPlan* cplan, const void* x, const void* y, co
     for (int phase = 0; phase < plan.bwd_phases; ++phase) {
       const int waves = std::max(plan.bwd_block_waves[phase], 1), slots = plan.bwd_phase_slots[phase];
       // With several launches every workgroup row of the partials is written by all of them.
-      const unsigned blocks = sum_gw ? (unsigned)row_gw_blocks(plan, rows) : row_blocks(plan.bwd_groups, phase, slots, rows);
+      const unsigned blocks = sum_gw ? (unsigned)row_gw_blocks(plan, rows) : row_blocks(plan.bwd_groups, phase, slots, rows, false);
       void* args[] = {&x, &y, &w, &g, &gw_out, &gx, &part, &rows};
       launch("uvu_rows_bwd", kernel(3 + phase, "luna_uvu_rows_bwd_p", phase),
              dim3(blocks, (unsigned)((slots + waves - 1) / waves)), dim3(64 * waves), s, args);

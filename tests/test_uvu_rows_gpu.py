@@ -74,3 +74,23 @@ def test_rows_copies_aliases_and_holes(shared):
 @pytest.mark.parametrize("needs", [(True, False, False), (False, True, False), (False, False, True), (True, False, True)])
 def test_rows_subsets_of_gradients(needs):
     check(*full(16, 1), 19, True, torch.float32, needs)
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_more_rows_than_waves(shared):
+    """Past 2^20 waves (two chunks of channels: 2^19 rows) the first workgroups take another row."""
+    rows, channels = (1 << 19) + 3, 65
+    tp = lunaeq.TensorProduct(f"{channels}x0e", "1x0e", f"{channels}x0e", [(0, 0, 0, "uvu", True)], shared_weights=shared,
+                              internal_weights=False)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x, g = (torch.randn(rows, channels, device=DEV, generator=gen) for _ in range(2))
+    y = torch.randn(rows, 1, device=DEV, generator=gen)
+    w = torch.randn(*((channels,) if shared else (rows, channels)), device=DEV, generator=gen)
+    ins = [t.requires_grad_() for t in (x, y, w)]
+    grads = torch.autograd.grad(tp(*ins), ins, g)
+    out = tp(x, y, w)
+    X, Y, W, G = (t.detach().double() for t in (x, y, w, g))
+    gw = G * X * Y
+    for name, a, r in (("out", out, X * Y * W), ("gx", grads[0], G * Y * W), ("gy", grads[1], (G * X * W).sum(1, keepdim=True)),
+                       ("gw", grads[2], gw.sum(0) if shared else gw)):
+        assert_close(a, r, torch.float32, name)
