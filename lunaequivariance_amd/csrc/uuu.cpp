@@ -594,13 +594,17 @@ std::string emit_forward(const UuuPlan& plan, bool env, bool l0) {
 
 // Backward groups held to three waves per SIMD (168 registers).  Left alone, the
 // compiler hoists every load of the lmax-3 group and takes 251 registers, two
-// waves: 64 channels, 2,083 nodes, 109,000 edges, step 769 us, at three waves
-// with 8 registers spilled 686 us.  Blocks wider than 7 components spill 46 to
+// waves: 64 channels, 2,083 nodes, 109,000 edges, step 804 us, at three waves
+// with 8 registers spilled 677 us; 10,000 nodes, 300,000 edges 2,101 and 1,897
+// us; 192 channels 2,272 and 2,010 us.  Only where every lane of every chunk has a
+// channel: with 8-32 channels (two to eight edges of a wave at once) the step took 10 to
+// 20 % longer, with 40, 80 and 96 up to 5, 3 and 9 %, with 128 between 7 %
+// less and 2 % more.  Blocks wider than 7 components spill 46 to
 // 240 registers at three waves, fp64 groups up to 31: left as they are, like the
 // groups whose estimate says that they fit by themselves (lmax 2: 56, 95
 // registers, which the hint would raise to 124).
 bool three_waves(const USpec& s, const UGroup& g) {
-  bool narrow = s.bits == 32 && cost(s, g.paths, true) > 80;
+  bool narrow = s.bits == 32 && g.ch % 64 == 0 && cost(s, g.paths, true) > 80;
   for (int b : g.xbs) narrow = narrow && s.xblocks[b].d <= 7;
   for (int b : g.ybs) narrow = narrow && s.yblocks[b].d <= 7;
   for (int b : g.obs) narrow = narrow && s.oblocks[b].d <= 7;

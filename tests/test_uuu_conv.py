@@ -302,3 +302,20 @@ def test_wide_edge_offset_plans_compile(tmp_path, monkeypatch):
     handle = ctypes.c_void_p()
     assert lib.luna_uvu_plan_create_ex(uvu.op.spec.encode(), None, 48, ctypes.byref(handle)) != 0
     assert b"edge_index_bits" in lib.luna_last_error()
+
+
+@pytest.mark.parametrize("channels,held", [(16, False), (64, True), (96, False)])
+def test_backward_registers_are_held_for_whole_chunks_only(tmp_path, monkeypatch, channels, held):
+    """lmax 3: the hint to three waves per SIMD needs a channel on every lane of every chunk."""
+    from lunaequivariance_amd import TensorProductConfig, _native
+    from lunaequivariance_amd.uuu_conv import NativeUuuPlan, build_uuu_conv_metadata, spec_text
+
+    if not _native.library_available():
+        pytest.skip("library not built")
+    monkeypatch.setenv("LUNAEQ_AMD_CACHE", str(tmp_path))
+    monkeypatch.setenv("LUNAEQ_AMD_DUMP", str(tmp_path))
+    ir = "+".join(f"{channels}x{l}{'eo'[l % 2]}" for l in range(4))
+    tp = TensorProductConfig(ir, ir, ir, uuu_paths(ir, ir, ir), internal_weights=False, shared_weights=False)
+    NativeUuuPlan(spec_text(build_uuu_conv_metadata(tp, torch.float32), torch.float32)).precompile()
+    backward = [p.read_text() for p in tmp_path.glob("uuu_bwd*.hip")]
+    assert backward and all(("amdgpu_waves_per_eu(3)" in text) == held for text in backward)
