@@ -173,9 +173,14 @@ constexpr int FR = 32 / T;  // fragments per 32 rows of a wave's tile
 // consecutive columns in consecutive banks.  When the whole K fits one chunk
 // the staged rows serve every tile of m.  With LIN the weight rows of a chunk
 // (forward) or tile (SWAP) are consecutive, so their addresses need one scalar
-// table entry; offsets are formed once, since fp32 matrix and vector
-// instructions of a SIMD do not overlap.  Rows past N and m past MN repeat the
-// last one: they only reach results that are not stored.
+// table entry; otherwise the entry of each weight row is a scalar load too, as
+// RUN consecutive lanes share a row (read per lane, before every weight load, they
+// took longer than the products: 20,000 rows, lmax 3, forward 80 channels 1,767 -> 702
+// us, gA and gW 96 channels 3,895 -> 1,466 us).  Offsets are formed once, since fp32
+// matrix and vector instructions of a SIMD do not overlap.  Rows past N and m past
+// MN repeat the last one: they only reach results that are not stored.  K past KN is
+// cleared; the last chunk's loads are skipped (forward, 66 against 107 us at 112
+// channels, lmax 1) or repeat another value (SWAP).
 template <int D, int KN, int MN, int TM, int KC, bool SWAP, bool LIN>
 __device__ __forceinline__ void product_tiles(const real* __restrict__ in, int ldi, const real* __restrict__ wt,
                                               const int* __restrict__ rows, real* __restrict__ out, int ldo, i64 n0,
@@ -184,15 +189,16 @@ __device__ __forceinline__ void product_tiles(const real* __restrict__ in, int l
   constexpr int LDI = (KC + 1) * D, LDW = TM + 1, LDO = (TM + 1) * D;
   constexpr int IN_PT = (NB * KC * D + 255) / 256, W_PT = KC * TM / 256;
   constexpr int CHUNKS = (KN + KC - 1) / KC;
+  constexpr int RUN = SWAP ? KC : TM, ROWS = SWAP ? MN : KN;  // lanes in a row on one weight row; weight rows
   real* const ins = lds;
   real* const ws = lds + NB * LDI;  // and, after the products, the results
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave % (TM / 32), wn = wave / (TM / 32);
   const int hi = lane / T, lo = lane % T;
   const int left = N - n0 < NB ? (int)(N - n0) : NB;
   in += n0 * ldi;
   out += n0 * ldo;
-  int oi[IN_PT], ow[W_PT];
+  int oi[IN_PT];
   #pragma unroll
   for (int i = 0; i < IN_PT; ++i) {
     const int idx = i * 256 + t, n = idx / (KC * D), e = idx % (KC * D);
@@ -202,8 +208,13 @@ __device__ __forceinline__ void product_tiles(const real* __restrict__ in, int l
   auto fetch_in = [&](int c) {
     #pragma unroll
     for (int i = 0; i < IN_PT; ++i) {
+      const int e = (i * 256 + t) % (KC * D);
+      const bool ok = KN % KC == 0 || c * KC * D + e < KN * D;
       rin[i] = 0;
-      if (KN % KC == 0 || c * KC * D + (i * 256 + t) % (KC * D) < KN * D) rin[i] = in[oi[i] + c * KC * D];
+      if (SWAP)
+        rin[i] = in[oi[i] + (ok ? c * KC * D : -e)];
+      else if (ok)
+        rin[i] = in[oi[i] + c * KC * D];
     }
   };
   auto fetch_w = [&](int mt, int c) {
@@ -214,12 +225,19 @@ __device__ __forceinline__ void product_tiles(const real* __restrict__ in, int l
       const int idx = i * 256 + t;
       const int kk = SWAP ? idx % KC : idx / TM, m = SWAP ? idx / KC : idx % TM;
       const int mc = MN % TM == 0 || m0 + m < MN ? m : MN - 1 - m0;
+      const int kc = KN % KC == 0 || c0 + kk < KN ? kk : KN - 1 - c0;
       rw[i] = 0;
-      if (KN % KC == 0 || c0 + kk < KN) {
-        if (LIN)
-          rw[i] = SWAP ? base[mc * KN + kk] : base[kk * MN + mc];
-        else
-          rw[i] = SWAP ? wt[rows[m0 + mc] + c0 + kk] : wt[rows[c0 + kk] + m0 + mc];
+      if (!SWAP && kc != kk) continue;
+      if (LIN) {
+        rw[i] = SWAP ? base[mc * KN + kc] : base[kc * MN + mc];
+      } else {
+        const int first = (SWAP ? m0 : c0) + i * (256 / RUN) + wave * (64 / RUN);
+        int row = rows[first < ROWS ? first : ROWS - 1];
+        if (RUN < 64) {
+          const int other = rows[first + 1 < ROWS ? first + 1 : ROWS - 1];
+          row = lane < RUN ? row : other;
+        }
+        rw[i] = wt[row + (SWAP ? c0 + kc : m0 + mc)];
       }
     }
   };
@@ -236,14 +254,14 @@ __device__ __forceinline__ void product_tiles(const real* __restrict__ in, int l
         #pragma unroll
         for (int i = 0; i < IN_PT; ++i) {
           const int idx = i * 256 + t, n = idx / (KC * D), e = idx % (KC * D);
-          if (n < NB) ins[n * LDI + e] = rin[i];
+          if (n < NB) ins[n * LDI + e] = !SWAP || KN % KC == 0 || c * KC * D + e < KN * D ? rin[i] : (real)0;
         }
       }
       #pragma unroll
       for (int i = 0; i < W_PT; ++i) {
         const int idx = i * 256 + t;
         const int kk = SWAP ? idx % KC : idx / TM, m = SWAP ? idx / KC : idx % TM;
-        ws[kk * LDW + m] = rw[i];
+        ws[kk * LDW + m] = !SWAP || KN % KC == 0 || c * KC + kk < KN ? rw[i] : (real)0;
       }
       __syncthreads();
       if (c + 1 < CHUNKS) {
@@ -291,19 +309,59 @@ __device__ __forceinline__ void grad_tile(const real* __restrict__ a, i64 lda, c
   const int wc = wave % (TC / 32), ww = wave / (TC / 32);
   const int hi = lane / T, lo = lane % T;
   const int wide_a = (C - c0 < TC ? C - c0 : TC) * D, wide_g = (MN - w0 < TW ? MN - w0 : TW) * D;
+  // Whole fp32 tiles test each value's bounds.  Where channels remain, and in fp64,
+  // that cost up to a fifth (20,000 rows, lmax 3, gA and gW: 80 channels 1,222 -> 1,082
+  // us, 160 channels 3,506 -> 3,013 us; 64 channels 428 us, 461 without the tests): there
+  // offsets within a step are formed once, channels past the last repeat it (their
+  // results are not stored), rows past the last repeat it and are cleared.
+  constexpr bool TESTED = BITS == 32 && C % TC == 0 && MN % TW == 0;
+  int oa[A_PT], og[G_PT];
+  #pragma unroll
+  for (int i = 0; i < A_PT; ++i) {
+    const int r = (i * 256 + t) / RA, e = (i * 256 + t) % RA;
+    oa[i] = (r < NS ? r : NS - 1) * (int)lda + c0 * D + (e < wide_a ? e : wide_a - 1);
+  }
+  #pragma unroll
+  for (int i = 0; i < G_PT; ++i) {
+    const int r = (i * 256 + t) / RG, e = (i * 256 + t) % RG;
+    og[i] = (r < NS ? r : NS - 1) * (int)ldg + w0 * D + (e < wide_g ? e : wide_g - 1);
+  }
   real ra[A_PT], rg[G_PT];
   auto fetch = [&](i64 n) {
-    #pragma unroll
-    for (int i = 0; i < A_PT; ++i) {
-      const int idx = i * 256 + t, r = idx / RA, e = idx % RA;
-      ra[i] = 0;
-      if (r < NS && n + r < n1 && e < wide_a) ra[i] = a[(n + r) * lda + c0 * D + e];
-    }
-    #pragma unroll
-    for (int i = 0; i < G_PT; ++i) {
-      const int idx = i * 256 + t, r = idx / RG, e = idx % RG;
-      rg[i] = 0;
-      if (r < NS && n + r < n1 && e < wide_g) rg[i] = g[(n + r) * ldg + w0 * D + e];
+    const real* const an = a + n * lda;
+    const real* const gn = g + n * ldg;
+    if (TESTED) {
+      #pragma unroll
+      for (int i = 0; i < A_PT; ++i) {
+        const int idx = i * 256 + t, r = idx / RA, e = idx % RA;
+        ra[i] = 0;
+        if (r < NS && n + r < n1 && e < wide_a) ra[i] = a[(n + r) * lda + c0 * D + e];
+      }
+      #pragma unroll
+      for (int i = 0; i < G_PT; ++i) {
+        const int idx = i * 256 + t, r = idx / RG, e = idx % RG;
+        rg[i] = 0;
+        if (r < NS && n + r < n1 && e < wide_g) rg[i] = g[(n + r) * ldg + w0 * D + e];
+      }
+    } else if (n + NS <= n1) {
+      #pragma unroll
+      for (int i = 0; i < A_PT; ++i) ra[i] = an[oa[i]];
+      #pragma unroll
+      for (int i = 0; i < G_PT; ++i) rg[i] = gn[og[i]];
+    } else {
+      const int last = (int)(n1 - n) - 1;
+      #pragma unroll
+      for (int i = 0; i < A_PT; ++i) {
+        const int r = (i * 256 + t) / RA, back = r > last ? (r < NS ? r : NS - 1) - last : 0;
+        ra[i] = an[oa[i] - back * (int)lda];
+        if (back) ra[i] = 0;
+      }
+      #pragma unroll
+      for (int i = 0; i < G_PT; ++i) {
+        const int r = (i * 256 + t) / RG, back = r > last ? (r < NS ? r : NS - 1) - last : 0;
+        rg[i] = gn[og[i] - back * (int)ldg];
+        if (back) rg[i] = 0;
+      }
     }
   };
   accv acc[FR][FR];
@@ -399,10 +457,13 @@ bool linear_rows(const CBlock& b, int n) {
 }
 
 // Channels (forward) or outputs (SWAP) per staged chunk: 64 floats or 32
-// doubles, half of that where only then a chunk's weight rows are consecutive.
+// doubles, half of that where only then a chunk's weight rows are consecutive
+// (forward) or less is multiplied past the outputs (SWAP; 160 channels, lmax 3,
+// 20,000 rows, gA and gW 3,562 -> 3,006 us).
 int product_chunk(const CPlan& p, const CBlock& b, bool swap) {
+  if (swap) return p.bits == 32 && (b.mul3 + 63) / 64 * 64 == (b.mul3 + 31) / 32 * 32 ? 64 : 32;
   const int kc = p.bits == 64 ? 32 : 64;
-  return !swap && !linear_rows(b, kc) && linear_rows(b, kc / 2) ? kc / 2 : kc;
+  return !linear_rows(b, kc) && linear_rows(b, kc / 2) ? kc / 2 : kc;
 }
 
 int lds_reals(const CPlan& p, bool grad) {

@@ -92,3 +92,12 @@ def test_misuse_raises():
         op.contraction.run("out", a, torch.randn(op.weight_numel, device=DEV, dtype=torch.float64))
     with pytest.raises(RuntimeError):
         op.contraction.run("out", a, torch.randn(op.weight_numel))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rows", [3, 700])
+@pytest.mark.parametrize("channels", [24, 48, 80, 96, 112, 160])
+def test_widths_whose_weight_rows_cross_paths(channels, rows, dtype):
+    """Tiles and chunks that hold channels of two or three paths, with and without a remainder."""
+    irreps = "+".join(f"{channels}x{ir}" for ir in ("0e", "1o", "2e"))
+    test_the_three_products((irreps, "1x0e+1x1o+1x2e", irreps), rows, dtype)
