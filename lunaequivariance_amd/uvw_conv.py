@@ -288,6 +288,26 @@ class LunaTPUVWConv:
             self._contraction = NativeContraction(self)
         return self._contraction
 
+    def contracts_natively(self, rows) -> bool:
+        """Where the contraction kernels are at least as fast as the library products, forward
+        and backward together (kernels and library, us; 20,000 rows unless given).
+
+        fp32: lmax 2, 128 channels 997 and 1,427, 224 channels 3,168 and 3,091, 384 channels
+        8,090 and 6,902 (2,000 rows: 933 and 927); lmax 3, 256 channels 10,576 and 9,852 (2,000
+        rows: 1,160 and 1,293).  Scalar blocks, which the library multiplies without copies:
+        256 channels 117 and 125 (60,000 rows: 331 and 237), 128 channels of 60,000 rows 105
+        and 157.  fp64: lmax 1, 256 channels 1,415 and 1,564, 384 channels 3,327 and 3,018
+        (2,000 rows: 389 and 522); scalars, 256 channels 246 and 199 (8,000 rows: 108 and 122).
+        """
+        if not self.native_contraction:
+            return False
+        width = max(min(blk["mul3"], blk["channels"]) for blk in self.blocks)
+        work = 2e-9 * rows * sum(blk["channels"] * blk["mul3"] * blk["d3"] for blk in self.blocks)
+        double = self.compute_dtype == torch.float64
+        if all(blk["d3"] == 1 for blk in self.blocks):
+            return width < 160 or work < (2 if double else 4)
+        return width < (320 if double else 224) or work < (15 if double else 20)
+
     def _unit_weights(self, like):
         key = (like.device, like.dtype)
         if key not in self._ones:
@@ -310,11 +330,12 @@ class LunaTPUVWConv:
         shared row [weight_numel] or per-row [rows, weight_numel].
 
         Shared weights: the contraction kernels (csrc/contract.cpp), every block in one
-        launch.  Output degrees above 5: one library 2-D GEMM per block over rows (n, k),
-        [rows * d3, C] x [C, mul3].  Per-row weights: a batched GEMM.  The blocks are taken
-        with one split (its backward is one concatenation).
+        launch.  Output degrees above 5 and wide products of many rows: one library 2-D
+        GEMM per block over rows (n, k), [rows * d3, C] x [C, mul3].  Per-row weights: a
+        batched GEMM.  The blocks are taken with one split (its backward is one
+        concatenation).
         """
-        if weight.dim() == 1 and self.native_contraction:
+        if weight.dim() == 1 and self.contracts_natively(rows):
             return _Contract.apply(self.contraction, "out", values, weight)
         key = weight.device
         if key not in self._perm_cache:

@@ -101,3 +101,20 @@ def test_widths_whose_weight_rows_cross_paths(channels, rows, dtype):
     """Tiles and chunks that hold channels of two or three paths, with and without a remainder."""
     irreps = "+".join(f"{channels}x{ir}" for ir in ("0e", "1o", "2e"))
     test_the_three_products((irreps, "1x0e+1x1o+1x2e", irreps), rows, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("layout,native", [
+    (("3x3o+2x0e", "1x3o+1x0e", "2x6e+4x0e+3x3o"), None),  # an output of degree 6
+    (("8x0e+8x1o", "1x0e+2x1o", "5x0e+8x1o+3x1e+2x2e"), False),  # as for wide products of many rows
+])
+def test_library_products(monkeypatch, layout, native, dtype):
+    """The contraction without the kernels, through two orders of derivatives."""
+    from lunaequivariance_amd.uvw_conv import LunaTPUVWConv
+    from tests.test_uvw_conv_gpu import check
+
+    if native is None:
+        assert not make_op(*layout, dtype).native_contraction
+    else:
+        monkeypatch.setattr(LunaTPUVWConv, "contracts_natively", lambda self, rows: native)
+    check(*layout, 9, 40, dtype, True, 3, env=True, orders=2)

@@ -124,3 +124,30 @@ def test_split_k_weight_gradient(monkeypatch):
     assert torch.allclose(_split_k_tn(rows, rows[:, :2]), rows.t() @ rows[:, :2], atol=1e-12)
     assert torch.autograd.gradcheck(_RowsTimesWeight.apply, (rows, weight))
     assert torch.autograd.gradgradcheck(_RowsTimesWeight.apply, (rows, weight))
+
+
+@pytest.mark.parametrize("irreps,dtype,most", [
+    ("128x0e+128x1o", torch.float32, None),      # below 224 channels: any number of rows
+    ("256x0e+256x1o", torch.float32, 19073),     # 20 GFLOP: 8 products of 256 x 256 a row
+    ("256x0e+256x1o", torch.float64, None),
+    ("384x0e+384x1o", torch.float64, 6357),      # 15 GFLOP
+    ("128x0e", torch.float32, None),
+    ("256x0e", torch.float32, 30517),            # 4 GFLOP, scalars only
+    ("256x0e", torch.float64, 15258),
+    ("1x6e", torch.float32, 0),                  # degree 6: never
+])
+def test_where_the_contraction_kernels_are_taken(irreps, dtype, most):
+    from lunaequivariance_amd import Irreps, TensorProductConfig
+    from lunaequivariance_amd.uvw_conv import LunaTPUVWConv
+
+    edge = "1x0e" if "1o" not in irreps else "1x0e+1x1o"
+    a, b = Irreps(irreps), Irreps(edge)
+    paths = [(i, j, k, "uvw", True) for i, (_, x) in enumerate(a) for j, (_, y) in enumerate(b)
+             for k, (_, z) in enumerate(a) if z in x * y]
+    op = LunaTPUVWConv(TensorProductConfig(irreps, edge, irreps, paths, shared_weights=True, internal_weights=False),
+                       dtype=dtype)
+    assert op.contracts_natively(1) == (most != 0)
+    if most is None:
+        assert op.contracts_natively(10 ** 9)
+    elif most:
+        assert op.contracts_natively(most) and not op.contracts_natively(most + 1)
