@@ -32,7 +32,8 @@ so derivatives of every order follow.
 from __future__ import annotations
 
 import ctypes
-from math import prod
+from functools import cached_property
+from math import inf, prod
 
 import torch
 
@@ -180,6 +181,7 @@ class LunaTPUVWConv:
 
     mode = "uvw_conv"
     index_mode = "uvw_conv"
+    _contraction = None  # the contraction's plan, made on first use
 
     def __init__(self, tp, *, dtype=None, index_bits=32):
         paths = TensorProductPaths.from_tensor_product(tp)
@@ -265,10 +267,6 @@ class LunaTPUVWConv:
                     "broadcast_weights": True}
             self.agg = LunaTPUVUConv(meta, dtype=dtype)
         self._ones = {}
-        self._contraction = None
-        # Every output block whose degree the contraction kernels stage.
-        self.native_contraction = bool(self.blocks) and all(
-            blk["d3"] <= NativeContraction.MAX_COMPONENTS for blk in self.blocks)
         # The reference's "paths" configuration string, the constant a compiled
         # graph passes to lunatp::uvw_conv_* (built here, outside tracing).
         from .ops import paths_config
@@ -279,8 +277,13 @@ class LunaTPUVWConv:
         state = dict(self.__dict__)
         state["_ones"] = {}
         state["_perm_cache"] = {}
-        state["_contraction"] = None
+        state.pop("_contraction", None)
         return state
+
+    @property
+    def native_contraction(self) -> bool:
+        """Whether the contraction kernels stage every output block's degree."""
+        return bool(self.blocks) and all(blk["d3"] <= NativeContraction.MAX_COMPONENTS for blk in self.blocks)
 
     @property
     def contraction(self) -> NativeContraction:
@@ -299,14 +302,18 @@ class LunaTPUVWConv:
         and 157.  fp64: lmax 1, 256 channels 1,415 and 1,564, 384 channels 3,327 and 3,018
         (2,000 rows: 389 and 522); scalars, 256 channels 246 and 199 (8,000 rows: 108 and 122).
         """
+        return rows <= self._native_rows
+
+    @cached_property
+    def _native_rows(self) -> float:
         if not self.native_contraction:
-            return False
+            return -1
         width = max(min(blk["mul3"], blk["channels"]) for blk in self.blocks)
-        work = 2e-9 * rows * sum(blk["channels"] * blk["mul3"] * blk["d3"] for blk in self.blocks)
+        gflop = 2e-9 * sum(blk["channels"] * blk["mul3"] * blk["d3"] for blk in self.blocks)  # a row
         double = self.compute_dtype == torch.float64
         if all(blk["d3"] == 1 for blk in self.blocks):
-            return width < 160 or work < (2 if double else 4)
-        return width < (320 if double else 224) or work < (15 if double else 20)
+            return inf if width < 160 else (2 if double else 4) / gflop
+        return inf if width < (320 if double else 224) else (15 if double else 20) / gflop
 
     def _unit_weights(self, like):
         key = (like.device, like.dtype)

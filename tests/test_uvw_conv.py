@@ -151,3 +151,21 @@ def test_where_the_contraction_kernels_are_taken(irreps, dtype, most):
         assert op.contracts_natively(10 ** 9)
     elif most:
         assert op.contracts_natively(most) and not op.contracts_natively(most + 1)
+
+
+def test_operators_saved_before_the_contraction_kernels_load():
+    """Their state has neither the plan's place nor a flag."""
+    import pickle
+
+    from lunaequivariance_amd import TensorProductConfig
+    from lunaequivariance_amd.uvw_conv import LunaTPUVWConv
+
+    op = LunaTPUVWConv(TensorProductConfig("4x0e", "1x0e", "4x0e", [(0, 0, 0, "uvw", True)], shared_weights=True,
+                                           internal_weights=False))
+    old = object.__new__(LunaTPUVWConv)
+    state = op.__getstate__()
+    for name in ("_contraction", "native_contraction"):
+        state.pop(name, None)
+    old.__dict__.update(state)
+    for loaded in (old, pickle.loads(pickle.dumps(op))):
+        assert loaded.contracts_natively(10) and loaded.contraction.weight_numel == 16
