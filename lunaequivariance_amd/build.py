@@ -89,6 +89,26 @@ def uvw_operators():
     return [LunaTPUVW(paths)]
 
 
+def uvw_conv_operators():
+    """Shared-weight UVW convolutions of 64 channels per degree, lmax 3 (fp32) and 2 (fp64)."""
+    import torch
+
+    from .irreps import Irreps
+    from .layout import TensorProductConfig
+    from .uvw_conv import create_uvw_conv_operator
+
+    ops = []
+    for lmax, dtype in ((3, torch.float32), (2, torch.float64)):
+        irs = [f"{l}{'eo'[l % 2]}" for l in range(lmax + 1)]
+        ir, sh = ("+".join(f"{m}x{name}" for name in irs) for m in (64, 1))
+        a, b = Irreps(ir), Irreps(sh)
+        paths = [(i, j, k, "uvw", True) for i, (_, x) in enumerate(a) for j, (_, y) in enumerate(b)
+                 for k, (_, z) in enumerate(a) if z in x * y]
+        ops.append(create_uvw_conv_operator(
+            TensorProductConfig(ir, sh, ir, paths, internal_weights=False, shared_weights=True), dtype=dtype))
+    return ops
+
+
 def uuu_operators():
     """UUU convolutions of the benchmark (64 channels per degree, lmax 2-4, fp32)
     and of the reference's standard test problem (fp32 and fp64)."""
@@ -120,6 +140,10 @@ def precompile() -> int:
     count = 1
     for op in standard_operators() + uvw_operators() + uuu_operators():
         op.plan.precompile()
+        count += 1
+    for op in uvw_conv_operators():
+        op.agg.plan.precompile()
+        op.contraction.precompile()
         count += 1
     return count
 

@@ -1415,7 +1415,6 @@ std::string emit_backward_w(const UvwSpec& s, int chunk_rows) {
     const UvwPath& q = s.paths[p];
     const int K = q.mul1 * q.mul2, mt = ktiles(q), nt = (q.mul3 + 31) / 32, d3 = q.d3;
     const std::set<int> is = term_is(q), js = term_js(q);
-    const std::set<std::pair<int, int>> iks = term_iks(q);
     c.line("  if (path == %d) {", p);
     for (int m = 0; m < mt; ++m)
       for (int n = 0; n < nt; ++n) c.line("    floatx16 acc%d_%d = (floatx16)(0.0f);", m, n);

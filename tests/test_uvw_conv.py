@@ -169,3 +169,14 @@ def test_operators_saved_before_the_contraction_kernels_load():
     old.__dict__.update(state)
     for loaded in (old, pickle.loads(pickle.dumps(op))):
         assert loaded.contracts_natively(10) and loaded.contraction.weight_numel == 16
+
+
+def test_contraction_compiles_without_gpu(tmp_path, monkeypatch):
+    """The build's UVW convolutions: aggregation and contraction kernels for gfx950, ahead of the first call."""
+    from lunaequivariance_amd import build
+
+    monkeypatch.setenv("LUNAEQ_AMD_CACHE", str(tmp_path))
+    for op in build.uvw_conv_operators():
+        op.agg.plan.precompile()
+        op.contraction.precompile()
+    assert len(list(tmp_path.glob("con_*.co"))) == 2 and len(list(tmp_path.glob("uvu_*.co"))) == 4
