@@ -17,9 +17,10 @@ class TensorProduct(torch.nn.Module):
     """Row-wise tensor product (``src/modules/tensorproduct.py:19-116``).
 
     ``uvw``: shared weights in fp32 on matrix-core kernels, fp64 and per-row
-    weights through the row form of the UVW convolution.  ``uvu`` and ``uuu``:
-    the convolution kernels over the identity graph (matrices only).  Weights
-    are the configuration's registered parameter unless given.
+    ``uvw``: shared weights in fp32 on matrix-core kernels, fp64 and per-row
+    weights through the row form of the UVW convolution.  ``uvu``: row kernels
+    (matrices only).  ``uuu``: the convolution kernels over the identity graph.
+    Weights are the configuration's registered parameter unless given.
     """
 
     def __init__(self, irreps_in1, irreps_in2=None, irreps_out=None, instructions=None,

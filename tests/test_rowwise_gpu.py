@@ -1,5 +1,5 @@
-"""Row-wise UVU and UUU tensor products (convolution kernels over the identity graph)
-against the fp64 oracle (the convolution oracle with row b's edge going from and to b).
+"""Row-wise UVU (row kernels) and UUU (convolution kernels over the identity graph) tensor
+products against the fp64 oracle (the convolution oracle with row b's edge going from and to b).
 
 Tolerance as for the convolution tests.  Cases follow the reference's
 ``tests/lunatp/test_uvu.py`` / ``test_uuu.py`` modes: per-row and shared weights,
