@@ -452,13 +452,12 @@ void emit_group_lanes(Code& c, const UGroup& g) {
   c.line("    const bool act = u < %d;", g.ch);
 }
 
-// Loop of one wave over its runs of a node's edges, nsub at once: the lane's edge is
-// `name` where left > sub.  What is left of the row is compared, not positions: with
-// int32 offsets a position past `end` wraps to a negative one near 2^31 edges.
+// Loop of one wave over its runs of a node's edges, nsub at once; the lane's edge is
+// `name` where that lies before `end`.  Positions are 64-bit: as int32 those past
+// the end, up to 575 ahead, would wrap to negative ones near 2^31 edges.
 void emit_edge_loop(Code& c, int nsub, const char* name) {
-  c.line("    for (eix left = end - beg - wave * %d, e0 = beg + (left > 0 ? wave * %d : 0); left > 0;", nsub, nsub);
-  c.line("         left -= %d * split, e0 += left > 0 ? %d * split : 0) {", nsub, nsub);
-  c.line("      const eix %s = left > sub ? e0 + sub : e0;", name);
+  c.line("    for (i64 e0 = (i64)beg + wave * %d; e0 < end; e0 += %d * split) {", nsub, nsub);
+  c.line("      const i64 %s = e0 + sub;", name);
 }
 
 // t{p}_k = sum_{(i,j,k)} c x_i y_j of path p, as sum_i x_i z_ik.
@@ -535,7 +534,7 @@ std::string emit_forward(const UuuPlan& plan, bool env, bool l0) {
         c.line("    real %s = 0;", accs.back().c_str());
       }
     emit_edge_loop(c, nsub, "e");
-    c.line("      if (act && left > sub) {");
+    c.line("      if (act && e < end) {");
     c.line("        const i64 sn = src[e];");
     for (int b : g.xbs)
       c.line("        const real* xr%d = x + sn * IN1 + %d + (i64)u * %d;", b, s.xblocks[b].off, s.xblocks[b].d);
@@ -647,9 +646,9 @@ std::string emit_backward(const UuuPlan& plan, bool env, bool gl0, bool want_gx,
           c.line("    real %s = 0;", gxs.back().c_str());
         }
     emit_edge_loop(c, nsub, "pos");
-    c.line("      const eix e = left > sub ? edge_ids[pos] : 0;");
+    c.line("      const eix e = pos < end ? edge_ids[pos] : 0;");
     if (want_genv) c.line("      real gev = 0;");
-    c.line("      if (act && left > sub) {");
+    c.line("      if (act && pos < end) {");
     c.line("        const i64 dn = dst[e];");
     for (const auto& yj : use.y)
       c.line("        const real y%d_%d = __builtin_nontemporal_load(y + (i64)e * IN2 + %d + (i64)u * %d);", yj.first,
@@ -734,7 +733,7 @@ std::string emit_backward(const UuuPlan& plan, bool env, bool gl0, bool want_gx,
     if (want_genv) {
       // Sum over the channels of this sub-group's edge; its first lane writes.
       if (g.cw > 1) lane_sum(c, {"gev"}, 1, g.cw / 2, "      ");
-      c.line("      if ((lane & %d) == 0 && left > sub) part[(i64)(%d + chunk) * num_edges + e] = gev;", g.cw - 1,
+      c.line("      if ((lane & %d) == 0 && pos < end) part[(i64)(%d + chunk) * num_edges + e] = gev;", g.cw - 1,
              g.genv_slot);
     }
     c.line("    }");
