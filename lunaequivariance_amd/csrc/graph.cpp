@@ -405,9 +405,11 @@ struct GraphKernels {
   GraphKernels() { kernels.tag = "graph"; }
 };
 
+// Never destroyed: unloading modules after main would call a HIP runtime that is
+// being taken down.
 GraphKernels& graph_kernels() {
-  static GraphKernels g;
-  return g;
+  static GraphKernels* const g = new GraphKernels;
+  return *g;
 }
 
 hipModule_t graph_module(const char* cache_dir) {
