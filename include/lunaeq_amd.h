@@ -106,10 +106,13 @@ int luna_uvu_plan_destroy(LunaUvuPlan* plan);
 int luna_uvu_plan_info(const LunaUvuPlan* plan, LunaUvuPlanInfo* info);
 
 /*
- * Compile (or fetch from cache) every kernel variant a plan can launch, without
- * touching a device.  Used to warm the code-object cache ahead of time.
+ * Compile (or fetch from cache) the forward and backward kernels that every layer runs
+ * (no envelope, no scalar features), without touching a device.  Used to warm the
+ * code-object cache ahead of time; luna_uvu_plan_precompile_all also compiles the
+ * kernels for few nodes and for few edges per node, and the row-wise products'.
  */
 int luna_uvu_plan_precompile(LunaUvuPlan* plan);
+int luna_uvu_plan_precompile_all(LunaUvuPlan* plan);
 
 /*
  * Forward: out[t] = sum over edges e with dst[e]==t of env[e] * TP(x[src[e]], y[e], w[e]).

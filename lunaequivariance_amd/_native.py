@@ -36,6 +36,7 @@ PROTOTYPES = {
     "luna_uvu_plan_destroy": (ctypes.c_int, [_VP]),
     "luna_uvu_plan_info": (ctypes.c_int, [_VP, ctypes.POINTER(PlanInfo)]),
     "luna_uvu_plan_precompile": (ctypes.c_int, [_VP]),
+    "luna_uvu_plan_precompile_all": (ctypes.c_int, [_VP]),
     "luna_uvu_conv_fwd": (ctypes.c_int, [_VP] + [_VP] * 4 + [_I32P] * 3 + [_VP, _VP, _I64, _I64, _VP]),
     "luna_uvu_conv_bwd_workspace": (ctypes.c_int, [_VP, _I64, _I64, ctypes.POINTER(ctypes.c_size_t)]),
     "luna_uvu_conv_bwd": (ctypes.c_int, [_VP] + [_VP] * 6 + [_I32P] * 5 + [_VP] * 5

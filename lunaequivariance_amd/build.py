@@ -138,11 +138,15 @@ def precompile() -> int:
 
     _native.check(_native.lib().luna_graph_precompile(_native.cache_dir().encode()), "luna_graph_precompile")
     count = 1
-    for op in standard_operators() + uvw_operators() + uuu_operators():
+    for op in standard_operators():
+        # Layers of one to two degrees are also run on graphs of a few nodes.
+        op.plan.precompile(everything=op.max_channels <= 32)
+        count += 1
+    for op in uvw_operators() + uuu_operators():
         op.plan.precompile()
         count += 1
     for op in uvw_conv_operators():
-        op.agg.plan.precompile()
+        op.agg.plan.precompile(everything=True)
         op.contraction.precompile()
         count += 1
     return count

@@ -250,6 +250,21 @@ int luna_uvu_plan_precompile(LunaUvuPlan* plan) {
   });
 }
 
+int luna_uvu_plan_precompile_all(LunaUvuPlan* plan) {
+  return guard_call([&] {
+    if (!plan) fail("luna_uvu_plan_precompile_all: null plan");
+    auto compile = [](Plan& p, std::initializer_list<const char*> variants) {
+      for (const char* v : variants) p.kernels.code_for(v, [&] { return source_for(p, v); });
+    };
+    const bool own = !plan->plan.spec.w_broadcast;  // a broadcast weight row has no gradient
+    if (own)
+      compile(plan->plan, {"fwd00", "bwd00111", "fws00", "rwf0", "rwf1", "rwb0111", "rwb1111"});
+    else
+      compile(plan->plan, {"fwd00", "bwd00011", "fws00", "rwf1", "rwb1011"});
+    if (plan->sparse) compile(*plan->sparse, {"fwd00", own ? "bwd00111" : "bwd00011"});
+  });
+}
+
 int luna_uvu_conv_fwd(const LunaUvuPlan* cplan, const void* x, const void* y, const void* w,
                       const void* env, const int32_t* src, const void* dst_rowptr,
                       const int32_t* node_order, void* out, void* l0, int64_t num_nodes,

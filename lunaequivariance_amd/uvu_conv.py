@@ -153,8 +153,11 @@ class NativePlan:
                       "luna_uvu_conv_bwd_workspace")
         return size.value
 
-    def precompile(self):
-        _native.check(_native.lib().luna_uvu_plan_precompile(self.handle), "luna_uvu_plan_precompile")
+    def precompile(self, everything=False):
+        """The kernels that every layer runs, or also those for small and sparse graphs and rows."""
+        lib = _native.lib()
+        call = lib.luna_uvu_plan_precompile_all if everything else lib.luna_uvu_plan_precompile
+        _native.check(call(self.handle), "luna_uvu_plan_precompile")
 
     def __del__(self):
         handle = getattr(self, "handle", None)

@@ -68,3 +68,15 @@ int main() {
   }
 }""")
     assert out == ["8:2:1:1", "12:2:1:1", "16:2:1:1", "17:3:1:1", "32:3:1:1", "33:0:1:1"]
+
+
+def test_all_kernels_of_a_plan_compile_without_gpu(tmp_path, monkeypatch):
+    """Ahead of the first call: a narrow layer on any graph (no envelope or scalar features) and by rows."""
+    from lunaequivariance_amd.build import standard_operators
+
+    monkeypatch.setenv("LUNAEQ_AMD_CACHE", str(tmp_path))
+    op = standard_operators()[2]
+    assert op.max_channels == 32
+    op.plan.precompile(everything=True)
+    names = sorted(p.name.split("_")[1] for p in tmp_path.glob("uvu_*.co"))
+    assert names == ["bwd00111", "bwd00111", "fwd00", "fwd00", "fws00", "rwb0111", "rwb1111", "rwf0", "rwf1"]
