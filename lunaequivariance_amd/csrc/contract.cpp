@@ -15,18 +15,20 @@
 // is made.  The three kernels run every output block in one launch.
 //
 // Bound and shape.  At 64 channels, lmax 3 and 2,083 rows the work is 1.7
-// GFLOP on 53 MB of A: 11 us of either.  Measured there 31 us (forward), 42
+// GFLOP on 53 MB of A: 11 us of either.  Measured there 32 us (forward), 42
 // us (gA) and 33 + 7 us (gW and its reduction), against about 550 us for the
-// library products, layout copies and concatenations they replaced (step 990
-// -> 481 us); at 20,011 fp64 rows of 32 channels, lmax 2 (180 MB of A, 38 us)
-// 53, 70 and 63 + 17 us (step 1,149 -> 343 us).  The launches are bound by
+// library products, layout copies and concatenations they replaced (step 975
+// -> 397 us); at 20,011 fp64 rows of 32 channels, lmax 2 (180 MB of A, 38 us)
+// 51, 67 and 64 + 18 us (step 1,142 -> 290 us).  The launches are bound by
 // latency in the first case (two workgroups per CU) and by the traffic of A
 // in the second.  A workgroup of four waves owns a 64 x 64 or 32 x 128 tile
 // (half as many columns in fp64, whose 64-bit tiles would halve the
 // workgroups per CU), each wave 32 x 32 on v_mfma_f32_32x32x2f32 or 32 x 16 on
 // v_mfma_f64_16x16x4f64; operands go through LDS, the next chunk is in
 // registers while the current one is multiplied, and results leave through
-// LDS as contiguous runs.
+// LDS as contiguous runs.  Wide products of many rows, where the matrix rate
+// counts and these tiles reach about 55 % of it, stay with the library
+// (LunaTPUVWConv.contracts_natively).
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>

@@ -479,10 +479,10 @@ void emit_dma_unit_body(Code& c, const UvwSpec& s, const Unit& u) {
     const std::set<std::pair<int, int>> iks = term_iks(q);
     // Fewer input than output components: contract x with the weights first
     // (2 l1 + 1 matrix steps instead of 2 l3 + 1) and couple the results, where
-    // both accumulators leave two waves per SIMD without spills.  200,000 rows, 64
-    // channels, lmax 2, forward: 621 us without, 616 / 600 / 560 us with up to 96 /
-    // 128 / 192 registers of accumulators, 547 us with 256 (37 spilled); 100,000 rows,
-    // lmax 1: 110 -> 92 us; 32 channels, lmax 2: 119 -> 115 us.
+    // both accumulators leave two waves per SIMD without spills.  Forward calls back
+    // to back, 200,000 rows, 64 channels, lmax 2: 583 us without, 583 / 566 / 523 us
+    // with up to 96 / 128 / 192 registers of accumulators (256 spill 37); 100,000 rows,
+    // lmax 1: 108 -> 89 us; 32 channels, lmax 2: 104 -> 97 us.
     const bool late = d1 < d3 && 16 * T * (d1 + d3) <= kLateRegisters;
     c.line("    const real* xrow = x + (i64)rrow * %d + %d + (lane >> 5) * 4;", s.in1, q.x_off);
     c.line("    const real* wrow = wt + %d + (i64)(lane / %d) * %d + wl;", q.w_off, wq, mul3);
