@@ -92,3 +92,36 @@ def test_third_order_chain_on_a_side_stream_and_in_a_graph(mode, shared):
         assert len(outputs) == len(expected)
         for n, (a, b) in enumerate(zip(outputs, expected)):
             torch.testing.assert_close(a, b, rtol=1e-12, atol=1e-13, msg=f"replay {replay}, output {n}")
+
+
+@pytest.mark.parametrize("nodes,edges", [(23, 30), (9, 1200)])  # few edges per node; few nodes of many edges
+def test_kernels_first_used_during_a_capture(nodes, edges):
+    """A program that warmed up on another graph captures one whose kernels no call has loaded yet."""
+    print(f"capture first use {nodes} {edges}", flush=True)
+    conv, graph, gen = problem("uvu", False)
+    warm = [t.requires_grad_() for t in fresh(conv, graph, gen, False)]
+
+    def step(graph, x, y, w, env, g):
+        out = conv(x, y, w, graph=graph, env=env)
+        return [out, *torch.autograd.grad(out, (x, y, w, env), g)]
+
+    src, dst = random_graph(nodes, edges, gen)
+    other = conv.create_graph(src.to(DEV), dst.to(DEV), nodes)
+    static = [t.requires_grad_() for t in fresh(conv, other, gen, False)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step(graph, *warm)
+    torch.cuda.current_stream().wait_stream(side)
+    captured = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(captured):
+        results = step(other, *static)
+    for _ in range(3):
+        with torch.no_grad():
+            for t in static:
+                t.copy_(torch.randn(t.shape, generator=gen, dtype=DT))
+        captured.replay()
+        torch.cuda.synchronize()
+        for n, (a, b) in enumerate(zip(results, step(other, *static))):
+            torch.testing.assert_close(a, b, rtol=1e-12, atol=1e-13, msg=f"replay, output {n}")
