@@ -56,6 +56,8 @@ struct CPlan {
   ModuleCache kernels;
 };
 
+// Values of a row whose offsets within a tile of up to 128 rows fit 32 bits.
+constexpr int kMaxRow = 1 << 23;
 // Degrees whose staged tiles fit 64 KB of LDS (4 rows x 160 channels x d3 doubles).
 constexpr int kMaxD3 = 11;
 
@@ -76,6 +78,7 @@ void parse(CPlan& p, const std::string& text) {
   p.adim = read_int(in, "aggregate_dim");
   p.out = read_int(in, "out_dim");
   p.wnum = read_int(in, "weight_numel");
+  if (p.adim > kMaxRow || p.out > kMaxRow) fail("contraction spec: rows of more than 2^23 values are not supported");
   const int nblocks = read_int(in, "blocks");
   for (int n = 0; n < nblocks; ++n) {
     CBlock b;

@@ -92,6 +92,7 @@ class NativeContraction:
     operator in one launch, on the layouts of the aggregate and of the output."""
 
     MAX_COMPONENTS = 11  # output blocks of degree 5; wider ones take the library products
+    MAX_ROW = 1 << 23    # values of a row of A or of the output
 
     def __init__(self, op):
         self.adim, self.out_dim, self.weight_numel = op.aggregate_dim, op.out_dim, op.weight_numel
@@ -282,8 +283,9 @@ class LunaTPUVWConv:
 
     @property
     def native_contraction(self) -> bool:
-        """Whether the contraction kernels stage every output block's degree."""
-        return bool(self.blocks) and all(blk["d3"] <= NativeContraction.MAX_COMPONENTS for blk in self.blocks)
+        """Whether the contraction kernels take rows of this width and stage every output degree."""
+        return (bool(self.blocks) and max(self.aggregate_dim, self.out_dim) <= NativeContraction.MAX_ROW
+                and all(blk["d3"] <= NativeContraction.MAX_COMPONENTS for blk in self.blocks))
 
     @property
     def contraction(self) -> NativeContraction:

@@ -182,3 +182,22 @@ def test_contraction_compiles_without_gpu(tmp_path, monkeypatch):
     names = [p.name.split("_")[1] for p in tmp_path.glob("uvu_*.co")]
     assert sorted(names) == 2 * ["bwd00011"] + 2 * ["fwd00"] + 2 * ["fws00"] + 2 * ["rwb1011"] + 2 * ["rwf1"]
     assert len(list(tmp_path.glob("con_*.co"))) == 2
+
+
+def test_rows_too_wide_for_the_contraction_kernels():
+    """Their offsets within a tile of up to 128 rows are 32-bit."""
+    import ctypes
+    from types import SimpleNamespace
+
+    from lunaequivariance_amd import _native
+    from lunaequivariance_amd.uvw_conv import LunaTPUVWConv
+
+    limit = 1 << 23
+    for adim, out, fits in ((limit, 8, True), (8, limit, True), (limit + 1, 8, False), (8, limit + 1, False)):
+        handle = ctypes.c_void_p()
+        spec = f"LUNACON1 32 {adim} {out} 64 1\n0 0 1 8 1 0 8 1\n".encode()
+        assert (_native.lib().luna_con_plan_create(spec, b"", ctypes.byref(handle)) == 0) == fits
+        if handle:
+            _native.lib().luna_con_plan_destroy(handle)
+        op = SimpleNamespace(blocks=[dict(d3=1)], aggregate_dim=adim, out_dim=out)
+        assert LunaTPUVWConv.native_contraction.fget(op) == fits
